@@ -260,5 +260,7 @@ void d2h(tn_ctx* c, void* dst, const void* src, size_t bytes);
 // n (<= TN_PUBLISH_MAX) doubles device -> host through the published scalars
 // (no stream synchronisation: the host polls the completion flag)
 void d2h_small(tn_ctx* c, double* dst, const double* src, int n);
+// the n values a kernel published with sequence number seq (polls its flag)
+void read_published(tn_ctx* c, double* dst, int n, unsigned long long seq);
 
 }  // namespace tn

@@ -48,6 +48,12 @@ void d2h_small(tn_ctx* c, double* dst, const double* src, int n)
     TN_REQUIRE(n >= 0 && n <= TN_PUBLISH_MAX && c->sc.h, TN_ERR_ARG, "d2h_small: bad size");
     const unsigned long long seq = ++c->sc.seq;
     TN_HIP(publish(src, n, c->sc.d, c->sc.flag_d, seq, c->stream));
+    read_published(c, dst, n, seq);
+}
+
+// the n values published with sequence number seq, once they are there
+void read_published(tn_ctx* c, double* dst, int n, unsigned long long seq)
+{
     volatile unsigned long long* f = c->sc.flag_h;
     const auto t0 = std::chrono::steady_clock::now();
     for (unsigned long spins = 1; *f != seq; spins++) {
@@ -780,33 +786,35 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
     hipStream_t s = c->stream;
     LanczosResult res;
     const int kmax = std::max(2, std::min(max_krylov, 500));
-    c->krylov.ensure((size_t)(kmax + 1) * N * 8);
+    TN_REQUIRE(N > 0 && N % 2 == 0, TN_ERR_ARG, "Lanczos: the padded vector length must be even");
+    c->krylov.ensure((size_t)(kmax + 2) * N * 8);
     double* V = c->krylov.as<double>();
+    double* hv = V + (size_t)(kmax + 1) * N;  // H v_j, before the three-term step
     c->lanczos_small.ensure(sizeof(double) * (4 * 512 + 64));
     double* h = c->lanczos_small.as<double>();  // [0, 512): coefficients, [512, 1024): Ritz coefficients
     double* zd = h + 512;
     double* nrm = h + 1024;
-    const long pcap = mdot_part_size(N, kmax + 1);
+    const long pcap = std::max(mdot_part_size(N, 1), lz_part_size(N, kmax + 1));
     c->part.ensure(pcap * 8);
     double* part = c->part.as<double>();
     std::vector<double> al(kmax), be(kmax), z(kmax), hh(kmax + 4);
-    // fused step kernels: 16-byte vector access needs an even length
-    const bool fused = N % 2 == 0 && kmax <= 512;
-    const bool pro = partial && fused;
+    const bool pro = partial;
     const double eta = std::sqrt(eps_op);
     std::vector<double> om_old(kmax + 2, 0.0), om(kmax + 2, 0.0), om_new(kmax + 2, 0.0);
     // the scaling of the next basis vector not launched yet (prescale)
     double pending = 0.0;
     c->x_prescale = 0.0;
 
-    auto read = [&](double* dst, const double* src, int n) {
-        if (n <= TN_PUBLISH_MAX) d2h_small(c, dst, src, n);
-        else d2h(c, dst, src, (size_t)n * 8);
+    // h[0..nh) and |w|^2 of the last lz_update
+    auto read = [&](double* dst, int nh) {
+        const unsigned long long seq = ++c->sc.seq;
+        TN_HIP(lz_publish(h, nh, N, part, c->sc.d, c->sc.flag_d, seq, s));
+        read_published(c, dst, nh + 1, seq);
     };
     auto norm_host = [&](const double* v) {
         TN_HIP(mdot(v, N, 1, v, N, nrm, part, (int)pcap, s));
         double v2 = 0;
-        read(&v2, nrm, 1);
+        d2h_small(c, &v2, nrm, 1);
         return std::sqrt(v2);
     };
 
@@ -841,7 +849,7 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
                 pending = 0.0;
             }
             try {
-                fn(c, op, vj, w);
+                fn(c, op, vj, hv);
             } catch (...) {
                 c->x_prescale = 0.0;
                 throw;
@@ -849,15 +857,15 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
             res.n_matvec++;
             // three-term step with the exact alpha = v_j.w (h[0] on the device),
             // then one classical Gram-Schmidt pass against every Krylov vector
-            // (h[1..j+1]) removes what rounding left; h[j+2] = |w|^2
-            TN_HIP(mdot(vj, N, 1, w, N, h, part, (int)pcap, s));
+            // (h[1..j+1]) removes what rounding left; |w|^2 comes last
+            TN_HIP(lz_dot(vj, hv, N, part, s));
             if (pro) {
                 // the same step and pass against v_{j-1}, v_j only
                 const int kk = j >= 1 ? 2 : 1;
                 const double* Vl = V + (long)(j + 1 - kk) * N;
-                TN_HIP(lz_step_dots(w, Vl, N, kk, h, j > 0 ? be[j - 1] : 0.0, N, h + 1, part, pcap, s));
-                TN_HIP(lz_update_norm(w, Vl, N, kk, h + 1, N, h + kk + 1, part, pcap, s));
-                read(hh.data(), h, kk + 2);
+                TN_HIP(lz_step(hv, w, Vl, N, kk, true, j > 0 ? be[j - 1] : 0.0, N, h, part, s));
+                TN_HIP(lz_update(w, Vl, N, kk, N, h + 1, part, s));
+                read(hh.data(), kk + 1);
                 al[j] = hh[0] + hh[kk];
                 be[j] = std::sqrt(std::max(hh[kk + 1], 0.0));
                 tnorm = std::max(tnorm, std::fabs(al[j]) + be[j] + (j > 0 ? be[j - 1] : 0.0));
@@ -875,9 +883,9 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
                 }
                 om_new[j + 1] = 1.0;
                 if (j > 0 && (force || wmax > eta || !std::isfinite(wmax))) {
-                    TN_HIP(mdot(V, N, j + 1, w, N, h + 1, part, (int)pcap, s));
-                    TN_HIP(lz_update_norm(w, V, N, j + 1, h + 1, N, h + j + 2, part, pcap, s));
-                    read(hh.data(), h, j + 3);
+                    TN_HIP(lz_step(w, w, V, N, j + 1, false, 0.0, N, h, part, s));
+                    TN_HIP(lz_update(w, V, N, j + 1, N, h + 1, part, s));
+                    read(hh.data(), j + 2);
                     al[j] += hh[j + 1];
                     const double bc = std::sqrt(std::max(hh[j + 2], 0.0));
                     // only rounding left: an invariant subspace (breakdown)
@@ -890,20 +898,12 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
                 }
                 std::swap(om_old, om);
                 std::swap(om, om_new);
-            } else if (fused) {
+            } else {
                 // three-term step fused with the Gram-Schmidt dot products, then
                 // the Gram-Schmidt update fused with the norm
-                TN_HIP(lz_step_dots(w, V, N, j + 1, h, j > 0 ? be[j - 1] : 0.0, N, h + 1, part, pcap, s));
-                TN_HIP(lz_update_norm(w, V, N, j + 1, h + 1, N, h + j + 2, part, pcap, s));
-            } else {
-                TN_HIP(three_term(w, vj, j > 0 ? V + (long)(j - 1) * N : nullptr, h, j > 0 ? be[j - 1] : 0.0, N,
-                                  s));
-                TN_HIP(mdot(V, N, j + 1, w, N, h + 1, part, (int)pcap, s));
-                TN_HIP(gemv_acc(V, N, j + 1, h + 1, -1.0, 1.0, w, N, s));
-                TN_HIP(mdot(w, N, 1, w, N, h + j + 2, part, (int)pcap, s));
-            }
-            if (!pro) {
-                read(hh.data(), h, j + 3);
+                TN_HIP(lz_step(hv, w, V, N, j + 1, true, j > 0 ? be[j - 1] : 0.0, N, h, part, s));
+                TN_HIP(lz_update(w, V, N, j + 1, N, h + 1, part, s));
+                read(hh.data(), j + 2);
                 al[j] = hh[0] + hh[j + 1];
                 be[j] = std::sqrt(std::max(hh[j + 2], 0.0));
                 tnorm = std::max(tnorm, std::fabs(al[j]) + be[j] + (j > 0 ? be[j - 1] : 0.0));

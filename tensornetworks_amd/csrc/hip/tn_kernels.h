@@ -163,18 +163,21 @@ hipError_t absmax(const double* x, long n, double* out, double* part, int part_c
 // v[n] *= 1/den[0] (den on device)
 hipError_t scale_by_inv(double* v, const double* den, long n, hipStream_t s);
 hipError_t axpby(double a, const double* x, double b, double* y, long n, hipStream_t s);
-// w -= alpha[0] v + beta u (u may be null); alpha is a device scalar
-// Fused Lanczos step (n even, vectors 16-byte aligned, k <= 512):
-//  step_dots : w <- w - alpha[0] V_{k-1} - beta V_{k-2} (the latter when k >= 2),
-//              then out[i] = V_i . w for i < k (two-stage, fixed order)
-//  update_norm: w <- w - sum_{i<k} coef[i] V_i, then out[0] = |w|^2 (two-stage)
-// part: mdot_part_size(n, k + 1) doubles.
-hipError_t lz_step_dots(double* w, const double* V, long ldv, int k, const double* alpha, double beta, long n,
-                        double* out, double* part, long part_cap, hipStream_t s);
-hipError_t lz_update_norm(double* w, const double* V, long ldv, int k, const double* coef, long n, double* out,
-                          double* part, long part_cap, hipStream_t s);
-hipError_t three_term(double* w, const double* v, const double* u, const double* alpha, double beta, long n,
-                      hipStream_t s);
+// Fused Lanczos step (n even, vectors 16-byte aligned, k <= 512), in this order
+// on one stream, part: lz_part_size(n, k) doubles of scratch, h: k + 1 doubles:
+//  lz_dot    : partial sums of alpha = v . w
+//  lz_step   : three: alpha to h[0], w <- y - alpha V_{k-1} - beta V_{k-2} (the
+//              latter when k >= 2; y and w different buffers); not three: w as
+//              it is.  Then partial sums of V_i . w, i < k
+//  lz_update : coef[i] = V_i . w, w <- w - sum_{i<k} coef[i] V_i, partial |w|^2
+//  lz_publish: h[0..nh) and |w|^2 to the host (see publish)
+long lz_part_size(long n, int k);
+hipError_t lz_dot(const double* v, const double* w, long n, double* part, hipStream_t s);
+hipError_t lz_step(const double* y, double* w, const double* V, long ldv, int k, bool three, double beta, long n,
+                   double* h, double* part, hipStream_t s);
+hipError_t lz_update(double* w, const double* V, long ldv, int k, long n, double* coef, double* part, hipStream_t s);
+hipError_t lz_publish(const double* h, int nh, long n, const double* part, double* host_dst,
+                      unsigned long long* host_flag, unsigned long long seq, hipStream_t s);
 // y = a x (y is not read; x and y may be the same buffer)
 hipError_t scale_copy(double a, const double* x, double* y, long n, hipStream_t s);
 
@@ -311,7 +314,7 @@ struct MixJob {  // FP32 in; with t.esel/t.osel set, the identity-channel form o
     long osx2;
 };
 // Fused Lanczos step for many problems (n even for every job), the batched
-// form of lz_step_dots / lz_update_norm.  part: bmdot_part_size(n, kmax, nmax)
+// form of lz_step / lz_update.  part: bmdot_part_size(n, kmax, nmax)
 // doubles for bstep_dots, n * ceil(nmax / 2048) for bupdate_norm.
 struct StepJob {  // w -= alpha[0] V_{k-1} + beta V_{k-2} (k >= 2), then out[i] = V_i . w, i < k;
     double* w;      // with beta_sq set, beta = sqrt(*beta_sq) read on the device

@@ -1674,131 +1674,318 @@ hipError_t mdot(const double* V, long ldv, int k, const double* w, long n, doubl
     return hipGetLastError();
 }
 
-// Fused Lanczos kernels.  A block owns a chunk of MD_BLOCK * MD_EPT entries,
-// each thread MD_EPT / 2 pairs (16-byte loads, consecutive lanes on
-// consecutive pairs).  update_norm visits the chunks in the reverse order of
-// step_dots, so its first chunks of the basis are the ones step_dots read
-// last (still in the last-level cache when the basis exceeds it).
-#define LZ_PAIRS (MD_EPT / 2)
-__global__ void __launch_bounds__(MD_BLOCK) lz_step_dots_k(double* __restrict__ w, const double* __restrict__ V,
-                                                           long ldv, int k, const double* __restrict__ alpha,
-                                                           double beta, long n, double* __restrict__ part)
+// One Lanczos step is four launches (lz_dot, lz_step, lz_update, lz_publish):
+// each kernel sums the partial results of the one before it in its own
+// prologue, in a fixed order, so no reduction has a launch of its own.  Bound
+// by launches and load latency up to n ~ 1e5, by the last-level cache or HBM
+// beyond; the grid of lz_step splits the basis vectors as well as the entries
+// (one workgroup per 2048 entries, taking the vectors one after the other,
+// left 45 of 256 CUs busy at n = 92160).  Measured for the vector part of an
+// iteration with a pass against k vectors, that form (with a second launch per
+// reduction) and this one: n = 2048, k ~ 28: 58 and 15 us; n = 92160, k ~ 84:
+// 224 and 43 us (the 62 MB basis read twice: 2.9 TB/s); n = 196608, k = 2
+// (partial re-orthogonalisation): 33 and 22 us.
+#define LZ_SMALL 131072  // entries up to which chunks are sized for latency
+
+// entry pairs per thread of lz_step: one while the vectors are short or few (a
+// workgroup per 512 entries), else four (2048 entries; up to LZ_SMALL at most
+// 64 partial sums per coefficient, which lz_update sums by one thread each)
+static inline int lz_step_pairs(long n, int k) { return n <= 8192 || (n <= LZ_SMALL && k <= 8) ? 1 : 4; }
+static inline long lz_step_blocks(long n, int k)
 {
-    __shared__ double red[MD_MAXK][MD_BLOCK / 64];
-    const long c0 = (long)blockIdx.x * MD_BLOCK * MD_EPT;
-    const double a = alpha[0];
-    const double* vj = V + (long)(k - 1) * ldv;
-    const double* vm = k >= 2 ? V + (long)(k - 2) * ldv : nullptr;
-    double2 wr[LZ_PAIRS];
-#pragma unroll
-    for (int e = 0; e < LZ_PAIRS; e++) {
-        const long idx = c0 + 2 * ((long)e * MD_BLOCK + threadIdx.x);
-        if (idx < n) {
-            double2 x = *(const double2*)(w + idx);
-            const double2 p = *(const double2*)(vj + idx);
-            x.x -= a * p.x;
-            x.y -= a * p.y;
-            if (vm) {
-                const double2 q = *(const double2*)(vm + idx);
-                x.x -= beta * q.x;
-                x.y -= beta * q.y;
-            }
-            *(double2*)(w + idx) = x;
-            wr[e] = x;
-        } else {
-            wr[e] = make_double2(0.0, 0.0);
-        }
-    }
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    for (int i = 0; i < k; i++) {
-        const double* vi = V + (long)i * ldv;
-        double acc = 0.0;
-#pragma unroll
-        for (int e = 0; e < LZ_PAIRS; e++) {
-            const long idx = c0 + 2 * ((long)e * MD_BLOCK + threadIdx.x);
-            if (idx < n) {
-                const double2 p = *(const double2*)(vi + idx);
-                acc += p.x * wr[e].x + p.y * wr[e].y;
-            }
-        }
-        acc = wave_sum(acc);
-        if (lane == 0) red[i][wid] = acc;
-    }
+    const long c = 2L * MD_BLOCK * lz_step_pairs(n, k);
+    return (n + c - 1) / c;
+}
+static inline long lz_dot_blocks(long n)
+{
+    const long c = n <= LZ_SMALL ? 2L * MD_BLOCK : 8L * MD_BLOCK;
+    return (n + c - 1) / c;
+}
+static inline long lz_norm_blocks(long n)
+{
+    const long c = n <= LZ_SMALL ? 128 : 8L * MD_BLOCK;
+    return (n + c - 1) / c;
+}
+long lz_part_size(long n, int k)
+{
+    const long few = lz_step_blocks(n, 1) * (k < 8 ? k : 8), all = lz_step_blocks(n, k) * (long)k;
+    return lz_dot_blocks(n) + lz_norm_blocks(n) + (few > all ? few : all);
+}
+
+// sum of v[0..n) over the workgroup (MD_BLOCK threads), the same on every thread
+__device__ __forceinline__ double block_sum(const double* __restrict__ v, int n, double* red)
+{
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += MD_BLOCK) acc += v[i];
+    acc = wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
     __syncthreads();
-    for (int i = threadIdx.x; i < k; i += MD_BLOCK) {
-        double sum = 0.0;
+    return (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+template <int P>
+__global__ void __launch_bounds__(MD_BLOCK) lz_dot_k(const double* __restrict__ v, const double* __restrict__ w,
+                                                     long n, double* __restrict__ part)
+{
+    __shared__ double red[4];
+    double acc = 0.0;
 #pragma unroll
-        for (int q = 0; q < MD_BLOCK / 64; q++) sum += red[i][q];
-        part[(long)i * gridDim.x + blockIdx.x] = sum;
+    for (int e = 0; e < P; e++) {
+        const long idx = 2 * ((long)(blockIdx.x * P + e) * MD_BLOCK + threadIdx.x);
+        if (idx < n) {
+            const double2 a = *(const double2*)(v + idx), b = *(const double2*)(w + idx);
+            acc += a.x * b.x + a.y * b.y;
+        }
+    }
+    acc = wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+}
+
+// na > 0: alpha = sum apart[0..na), w <- y - alpha V_{k-1} - beta V_{k-2} (the
+// latter when k >= 2), alpha to aout[0]; na = 0: w is read as it is.  Then
+// part[i*gridDim.x + block] = V_i . w over the block's entries, for the ng
+// vectors i of block row blockIdx.y (w is formed by every block row, written
+// by the first: y and w are different buffers).
+template <int P>
+__global__ void __launch_bounds__(MD_BLOCK) lz_step_k(const double* __restrict__ y, double* __restrict__ w,
+                                                      const double* __restrict__ V, long ldv, int k,
+                                                      const double* __restrict__ apart, int na,
+                                                      double* __restrict__ aout, double beta, long n, int ng,
+                                                      double* __restrict__ part)
+{
+    __shared__ double ared[4];
+    __shared__ double red[2][8][4];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const long c0 = (long)blockIdx.x * 2 * MD_BLOCK * P;
+    double2 x[P];
+    if (na > 0) {
+        const double* vj = V + (long)(k - 1) * ldv;
+        const double* vm = k >= 2 ? V + (long)(k - 2) * ldv : vj;
+        const double b = k >= 2 ? beta : 0.0;
+        double2 p[P], q[P];
+#pragma unroll
+        for (int e = 0; e < P; e++) {
+            const long idx = c0 + 2 * (e * MD_BLOCK + tid);
+            const bool in = idx < n;
+            x[e] = in ? *(const double2*)(y + idx) : make_double2(0.0, 0.0);
+            p[e] = in ? *(const double2*)(vj + idx) : make_double2(0.0, 0.0);
+            q[e] = in ? *(const double2*)(vm + idx) : make_double2(0.0, 0.0);
+        }
+        const double a = block_sum(apart, na, ared);
+        if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) aout[0] = a;
+#pragma unroll
+        for (int e = 0; e < P; e++) {
+            x[e].x -= a * p[e].x;
+            x[e].y -= a * p[e].y;
+            x[e].x -= b * q[e].x;
+            x[e].y -= b * q[e].y;
+            const long idx = c0 + 2 * (e * MD_BLOCK + tid);
+            if (blockIdx.y == 0 && idx < n) *(double2*)(w + idx) = x[e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < P; e++) {
+            const long idx = c0 + 2 * (e * MD_BLOCK + tid);
+            x[e] = idx < n ? *(const double2*)(w + idx) : make_double2(0.0, 0.0);
+        }
+    }
+    const int i1 = min(k, (int)(blockIdx.y + 1) * ng);
+    int par = 0;
+    for (int i0 = blockIdx.y * ng; i0 < i1; i0 += 8, par ^= 1) {
+        // eight vectors at a time: their loads and their lane reductions are
+        // independent (a vector past the last one repeats it and is dropped)
+        double acc[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const double* vi = V + (long)min(i0 + u, i1 - 1) * ldv;
+            double s = 0.0;
+#pragma unroll
+            for (int e = 0; e < P; e++) {
+                const long idx = c0 + 2 * (e * MD_BLOCK + tid);
+                if (idx < n) {
+                    const double2 v = *(const double2*)(vi + idx);
+                    s += v.x * x[e].x + v.y * x[e].y;
+                }
+            }
+            acc[u] = s;
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1)
+#pragma unroll
+            for (int u = 0; u < 8; u++) acc[u] += __shfl_xor(acc[u], o, 64);
+        if (lane == 0) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) red[par][u][wid] = acc[u];
+        }
+        __syncthreads();  // the other slot of red is read before the next round's barrier
+        if (tid < 8 && i0 + tid < i1)
+            part[(long)(i0 + tid) * gridDim.x + blockIdx.x] =
+                (red[par][tid][0] + red[par][tid][1]) + (red[par][tid][2] + red[par][tid][3]);
     }
 }
 
-__global__ void __launch_bounds__(MD_BLOCK) lz_update_norm_k(double* __restrict__ w, const double* __restrict__ V,
-                                                             long ldv, int k, const double* __restrict__ coef,
-                                                             long n, double* __restrict__ part)
+// c_i = sum_b part[i*G + b] (G > 0; written to coef by the first workgroup) or
+// coef[i] (G = 0); w <- w - sum_{i<k} c_i V_i; npart[block] = |w|^2 over the
+// block's entries.  KG groups of MD_BLOCK / KG threads take every KG-th
+// vector, each thread P pairs of entries: (4, 1) for short vectors (128
+// entries per workgroup), (1, 4) for long ones.  Workgroups walk the entries in
+// the reverse order of lz_step, whose last reads of the basis are still in the
+// last-level cache when the basis exceeds it.
+template <int KG, int P>
+__global__ void __launch_bounds__(MD_BLOCK) lz_update_k(double* __restrict__ w, const double* __restrict__ V,
+                                                        long ldv, int k, const double* __restrict__ part, int G,
+                                                        double* __restrict__ coef, long n,
+                                                        double* __restrict__ npart)
 {
+    constexpr int TG = MD_BLOCK / KG;
     __shared__ double c[MD_MAXK];
-    __shared__ double red[MD_BLOCK / 64];
-    for (int i = threadIdx.x; i < k; i += MD_BLOCK) c[i] = coef[i];
-    __syncthreads();
-    const int blk = gridDim.x - 1 - blockIdx.x;
-    const long c0 = (long)blk * MD_BLOCK * MD_EPT;
-    double2 acc[LZ_PAIRS];
-#pragma unroll
-    for (int e = 0; e < LZ_PAIRS; e++) {
-        const long idx = c0 + 2 * ((long)e * MD_BLOCK + threadIdx.x);
-        acc[e] = idx < n ? *(const double2*)(w + idx) : make_double2(0.0, 0.0);
+    __shared__ double2 sub[KG][TG * P];
+    __shared__ double red[4];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int t = tid % TG, kg = tid / TG;
+    if (G == 0) {
+        for (int i = tid; i < k; i += MD_BLOCK) c[i] = coef[i];
+    } else if (G <= 64) {
+        for (int i = tid; i < k; i += MD_BLOCK) {
+            double s = 0.0;
+#pragma unroll 8
+            for (int b = 0; b < G; b++) s += part[(long)i * G + b];
+            c[i] = s;
+        }
+    } else {
+        for (int i = wid; i < k; i += 4) {
+            double s = 0.0;
+            for (int b = lane; b < G; b += 64) s += part[(long)i * G + b];
+            s = wave_sum(s);
+            if (lane == 0) c[i] = s;
+        }
     }
-    for (int i = 0; i < k; i++) {
+    __syncthreads();
+    if (G > 0 && blockIdx.x == 0)
+        for (int i = tid; i < k; i += MD_BLOCK) coef[i] = c[i];
+    const int blk = gridDim.x - 1 - blockIdx.x;
+    const long c0 = (long)blk * 2 * TG * P;
+    double2 acc[P];
+#pragma unroll
+    for (int e = 0; e < P; e++) acc[e] = make_double2(0.0, 0.0);
+#pragma unroll 4
+    for (int i = kg; i < k; i += KG) {
         const double* vi = V + (long)i * ldv;
         const double ci = c[i];
 #pragma unroll
-        for (int e = 0; e < LZ_PAIRS; e++) {
-            const long idx = c0 + 2 * ((long)e * MD_BLOCK + threadIdx.x);
+        for (int e = 0; e < P; e++) {
+            const long idx = c0 + 2 * ((long)e * TG + t);
             if (idx < n) {
                 const double2 p = *(const double2*)(vi + idx);
-                acc[e].x -= ci * p.x;
-                acc[e].y -= ci * p.y;
+                acc[e].x += ci * p.x;
+                acc[e].y += ci * p.y;
             }
         }
     }
-    double sq = 0.0;
+    if constexpr (KG > 1) {
 #pragma unroll
-    for (int e = 0; e < LZ_PAIRS; e++) {
-        const long idx = c0 + 2 * ((long)e * MD_BLOCK + threadIdx.x);
-        if (idx < n) {
-            *(double2*)(w + idx) = acc[e];
-            sq += acc[e].x * acc[e].x + acc[e].y * acc[e].y;
+        for (int e = 0; e < P; e++) sub[kg][e * TG + t] = acc[e];
+        __syncthreads();
+    }
+    double sq = 0.0;
+    if (kg == 0) {
+#pragma unroll
+        for (int e = 0; e < P; e++) {
+            const long idx = c0 + 2 * ((long)e * TG + t);
+            if (idx < n) {
+                double2 x = *(const double2*)(w + idx);
+                double2 s = acc[e];
+                if constexpr (KG > 1) {
+#pragma unroll
+                    for (int g = 1; g < KG; g++) {
+                        const double2 o = sub[g][e * TG + t];
+                        s.x += o.x;
+                        s.y += o.y;
+                    }
+                }
+                x.x -= s.x;
+                x.y -= s.y;
+                *(double2*)(w + idx) = x;
+                sq += x.x * x.x + x.y * x.y;
+            }
         }
     }
     sq = wave_sum(sq);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sq;
+    if (lane == 0) red[wid] = sq;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double sum = 0.0;
-#pragma unroll
-        for (int q = 0; q < MD_BLOCK / 64; q++) sum += red[q];
-        part[blk] = sum;
-    }
+    if (tid == 0) npart[blk] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-hipError_t lz_step_dots(double* w, const double* V, long ldv, int k, const double* alpha, double beta, long n,
-                        double* out, double* part, long part_cap, hipStream_t s)
+hipError_t lz_dot(const double* v, const double* w, long n, double* part, hipStream_t s)
 {
-    const long G = (n + MD_BLOCK * MD_EPT - 1) / (MD_BLOCK * MD_EPT);
-    if (k < 1 || k > MD_MAXK || (n & 1) || G * k > part_cap) return hipErrorInvalidValue;
-    lz_step_dots_k<<<G, MD_BLOCK, 0, s>>>(w, V, ldv, k, alpha, beta, n, part);
-    mdot2_k<<<k, 256, 0, s>>>(part, (int)G, out);
+    if (n <= 0 || (n & 1)) return hipErrorInvalidValue;
+    const int G = (int)lz_dot_blocks(n);
+    if (n <= LZ_SMALL) lz_dot_k<1><<<G, MD_BLOCK, 0, s>>>(v, w, n, part);
+    else lz_dot_k<4><<<G, MD_BLOCK, 0, s>>>(v, w, n, part);
     return hipGetLastError();
 }
 
-hipError_t lz_update_norm(double* w, const double* V, long ldv, int k, const double* coef, long n, double* out,
-                          double* part, long part_cap, hipStream_t s)
+hipError_t lz_step(const double* y, double* w, const double* V, long ldv, int k, bool three, double beta, long n,
+                   double* h, double* part, hipStream_t s)
 {
-    const long G = (n + MD_BLOCK * MD_EPT - 1) / (MD_BLOCK * MD_EPT);
-    if (k < 1 || k > MD_MAXK || (n & 1) || G > part_cap) return hipErrorInvalidValue;
-    lz_update_norm_k<<<G, MD_BLOCK, 0, s>>>(w, V, ldv, k, coef, n, part);
-    mdot2_k<<<1, 256, 0, s>>>(part, (int)G, out);
+    if (k < 1 || k > MD_MAXK || n <= 0 || (n & 1) || (three && y == w)) return hipErrorInvalidValue;
+    const long G = lz_step_blocks(n, k), na = lz_dot_blocks(n);
+    double* dots = part + na + lz_norm_blocks(n);
+    // block rows of eight or more vectors each until the chip is full
+    const int groups = (k + 7) / 8;
+    const int S = (int)(G >= 512 ? 1 : (512 / G < groups ? 512 / G : groups));
+    const int ng = 8 * ((groups + S - 1) / S);
+    const dim3 grid(G, (k + ng - 1) / ng);
+    const int nap = three ? (int)na : 0;
+    if (lz_step_pairs(n, k) == 1) lz_step_k<1><<<grid, MD_BLOCK, 0, s>>>(y, w, V, ldv, k, part, nap, h, beta, n, ng, dots);
+    else lz_step_k<4><<<grid, MD_BLOCK, 0, s>>>(y, w, V, ldv, k, part, nap, h, beta, n, ng, dots);
+    return hipGetLastError();
+}
+
+hipError_t lz_update(double* w, const double* V, long ldv, int k, long n, double* coef, double* part, hipStream_t s)
+{
+    if (k < 1 || k > MD_MAXK || n <= 0 || (n & 1)) return hipErrorInvalidValue;
+    int G = (int)lz_step_blocks(n, k);
+    double* npart = part + lz_dot_blocks(n);
+    double* dots = npart + lz_norm_blocks(n);
+    // summing the partial dots in every workgroup costs k*G reads each: for
+    // long vectors and more than a few coefficients a launch of its own is
+    // cheaper
+    if (G > 64 && k > 8) {
+        mdot2_k<<<k, 256, 0, s>>>(dots, G, coef);
+        G = 0;
+    }
+    const int Gn = (int)lz_norm_blocks(n);
+    if (n <= LZ_SMALL) lz_update_k<4, 1><<<Gn, MD_BLOCK, 0, s>>>(w, V, ldv, k, dots, G, coef, n, npart);
+    else lz_update_k<1, 4><<<Gn, MD_BLOCK, 0, s>>>(w, V, ldv, k, dots, G, coef, n, npart);
+    return hipGetLastError();
+}
+
+// h[0..nh) and then sum npart[0..G) (|w|^2) to the host, as publish does
+__global__ void __launch_bounds__(MD_BLOCK) lz_publish_k(const double* __restrict__ h, int nh,
+                                                         const double* __restrict__ npart, int G, double* host_dst,
+                                                         unsigned long long* host_flag, unsigned long long seq)
+{
+    __shared__ double red[4];
+    const double nn = block_sum(npart, G, red);
+    for (int t = threadIdx.x; t < nh; t += MD_BLOCK) host_dst[t] = h[t];
+    if (threadIdx.x == 0) host_dst[nh] = nn;
+    __threadfence_system();  // every wave's stores before the flag (see publish_k)
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        __threadfence_system();
+        *(volatile unsigned long long*)host_flag = seq;
+    }
+}
+
+hipError_t lz_publish(const double* h, int nh, long n, const double* part, double* host_dst,
+                      unsigned long long* host_flag, unsigned long long seq, hipStream_t s)
+{
+    if (nh < 0 || nh >= TN_PUBLISH_MAX) return hipErrorInvalidValue;
+    lz_publish_k<<<1, MD_BLOCK, 0, s>>>(h, nh, part + lz_dot_blocks(n), (int)lz_norm_blocks(n), host_dst, host_flag,
+                                        seq);
     return hipGetLastError();
 }
 
@@ -1892,26 +2079,6 @@ hipError_t axpby(double a, const double* x, double b, double* y, long n, hipStre
     long blocks = (n + 255) / 256;
     if (blocks > 8192) blocks = 8192;
     axpby_k<<<blocks, 256, 0, s>>>(a, x, b, y, n);
-    return hipGetLastError();
-}
-
-// w -= alpha[0] v + beta u   (the three-term Lanczos step; alpha on the device)
-__global__ void three_term_k(double* __restrict__ w, const double* __restrict__ v, const double* __restrict__ u,
-                             const double* __restrict__ alpha, double beta, long n)
-{
-    const double a = alpha[0];
-    for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-        double r = w[i] - a * v[i];
-        if (u) r -= beta * u[i];
-        w[i] = r;
-    }
-}
-hipError_t three_term(double* w, const double* v, const double* u, const double* alpha, double beta, long n,
-                      hipStream_t s)
-{
-    long blocks = (n + 255) / 256;
-    if (blocks > 8192) blocks = 8192;
-    three_term_k<<<blocks, 256, 0, s>>>(w, v, u, alpha, beta, n);
     return hipGetLastError();
 }
 
@@ -2767,7 +2934,7 @@ hipError_t bmdot(const DotJob* jobs, int n, int kmax, long nmax, double* part, h
 long bmdot_part_size(int n, int kmax, long nmax) { return (long)n * kmax * ((nmax + BV_CHUNK - 1) / BV_CHUNK); }
 
 // Fused Lanczos step, batched: block (b, q) owns chunk b of job q's vectors
-// (BV_CHUNK entries as BV_EPT / 2 pairs per thread), the layout of lz_step_dots_k.
+// (BV_CHUNK entries as BV_EPT / 2 pairs per thread), no split of the basis vectors.
 #define BV_PAIRS (BV_EPT / 2)
 __global__ void __launch_bounds__(BV_BLOCK) bstep_dots_k(const StepJob* __restrict__ jobs, int kmax, int G,
                                                          double* __restrict__ part)
@@ -2851,7 +3018,7 @@ hipError_t bstep_dots(const StepJob* jobs, int n, int kmax, long nmax, double* p
     return hipGetLastError();
 }
 
-// chunks in reverse order of bstep_dots_k (see lz_update_norm_k)
+// chunks in reverse order of bstep_dots_k (see lz_update_k)
 __global__ void __launch_bounds__(BV_BLOCK) bupdate_norm_k(const UpdJob* __restrict__ jobs, int G,
                                                            double* __restrict__ part)
 {
