@@ -30,8 +30,8 @@ HIP_FLAGS = [
     "-Wno-unused-result", "-I", INCLUDE,
 ]
 
-HIP_SOURCES = ["hip/tn_kernels.hip", "hip/tn_engine.hip", "hip/tn_chain.hip", "hip/tn_batch.hip", "hip/tn_precond.hip"]
-HIP_HEADERS = ["hip/tn_kernels.h", "hip/tn_engine.h", "hip/tn_chain.h"]
+HIP_SOURCES = ["hip/tn_gemm.hip", "hip/tn_kernels.hip", "hip/tn_engine.hip", "hip/tn_chain.hip", "hip/tn_batch.hip", "hip/tn_precond.hip"]
+HIP_HEADERS = ["hip/tn_kernels.h", "hip/tn_device.h", "hip/tn_engine.h", "hip/tn_chain.h"]
 CXX_SOURCES = ["host/tensornetworks.cpp"]
 CXX_HEADERS = []
 # host-only C++ linked into the ABI library (no device code)
@@ -85,7 +85,7 @@ def _compile_host(src):
 def build(verbose=True):
     os.makedirs(LIBDIR, exist_ok=True)
     os.makedirs(BUILD, exist_ok=True)
-    with ThreadPoolExecutor(max_workers=4) as ex:
+    with ThreadPoolExecutor(max_workers=6) as ex:
         objs = list(ex.map(_compile_hip, HIP_SOURCES))
     objs += [_compile_host(s) for s in ABI_HOST_SOURCES]
     lib = os.path.join(LIBDIR, "libtn_hip.so")
