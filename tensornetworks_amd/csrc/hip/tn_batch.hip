@@ -214,7 +214,7 @@ std::vector<GroupLaunch> gemm_group_stage(tn_batch* b, const std::vector<GemmDes
                        g.a_kmajor == list[0].a_kmajor && g.b_kmajor == list[0].b_kmajor,
                    TN_ERR_ARG, "gemm_group: mixed problem types");
         int tile = gemm_choice(c, g).first;
-        if (!gemm_tile_ok(tile, g.tin, g.M, g.N, g.K)) tile = gemm_default_tile(g.M, g.N, 1);
+        if (!gemm_tile_ok(tile, g.tin, g.M, g.N, g.K)) tile = gemm_grouped_tile(g.M, g.N);
         groups[{tile, gemm_k_step(g.tin, g.K)}].push_back(q);
     }
     for (const auto& kv : groups) {

@@ -122,12 +122,18 @@ namespace tn {
 
 // GEMM on the context's stream.  With g.tile == 0 and ctx->autotune set, the
 // tile and k-split come from the per-shape table (tuned on first use by timing
-// every candidate into scratch memory); otherwise the built-in choice.
-void gemm_run(tn_ctx* c, const GemmDesc& g);
+// every candidate into scratch memory); otherwise from gemm_default.
+// Every tile sums over k in increasing order, so the result does not depend on
+// the built-in choice unless it splits k; split = true allows that (FP64
+// environments and the Heff stages; not gauge moves, whose rounding decides the
+// basis of nearly dependent columns, nor reduced-precision environments, whose
+// rounding reaches the energies).
+void gemm_run(tn_ctx* c, const GemmDesc& g, bool split = false);
 // the same GEMM with an explicit k-split (ks > 1 needs batch == 1, K % (64 ks) == 0)
 void gemm_split(tn_ctx* c, const GemmDesc& g, int ks);
-// (tile code, k-split) gemm_run would use for g (tuning it first when
-// autotuning is on and the shape is new)
+// (tile code, k-split) of a problem in a grouped launch: the tuning table's
+// (tuned first when autotuning is on and the shape is new), else the built-in
+// tile
 std::pair<int, int> gemm_choice(tn_ctx* c, const GemmDesc& g);
 
 // --- effective Hamiltonian operator (internal padded layout) -------------

@@ -157,14 +157,21 @@ std::pair<int, int> gemm_choice(tn_ctx* c, const GemmDesc& g)
     const std::array<long, 9> key{g.tin, g.tout, g.a_kmajor, g.b_kmajor, g.M, g.N, g.K, g.batch, g.accumulate};
     auto it = c->tune.find(key);
     if (it != c->tune.end()) return it->second;
-    if (!c->autotune) return {gemm_default_tile(g.M, g.N, g.batch), 1};
+    if (!c->autotune) return {gemm_grouped_tile(g.M, g.N), 1};
     return c->tune.emplace(key, tune_gemm(c, g)).first->second;
 }
 
-void gemm_run(tn_ctx* c, const GemmDesc& g)
+void gemm_run(tn_ctx* c, const GemmDesc& g, bool split)
 {
-    if (g.tile != 0 || !c->autotune) {
+    if (g.tile != 0) {
         TN_HIP(gemm(g, c->stream));
+        return;
+    }
+    if (!c->autotune) {
+        GemmDesc t = g;
+        int ks = 1;
+        gemm_default(g.tin, g.M, g.N, g.K, g.batch, split, &t.tile, &ks);
+        gemm_split(c, t, ks);
         return;
     }
     const std::array<long, 9> key{g.tin, g.tout, g.a_kmajor, g.b_kmajor, g.M, g.N, g.K, g.batch, g.accumulate};
@@ -324,7 +331,9 @@ void gemm_run_fixed(tn_ctx* c, const GemmDesc& g)
     if (t.tile == 0) {
         const std::array<long, 9> key{g.tin, g.tout, g.a_kmajor, g.b_kmajor, g.M, g.N, g.K, g.batch, g.accumulate};
         auto it = c->tune.find(key);
-        t.tile = it != c->tune.end() ? it->second.first : gemm_default_tile(g.M, g.N, g.batch);
+        int ks;
+        if (it != c->tune.end()) t.tile = it->second.first;
+        else gemm_default(g.tin, g.M, g.N, g.K, g.batch, false, &t.tile, &ks);
     }
     TN_HIP(gemm(t, c->stream));
 }
@@ -409,7 +418,7 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
     }
     auto run = [&](const GemmDesc& g) {
         if (scr) gemm_run_fixed(c, g);
-        else gemm_run(c, g);
+        else gemm_run(c, g, true);
     };
     if (op.precision == TN_FP64) {
         if (!scr) {
@@ -546,11 +555,11 @@ void env_left(tn_ctx* c, int prec, int p, int D1p, int D2p, int Dw1, int Dw2, co
         c->T1.ensure(nX * 8);
         c->T2.ensure(nY * 8);
         e1.tin = T_F64; e1.tout = T_F64; e1.A = Lin; e1.B = A; e1.C = c->T1.p;
-        gemm_run(c, e1);
+        gemm_run(c, e1, true);
         TN_HIP(wmix(T_F64, T_F64, c->T1.p, (long)Dw1 * p * D2p, c->T2.p, (long)p * Dw2 * D2p, D1p,
                     D2p, mix.t, s));
         e3.tin = T_F64; e3.tout = T_F64; e3.A = A; e3.B = c->T2.p; e3.C = Lout;
-        gemm_run(c, e3);
+        gemm_run(c, e3, true);
     } else {
         const int tl = lo_type(prec);
         const size_t es = dtype_size(tl);
@@ -588,11 +597,11 @@ void env_right(tn_ctx* c, int prec, int p, int D1p, int D2p, int Dw1, int Dw2, c
         c->T1.ensure(nX * 8);
         c->T2.ensure(nY * 8);
         f1.tin = T_F64; f1.tout = T_F64; f1.A = A; f1.B = Rin; f1.C = c->T1.p;
-        gemm_run(c, f1);
+        gemm_run(c, f1, true);
         TN_HIP(wmix(T_F64, T_F64, c->T1.p, (long)p * Dw2 * D2p, c->T2.p, (long)Dw1 * p * D2p, D1p,
                     D2p, mix.t, s));
         f3.tin = T_F64; f3.tout = T_F64; f3.A = A; f3.B = c->T2.p; f3.C = Rout;
-        gemm_run(c, f3);
+        gemm_run(c, f3, true);
     } else {
         const int tl = lo_type(prec);
         const size_t es = dtype_size(tl);

@@ -1,10 +1,12 @@
 // tn_gemm.hip -- the matrix-core GEMMs (gfx950).
 //
-// * gemm_k     : LDS-tiled GEMM on the matrix cores (v_mfma 16x16, fp64/fp32/bf16
-//                operands, fp32/fp64 accumulate), register-prefetch pipelined,
-//                XCD-aware tile order.  The three stages of Heff*psi and of the
-//                environment updates (MPSSite_Contractions.C:155-400) are GEMMs
-//                once the MPO index is mixed (wmix, tn_kernels.hip).
+// * gemm_pipe_k : FP64 and FP32 GEMM (v_mfma 16x16x4), operands copied straight
+//                into LDS, several stages deep, XCD-aware tile order.  The three
+//                stages of Heff*psi and of the environment updates
+//                (MPSSite_Contractions.C:155-400) are GEMMs once the MPO index is
+//                mixed (wmix, tn_kernels.hip).
+// * gemm_grouped_k : one launch over the tiles of many problems.
+// * gemm_k     : bf16 GEMM, register-prefetch pipelined.
 // * gemm_x3_k  : the split-bfloat16 product.
 // * x3_stage1_mix_k : its Heff stage 1 with the MPO stage in the epilogue.
 #include "tn_device.h"
@@ -195,6 +197,224 @@ __global__ void __launch_bounds__(256) gemm_k(GemmParams p)
     gemm_tile<TI, TO, BM, BN, BK, AKM, BKM>((const TI*)p.A + bz * p.sA, (const TI*)p.B + bz * p.sB,
                                             (TO*)p.C + bz * p.sC, p.lda, p.ldb, p.ldc, p.K, p.alpha,
                                             p.accumulate, tm * BM, tn * BN, As, Bs);
+}
+
+// ---------------------------------------------------------------------------
+// FP64 and FP32 tiles, staged by the copy engine of the vector memory path:
+// global memory straight into LDS (no registers, no LDS store instructions),
+// S stages deep, one barrier per K step.  Bound by the matrix pipes once two
+// waves per SIMD are resident; what the register-staged loop (gemm_tile) lost
+// was the wait for its stores and its second barrier per step.  FP64,
+// 3072 x 4096 x 1024: 419 us (register-staged, its best tile) -> 364 us, 70.7
+// of the 72.6 TFLOP/s a large library product reaches.
+//
+// An operand stage holds 128 bytes of K per row as 16-byte units (K-major
+// operands: [row][unit], row-major ones: [k][row]).  A copy writes 64
+// consecutive units in lane order, so the bank swizzle is applied to the
+// global address: slot u of row r holds unit u ^ (r & 7) (K-major), slot u of
+// k-row k holds unit u ^ sw(k) (row-major).  Fragment reads then touch every
+// bank once per 128 bytes.
+__device__ __forceinline__ uint32_t lds_offset(const void* p)
+{
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
+}
+// 64 lanes copy 16 bytes each from base + off (off per lane) to LDS address
+// dst + 16 * lane (dst uniform)
+__device__ __forceinline__ void copy_to_lds(const void* base, uint32_t off, uint32_t dst)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(dst), "v"(off), "s"(base)
+                 : "memory");
+}
+// all but the last N copies have arrived and every LDS read has returned
+template <int N> __device__ __forceinline__ void wait_copies()
+{
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");
+}
+
+// one operand's stage: ROWS x BK values, loads and fragment reads
+template <typename TI, int ROWS, int BK, bool KM> struct Stage {
+    static constexpr int E = 16 / sizeof(TI);          // values per unit
+    static constexpr int UNITS = ROWS * BK / E;        // units per stage
+    static constexpr int UPK = BK / E;                 // units per row (K-major)
+    static constexpr int UPR = ROWS / E;               // units per k-row (row-major)
+    static constexpr bool F64 = sizeof(TI) == 8;
+    static __device__ __forceinline__ int rsw(int row)
+    {
+        return UPK == 8 && !F64 ? (row & 7) : ((row >> 1) & (UPK - 1));
+    }
+    static __device__ __forceinline__ int ksw(int k)
+    {
+        return (F64 ? (((k >> 1) & 1) << 3) : ((k & 3) << 2)) & (UPR - 1);
+    }
+    // byte offset, from the operand's first row and K index of the step, of the
+    // unit that slot `slot` holds
+    static __device__ __forceinline__ uint32_t goff(int slot, long ld)
+    {
+        if constexpr (KM) {
+            const int row = slot / UPK, u = (slot % UPK) ^ rsw(row);
+            return (uint32_t)((row * ld + u * E) * (long)sizeof(TI));
+        } else {
+            const int k = slot / UPR, u = (slot % UPR) ^ ksw(k);
+            return (uint32_t)((k * ld + u * E) * (long)sizeof(TI));
+        }
+    }
+    // values between the starts of consecutive K steps
+    static __device__ __forceinline__ long kstep(long ld) { return KM ? (long)BK : (long)BK * ld; }
+    // operand(row, k)
+    static __device__ __forceinline__ TI at(const TI* S, int row, int k)
+    {
+        if constexpr (KM) return S[row * BK + (((k / E) ^ rsw(row)) * E) + k % E];
+        else return S[k * ROWS + ((row / E) ^ ksw(k)) * E + row % E];
+    }
+    // FP64: operand(row, 2u) and operand(row, 2u + 1)
+    static __device__ __forceinline__ double2 pair(const TI* S, int row, int u)
+    {
+        if constexpr (KM) return *(const double2*)(S + row * BK + ((u ^ rsw(row)) * E));
+        else return make_double2(at(S, row, 2 * u), at(S, row, 2 * u + 1));
+    }
+};
+
+template <int BM, int BN, int BK, int S, typename TI> constexpr int stage_bytes()
+{
+    return S * (BM + BN) * BK * (int)sizeof(TI);
+}
+
+// One BM x BN output tile: WGM x WGN waves of (BM / WGM) x (BN / WGN).  The
+// caller's LDS holds S stages (stage_bytes) and is free when the tile starts;
+// every copy has arrived and every LDS read has returned when it ends, but
+// other waves may still be reading (barrier before reusing the LDS).
+//
+// Sums over k in increasing order for every tile shape and operand layout (a
+// 16-byte FP64 fragment read, two k per lane, would give another order and only
+// 2-4 % more speed at 3072 x 4096 x 1024).
+template <typename TI, typename TO, int BM, int BN, int BK, int WGM, int WGN, int S, bool AKM, bool BKM>
+__device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __restrict__ B, TO* __restrict__ C,
+                                          long lda, long ldb, long ldc, int K, float alpha, int accumulate, int m0,
+                                          int n0, TI* __restrict__ sm)
+{
+    typedef MT<TI> T;
+    typedef typename T::acc_t acc_t;
+    typedef Stage<TI, BM, BK, AKM> SA;
+    typedef Stage<TI, BN, BK, BKM> SB;
+    constexpr int NW = WGM * WGN, WM = BM / WGM, WN = BN / WGN, FM = WM / 16, FN = WN / 16;
+    constexpr int CA = SA::UNITS / 64, CB = SB::UNITS / 64, CH = CA + CB;
+    static_assert(FM * 16 * WGM == BM && FN * 16 * WGN == BN, "wave tile");
+    static_assert(CA * 64 == SA::UNITS && CB * 64 == SB::UNITS && CH % NW == 0, "copies per wave");
+    constexpr int L = CH / NW;              // copies per wave and step
+    constexpr int STG = (BM + BN) * BK;     // values per stage
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm0 = (wid / WGN) * WM, wn0 = (wid % WGN) * WN;
+    const int r = lane & 15, kq = lane >> 4;
+
+    const TI* Ab = AKM ? A + (long)m0 * lda : A + m0;
+    const TI* Bb = BKM ? B + (long)n0 * ldb : B + n0;
+    uint32_t off[L];
+#pragma unroll
+    for (int i = 0; i < L; i++) {
+        const int c = wid * L + i;
+        off[i] = c < CA ? SA::goff(c * 64 + lane, lda) : SB::goff((c - CA) * 64 + lane, ldb);
+    }
+    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_offset(sm));
+    const long ka = SA::kstep(lda), kb = SB::kstep(ldb);
+    auto issue = [&](int st) {  // the next K step into stage st
+#pragma unroll
+        for (int i = 0; i < L; i++) {
+            const int c = wid * L + i;
+            copy_to_lds(c < CA ? (const void*)Ab : (const void*)Bb, off[i],
+                        base + (uint32_t)(st * STG * (int)sizeof(TI) + c * 1024));
+        }
+        Ab += ka;
+        Bb += kb;
+    };
+    acc_t acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[i][j][q] = 0;
+
+    const int nk = K / BK;
+#pragma unroll
+    for (int t = 0; t < S - 1; t++)
+        if (t < nk) issue(t);
+    int st = 0;
+    for (int t = 0; t < nk; t++) {
+        // stage st has arrived (this wave's copies, then, past the barrier,
+        // everyone's), and everyone is done reading the stage before it
+        if (t + S - 2 < nk) wait_copies<(S - 2) * L>();
+        else wait_copies<0>();
+        __builtin_amdgcn_s_barrier();
+        if (t + S - 1 < nk) issue(st == 0 ? S - 1 : st - 1);
+        const TI* As = sm + st * STG;
+        const TI* Bs = As + BM * BK;
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int kk = 0; kk < BK; kk += 4) {
+                TI a[FM], b[FN];
+#pragma unroll
+                for (int i = 0; i < FM; i++) a[i] = SA::at(As, wm0 + i * 16 + r, kk + kq);
+#pragma unroll
+                for (int j = 0; j < FN; j++) b[j] = SB::at(Bs, wn0 + j * 16 + r, kk + kq);
+#pragma unroll
+                for (int i = 0; i < FM; i++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++) acc[i][j] = mma(a[i], b[j], acc[i][j]);
+            }
+        __builtin_amdgcn_s_setprio(0);
+        asm volatile("" : : : "memory");
+        st = st + 1 == S ? 0 : st + 1;
+    }
+    wait_copies<0>();
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const long row = m0 + wm0 + i * 16 + T::crow(lane, q);
+                const long col = n0 + wn0 + j * 16 + r;
+                TO* cp = C + row * ldc + col;
+                if constexpr (std::is_same<TO, double>::value) {
+                    double v = (double)acc[i][j][q] * (double)alpha;
+                    if (accumulate) v += to_d(*cp);
+                    *cp = v;
+                } else {
+                    float v = (float)acc[i][j][q] * alpha;
+                    if (accumulate) v += to_f(*cp);
+                    *cp = cvt_from_f<TO>(v);
+                }
+            }
+}
+
+// XCD-aware tile order: consecutive block ids land on different XCDs, so each
+// XCD gets a contiguous range of tiles, and inside it 8 tile rows at a time go
+// column by column (tiles resident together share 8 row blocks of A and a few
+// column blocks of B)
+__device__ __forceinline__ void tile_of_block(int bid, int ntm, int ntn, int& tm, int& tn)
+{
+    const int nblk = ntm * ntn;
+    if ((nblk & 7) == 0) bid = (bid & 7) * (nblk >> 3) + (bid >> 3);
+    constexpr int GM = 8;
+    const int gsz = GM * ntn, g = bid / gsz, first = g * GM;
+    const int rows = ntm - first < GM ? ntm - first : GM;
+    const int local = bid - g * gsz;
+    tm = first + local % rows;
+    tn = local / rows;
+}
+
+template <typename TI, typename TO, int BM, int BN, int BK, int WGM, int WGN, int S, int OCC, bool AKM, bool BKM>
+__global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_pipe_k(GemmParams p)
+{
+    __shared__ __attribute__((aligned(1024))) TI sm[stage_bytes<BM, BN, BK, S, TI>() / sizeof(TI)];
+    int tm, tn;
+    tile_of_block(blockIdx.x, p.M / BM, p.N / BN, tm, tn);
+    const long bz = blockIdx.y;
+    pipe_tile<TI, TO, BM, BN, BK, WGM, WGN, S, AKM, BKM>((const TI*)p.A + bz * p.sA, (const TI*)p.B + bz * p.sB,
+                                                         (TO*)p.C + bz * p.sC, p.lda, p.ldb, p.ldc, p.K, p.alpha,
+                                                         p.accumulate, tm * BM, tn * BN, sm);
 }
 
 // Split-product LDS layout for BK = 32: rows of 64 bytes without padding,
@@ -542,13 +762,11 @@ __global__ void __launch_bounds__(512) gemm_x3w_k(GemmX3Params p)
 // (problem q owns tiles [off[q], off[q+1]), row-major over its N/BN columns).
 // Workgroups stride over the tile list; the owning problem is found by a
 // binary search of off.
-template <typename TI, typename TO, int BM, int BN, int BK, bool AKM, bool BKM>
-__global__ void __launch_bounds__(256) gemm_grouped_k(const GemmProb* __restrict__ probs,
-                                                      const int* __restrict__ off, int nprob)
+template <typename TI, typename TO, int BM, int BN, int BK, int WGM, int WGN, int S, int OCC, bool AKM, bool BKM>
+__global__ void __launch_bounds__(256, OCC) gemm_grouped_k(const GemmProb* __restrict__ probs,
+                                                           const int* __restrict__ off, int nprob)
 {
-    constexpr int LDK = BK + MT<TI>::PAD;
-    __shared__ __attribute__((aligned(16))) TI As[BM * LDK];
-    __shared__ __attribute__((aligned(16))) TI Bs[BN * LDK];
+    __shared__ __attribute__((aligned(1024))) TI sm[stage_bytes<BM, BN, BK, S, TI>() / sizeof(TI)];
     const int total = off[nprob];
     for (int t = blockIdx.x; t < total; t += gridDim.x) {
         int lo = 0, hi = nprob - 1;
@@ -561,8 +779,8 @@ __global__ void __launch_bounds__(256) gemm_grouped_k(const GemmProb* __restrict
         const int local = t - off[lo], ntn = q.N / BN;
         const int tm = local / ntn, tn = local - tm * ntn;
         __syncthreads();  // LDS of the previous tile is free
-        gemm_tile<TI, TO, BM, BN, BK, AKM, BKM>((const TI*)q.A, (const TI*)q.B, (TO*)q.C, q.lda, q.ldb, q.ldc, q.K,
-                                                q.alpha, q.accumulate, tm * BM, tn * BN, As, Bs);
+        pipe_tile<TI, TO, BM, BN, BK, WGM, WGN, S, AKM, BKM>((const TI*)q.A, (const TI*)q.B, (TO*)q.C, q.lda, q.ldb,
+                                                             q.ldc, q.K, q.alpha, q.accumulate, tm * BM, tn * BN, sm);
     }
 }
 
@@ -585,9 +803,10 @@ static const int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 int gemm_num_tiles() { return kNumTiles; }
 const char* gemm_tile_name(int code) { return (code >= 1 && code <= kNumTiles) ? kTiles[code - 1].name : "auto"; }
 
-template <typename TI, typename TO, int BK, bool AKM, bool BKM>
-static hipError_t launch_tile(int code, const GemmParams& p, int batch, hipStream_t s)
+template <typename TO, int BK, bool AKM, bool BKM>
+static hipError_t launch_bf16(int code, const GemmParams& p, int batch, hipStream_t s)
 {
+    typedef bf16 TI;
     const TileCfg& t = kTiles[code];
     dim3 grid((p.M / t.bm) * (p.N / t.bn), batch);
     switch (code) {
@@ -605,49 +824,64 @@ static hipError_t launch_tile(int code, const GemmParams& p, int batch, hipStrea
     return hipGetLastError();
 }
 
-template <typename TI, typename TO, int BK, bool AKM, bool BKM>
-static hipError_t launch_grouped(int code, const GemmProb* probs, const int* off, int nprob, int grid,
-                                 hipStream_t s)
+// FP64 / FP32: waves, LDS stages and workgroups per CU of every tile.  The
+// small tiles have little work between barriers and take four stages; the
+// "deep" codes take one stage more than their plain form.
+#define PIPE_TILES(X)                                                                                       \
+    X(0, 128, 128, 2, 2, 2, 2) X(1, 128, 64, 2, 2, 2, 3) X(2, 64, 128, 2, 2, 2, 3) X(3, 64, 64, 2, 2, 2, 4) \
+    X(4, 32, 64, 1, 4, 4, 3) X(5, 64, 32, 2, 2, 4, 3) X(6, 32, 32, 2, 2, 4, 4) X(7, 128, 128, 2, 2, 3, 1)   \
+    X(8, 128, 64, 2, 2, 3, 2) X(9, 64, 128, 2, 2, 3, 2)
+
+template <typename TI, typename TO, bool AKM, bool BKM>
+static hipError_t launch_pipe(int code, const GemmParams& p, int batch, hipStream_t s)
 {
+    constexpr int BK = 128 / sizeof(TI);
+    if (p.K % BK) {
+        // FP32 with K an odd multiple of 16: the smallest tile on 64-byte rows
+        if constexpr (std::is_same<TI, float>::value) {
+            const dim3 grid((p.M / 32) * (p.N / 32), batch);
+            gemm_pipe_k<TI, TO, 32, 32, 16, 2, 2, 4, 4, AKM, BKM><<<grid, 256, 0, s>>>(p);
+            return hipGetLastError();
+        }
+        return hipErrorInvalidValue;
+    }
+    const TileCfg& t = kTiles[code];
+    const dim3 grid((p.M / t.bm) * (p.N / t.bn), batch);
     switch (code) {
-    case 0: gemm_grouped_k<TI, TO, 128, 128, BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    case 1: gemm_grouped_k<TI, TO, 128, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    case 2: gemm_grouped_k<TI, TO, 64, 128, BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    case 3: gemm_grouped_k<TI, TO, 64, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    case 4: gemm_grouped_k<TI, TO, 32, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    case 5: gemm_grouped_k<TI, TO, 64, 32, BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    case 6: gemm_grouped_k<TI, TO, 32, 32, BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    case 7: gemm_grouped_k<TI, TO, 128, 128, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    case 8: gemm_grouped_k<TI, TO, 128, 64, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
-    default: gemm_grouped_k<TI, TO, 64, 128, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); break;
+#define PIPE_CASE(c, bm, bn, wm, wn, st, occ)                                                      \
+    case c: gemm_pipe_k<TI, TO, bm, bn, BK, wm, wn, st, occ, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+        PIPE_TILES(PIPE_CASE)
+#undef PIPE_CASE
+    default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
 template <typename TI, typename TO, bool AKM, bool BKM>
-static hipError_t grouped_typed(int code, int bk, const GemmProb* probs, const int* off, int nprob, int grid,
-                                hipStream_t s)
+static hipError_t launch_grouped(int code, int bk, const GemmProb* probs, const int* off, int nprob, int grid,
+                                 hipStream_t s)
 {
-    if constexpr (std::is_same<TI, double>::value) {
-        return launch_grouped<TI, TO, 16, AKM, BKM>(code, probs, off, nprob, grid, s);
-    } else if constexpr (std::is_same<TI, float>::value) {
-        if (bk == 32) return launch_grouped<TI, TO, 32, AKM, BKM>(code, probs, off, nprob, grid, s);
-        return launch_grouped<TI, TO, 16, AKM, BKM>(code, probs, off, nprob, grid, s);
-    } else {
-        if (bk == 64) return launch_grouped<TI, TO, 64, AKM, BKM>(code, probs, off, nprob, grid, s);
-        return launch_grouped<TI, TO, 32, AKM, BKM>(code, probs, off, nprob, grid, s);
+    constexpr int BK = 128 / sizeof(TI);
+    if (bk != BK) return hipErrorInvalidValue;
+    switch (code) {
+#define PIPE_CASE(c, bm, bn, wm, wn, st, occ)                                                                       \
+    case c:                                                                                                         \
+        gemm_grouped_k<TI, TO, bm, bn, BK, wm, wn, st, occ, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); \
+        break;
+        PIPE_TILES(PIPE_CASE)
+#undef PIPE_CASE
+    default: return hipErrorInvalidValue;
     }
+    return hipGetLastError();
 }
 
 template <bool AKM, bool BKM>
 static hipError_t grouped_layout(int tin, int tout, int code, int bk, const GemmProb* probs, const int* off,
                                  int nprob, int grid, hipStream_t s)
 {
-    if (tin == T_F64 && tout == T_F64) return grouped_typed<double, double, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
-    if (tin == T_F32 && tout == T_F32) return grouped_typed<float, float, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
-    if (tin == T_F32 && tout == T_F64) return grouped_typed<float, double, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
-    if (tin == T_BF16 && tout == T_F32) return grouped_typed<bf16, float, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
-    if (tin == T_BF16 && tout == T_F64) return grouped_typed<bf16, double, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
+    if (tin == T_F64 && tout == T_F64) return launch_grouped<double, double, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
+    if (tin == T_F32 && tout == T_F32) return launch_grouped<float, float, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
+    if (tin == T_F32 && tout == T_F64) return launch_grouped<float, double, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
     return hipErrorInvalidValue;
 }
 
@@ -711,7 +945,7 @@ bool gemm_tile_ok(int code, int tin, int M, int N, int K)
 }
 int gemm_tile_bm(int code) { return (code >= 1 && code <= kNumTiles) ? kTiles[code - 1].bm : 0; }
 int gemm_tile_bn(int code) { return (code >= 1 && code <= kNumTiles) ? kTiles[code - 1].bn : 0; }
-int gemm_default_tile(int M, int N, int batch) { return choose_tile(M, N, batch) + 1; }
+int gemm_grouped_tile(int M, int N) { return choose_tile(M, N, 1) + 1; }
 int gemm_k_step(int tin, int K)
 {
     if (tin == T_F64) return 16;
@@ -731,8 +965,9 @@ hipError_t gemm_grouped(int tin, int tout, bool akm, bool bkm, int tile, int bk,
     return grouped_layout<false, true>(tin, tout, tile - 1, bk, probs, off, nprob, grid, s);
 }
 
-// Pick the largest tile that divides the problem and still gives >= ~1.5
-// workgroups per CU (256 CUs); fall back to the tile with the most blocks.
+// bf16 and split bf16: pick the largest tile that divides the problem and still
+// gives >= ~1.5 workgroups per CU (256 CUs); fall back to the tile with the
+// most blocks.
 static int choose_tile(int M, int N, int batch)
 {
     int best = -1;
@@ -746,6 +981,52 @@ static int choose_tile(int M, int N, int batch)
     return best;
 }
 
+// FP64 / FP32 tile and k-split from a model of the time, in us, fitted to the
+// tiles timed one by one (M x N x K from 32 x 96 x 128 to 3072 x 4096 x 1024, all
+// layouts; within 8 % of the measured time from 5 us up):
+//   3.7 + steps * max(n * busy, alone)   + for a split  3 + bytes / 10 TB/s
+// steps: K steps (16 FP64, 32 FP32 values) of one workgroup; n: workgroups on the
+// fullest CU; busy: matrix-pipe time of a workgroup's step; alone: the step of a
+// workgroup that has a CU to itself (copy, barrier and instruction latency).
+struct PipeCost { int code; float busy64, alone64, busy32, alone32; };
+static const PipeCost kPipeCost[] = {
+    {1, 0.933f, 1.05f, 1.016f, 1.15f},   // 128x64
+    {2, 0.933f, 1.05f, 1.016f, 1.15f},   // 64x128
+    {3, 0.485f, 0.53f, 0.608f, 0.70f},   // 64x64
+    {4, 0.259f, 0.30f, 0.353f, 0.45f},   // 32x64
+    {5, 0.259f, 0.30f, 0.353f, 0.45f},   // 64x32
+    {6, 0.138f, 0.235f, 0.205f, 0.355f}, // 32x32
+};
+void gemm_default(int tin, int M, int N, int K, int batch, bool split, int* tile, int* ksplit)
+{
+    *ksplit = 1;
+    if (tin != T_F64 && tin != T_F32) {
+        *tile = choose_tile(M, N, batch) + 1;
+        return;
+    }
+    const bool f64 = tin == T_F64;
+    const int bk = f64 ? 16 : 32;
+    float best = 1e30f;
+    *tile = 7;
+    for (const PipeCost& c : kPipeCost) {
+        const TileCfg& t = kTiles[c.code];
+        if (M % t.bm || N % t.bn) continue;
+        for (int ks = 1; ks <= 4; ks *= 2) {
+            if (ks > 1 && (!split || batch != 1 || K % (64 * ks))) break;
+            const long blocks = (long)(M / t.bm) * (N / t.bn) * batch * ks;
+            const float n = (float)((blocks + 255) / 256);
+            const float busy = n * (f64 ? c.busy64 : c.busy32), alone = f64 ? c.alone64 : c.alone32;
+            float us = 3.7f + (float)(K / ks) / bk * (busy > alone ? busy : alone);
+            if (ks > 1) us += 3.0f + (float)M * N * (2 * ks * (f64 ? 8 : 4) + 8) * 1e-7f;
+            if (us < best) {
+                best = us;
+                *tile = c.code + 1;
+                *ksplit = ks;
+            }
+        }
+    }
+}
+
 template <typename TI, typename TO, bool AKM, bool BKM>
 static hipError_t gemm_typed(const GemmDesc& g, hipStream_t s)
 {
@@ -755,21 +1036,22 @@ static hipError_t gemm_typed(const GemmDesc& g, hipStream_t s)
     p.lda = g.lda; p.ldb = g.ldb; p.ldc = g.ldc;
     p.sA = g.sA; p.sB = g.sB; p.sC = g.sC;
     p.alpha = g.alpha; p.accumulate = g.accumulate;
-    int code = g.tile > 0 ? g.tile - 1 : choose_tile(g.M, g.N, g.batch);
+    int code = g.tile - 1;
+    if (g.tile <= 0) {
+        int ks;
+        gemm_default(g.tin, g.M, g.N, g.K, g.batch, false, &code, &ks);
+        code--;
+    }
     if (code < 0 || code >= kNumTiles || kTiles[code].x3only || g.M % kTiles[code].bm || g.N % kTiles[code].bn)
         return hipErrorInvalidValue;
     if (kTiles[code].deep && g.K % (2 * gemm_k_step(g.tin, g.K))) return hipErrorInvalidValue;
-    if constexpr (std::is_same<TI, double>::value) {
-        if (g.K % 16) return hipErrorInvalidValue;
-        return launch_tile<TI, TO, 16, AKM, BKM>(code, p, g.batch, s);
-    } else if constexpr (std::is_same<TI, float>::value) {
-        if (g.K % 32 == 0) return launch_tile<TI, TO, 32, AKM, BKM>(code, p, g.batch, s);
-        if (g.K % 16) return hipErrorInvalidValue;
-        return launch_tile<TI, TO, 16, AKM, BKM>(code, p, g.batch, s);
-    } else {
-        if (g.K % 64 == 0) return launch_tile<TI, TO, 64, AKM, BKM>(code, p, g.batch, s);
+    if constexpr (std::is_same<TI, bf16>::value) {
+        if (g.K % 64 == 0) return launch_bf16<TO, 64, AKM, BKM>(code, p, g.batch, s);
         if (g.K % 32) return hipErrorInvalidValue;
-        return launch_tile<TI, TO, 32, AKM, BKM>(code, p, g.batch, s);
+        return launch_bf16<TO, 32, AKM, BKM>(code, p, g.batch, s);
+    } else {
+        if (g.K % 16) return hipErrorInvalidValue;
+        return launch_pipe<TI, TO, AKM, BKM>(code, p, g.batch, s);
     }
 }
 

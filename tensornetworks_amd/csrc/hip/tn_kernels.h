@@ -61,7 +61,10 @@ int gemm_tile_bm(int code);
 // tile code usable for an M x N x K problem of input type tin
 bool gemm_tile_ok(int code, int tin, int M, int N, int K);
 int gemm_tile_bn(int code);
-int gemm_default_tile(int M, int N, int batch);
+// built-in choice of the tile code and, with split (batch 1), of the k-split
+void gemm_default(int tin, int M, int N, int K, int batch, bool split, int* tile, int* ksplit);
+// built-in tile code of one problem of a grouped launch
+int gemm_grouped_tile(int M, int N);
 int gemm_k_step(int tin, int K);
 // split-K epilogue: C[i*ldc + j] = (accumulate ? C : 0) + sum_{z<ks} W[z][i][j]
 // (W: ks x M x N of type tacc, T_F64 or T_F32)

@@ -1,0 +1,68 @@
+"""FP64 / FP32 GEMM tiles: fewer K steps than LDS stages, every operand layout,
+one bit pattern from every tile, and the built-in k-split."""
+import numpy as np
+import pytest
+
+import tensornetworks_amd as tn
+
+pytestmark = pytest.mark.gpu
+
+
+def _product(ctx, tin, akm, bkm, M, N, K, tile, seed=5, ksplit=1):
+    rng = np.random.default_rng(seed)
+    A, B = rng.uniform(-1.0, 1.0, (M, K)), rng.uniform(-1.0, 1.0, (K, N))
+    if tin == tn.TN_FP32:
+        A, B = A.astype(np.float32).astype(np.float64), B.astype(np.float32).astype(np.float64)
+    C = ctx.gemm_test(A if akm else np.ascontiguousarray(A.T), np.ascontiguousarray(B.T) if bkm else B, tin, 0, akm,
+                      bkm, M, N, K, 1, tile, ksplit)[0]
+    u = 2.0 ** -53 if tin == tn.TN_FP64 else 2.0 ** -24
+    # K roundings of sums bounded by |A| |B|, and the final one
+    bound = (K + 1) * u * (np.abs(A) @ np.abs(B))
+    assert np.all(np.abs(C - A @ B) <= bound + 2.0 ** -53 * K * (np.abs(A) @ np.abs(B))), (tin, akm, bkm, tile, K)
+    return C
+
+
+@pytest.mark.parametrize("tin", [tn.TN_FP64, tn.TN_FP32])
+@pytest.mark.parametrize("akm,bkm", [(True, True), (True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("K", [32, 64, 96, 160, 448])
+def test_every_tile_gives_the_same_bits(ctx, tin, akm, bkm, K):
+    M, N = 128, 256
+    ref = _product(ctx, tin, akm, bkm, M, N, K, 7)
+    deep = 32 if tin == tn.TN_FP64 else 64  # the K multiple the deep codes ask for
+    for tile in range(0, 11):
+        if tile >= 8 and K % deep:
+            with pytest.raises(tn.TnError):
+                _product(ctx, tin, akm, bkm, M, N, K, tile)
+            continue
+        assert np.array_equal(_product(ctx, tin, akm, bkm, M, N, K, tile), ref), tile
+
+
+@pytest.mark.parametrize("tin", [tn.TN_FP64, tn.TN_FP32])
+@pytest.mark.parametrize("akm,bkm", [(True, True), (True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("M,N,K", [(32, 32, 16), (64, 32, 48), (96, 160, 112), (128, 128, 16)])
+def test_odd_multiples_of_sixteen(ctx, tin, akm, bkm, M, N, K):
+    for tile in (0, 7):
+        _product(ctx, tin, akm, bkm, M, N, K, tile)
+
+
+@pytest.mark.parametrize("D1,D2,d", [(30, 30, 2), (320, 64, 2), (64, 320, 3), (288, 224, 2)])
+@pytest.mark.parametrize("prec,u", [(tn.TN_FP64, 2.0 ** -53), (tn.TN_FP32, 2.0 ** -24)])
+def test_heff_with_built_in_split(ctx, D1, D2, d, prec, u):
+    # stage 3 sums over (w, a'): split over K for the wide left environments
+    rng = np.random.default_rng(D1 + D2)
+    W = np.ascontiguousarray(rng.uniform(-1.0, 1.0, (3, 3, d, d)))
+    L, R = rng.uniform(-1.0, 1.0, (D1, 3, D1)), rng.uniform(-1.0, 1.0, (D2, 3, D2))
+    x = rng.uniform(-1.0, 1.0, (D1, d, D2))
+
+    def contract(W, L, R, x):
+        T = np.einsum("anb,cwb->anwc", x, R, optimize=True)
+        T = np.einsum("anwc,vwmn->vamc", T, W, optimize=True)
+        return np.einsum("eva,vamc->emc", L, T, optimize=True)
+
+    ctx.site_bind(W, np.ascontiguousarray(L.transpose(2, 0, 1)).ravel(),
+                  np.ascontiguousarray(R.transpose(2, 0, 1)).ravel(), d, D1, D2, prec)
+    y = ctx.heff_apply(np.ascontiguousarray(x.transpose(2, 0, 1)).ravel()).reshape(D2, D1, d).transpose(1, 2, 0)
+    ref = contract(W, L, R, x)
+    size = contract(np.abs(W), np.abs(L), np.abs(R), np.abs(x))
+    # one rounding per term of the three nested sums
+    assert np.all(np.abs(y - ref) <= (D2 + 3 * d + 3 * D1 + 8) * u * size)
