@@ -269,7 +269,7 @@ struct HeffLaunch {
     long nmax = 0;
     std::vector<GroupLaunch> g1, g3;
     const MixJob* mix = nullptr;
-    int nmix = 0, Xmax = 0, Bnmax = 0;
+    int nmix = 0, Xmax = 0, Bnmax = 0, nout = 0, nnz = 0;
 };
 
 HeffLaunch heff_batch_stage(tn_batch* b, const std::vector<Slot>& S, const std::vector<const double*>& x,
@@ -325,6 +325,10 @@ HeffLaunch heff_batch_stage(tn_batch* b, const std::vector<Slot>& S, const std::
     h.nmix = (int)mj.size();
     h.Xmax = Xmax;
     h.Bnmax = Bnmax;
+    for (const MixJob& m : mj) {
+        h.nout = std::max(h.nout, m.t.nout);
+        h.nnz = std::max(h.nnz, m.t.nnz);
+    }
     h.g3 = gemm_group_stage(b, g3s);  // the accumulate flag travels per problem
     return h;
 }
@@ -336,7 +340,7 @@ void heff_batch_launch(tn_batch* b, const HeffLaunch& h, bool conv_done = false)
     hipStream_t s = b->ctx->stream;
     if (!conv_done) TN_HIP(bconvert(h.conv, h.nconv, h.nmax, s));
     gemm_group_launch(b, h.g1);
-    TN_HIP(bwmix(T_F32, h.mix, h.nmix, h.Xmax, h.Bnmax, s));
+    TN_HIP(bwmix(T_F32, h.mix, h.nmix, h.Xmax, h.Bnmax, h.nout, h.nnz, s));
     gemm_group_launch(b, h.g3);
 }
 
@@ -1021,7 +1025,12 @@ void env_batch(tn_batch* b, const std::vector<Slot>& S, int dir, tn_sweep_stats*
     if (cj.empty()) return;
     TN_HIP(bconvert(push(b, cj), (int)cj.size(), nmax, s));
     gemm_group(b, e1s);
-    TN_HIP(bwmix(T_F32, push(b, mj), (int)mj.size(), Xmax, Bnmax, s));
+    int nout = 0, nnz = 0;
+    for (const MixJob& m : mj) {
+        nout = std::max(nout, m.t.nout);
+        nnz = std::max(nnz, m.t.nnz);
+    }
+    TN_HIP(bwmix(T_F32, push(b, mj), (int)mj.size(), Xmax, Bnmax, nout, nnz, s));
     std::vector<GemmDesc> e3a, e3b;
     for (auto& g : e3s) (g.a_kmajor ? e3b : e3a).push_back(g);
     gemm_group(b, e3a);

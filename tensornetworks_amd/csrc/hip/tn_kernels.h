@@ -365,7 +365,8 @@ struct DiagJob {  // G[i][i] += v, i0 <= i < i1
     double v;
 };
 hipError_t badd_diag(const DiagJob* jobs, int n, int lenmax, hipStream_t s);
-hipError_t bwmix(int tout, const MixJob* jobs, int n, int Xmax, int Bnmax, hipStream_t s);
+// nout_max, nnz_max: the largest table of the jobs
+hipError_t bwmix(int tout, const MixJob* jobs, int n, int Xmax, int Bnmax, int nout_max, int nnz_max, hipStream_t s);
 hipError_t add_diag(double* G, long ldg, int i0, int i1, double v, hipStream_t s);
 hipError_t eye_deviation(const double* G, long ldg, int n, double* out, double* part, hipStream_t s);
 

@@ -9,45 +9,97 @@
 namespace tn {
 
 // ---------------------------------------------------------------------------
-// MPO mixing
-template <typename TI, typename TO>
-__global__ void __launch_bounds__(256) wmix_k(const TI* __restrict__ in, long isx,
-                                              TO* __restrict__ out, long osx, int Bn, int nout,
-                                              const int* __restrict__ optr,
-                                              const long* __restrict__ ooff,
-                                              const long* __restrict__ eoff,
-                                              const double* __restrict__ eval,
-                                              const float* __restrict__ evalf)
+// MPO mixing.  Bound by HBM for large bonds (D = 1024 FP64: 250 MB in 51 us) and
+// by latency below: every entry is a chain offset / value / selector, then the
+// data.  The table is staged in LDS first (one latency instead of one per
+// entry), and the outputs are spread over the grid's z until about three
+// workgroups per CU exist.  Before (one workgroup walking all outputs with the
+// table in global memory) and after: transposed FP64 form, D = 8: 11.5 and
+// 4.1 us; 320 x 224, d = 2: 15.5 and 7.5 us; D = 256, d = 3: 21.7 and 6.9 us;
+// FP32 512 x 448, d = 3: 16.5 and 10.7 us; plain FP64 form, D = 256, d = 2: 6.9
+// and 6.4 us.  Sums keep the table's order.
+#define MIX_MAXO 64
+#define MIX_MAXE 512
+template <typename V> struct MixLds {
+    int optr[MIX_MAXO + 1], osel[MIX_MAXO], esel[MIX_MAXE];
+    long ooff[MIX_MAXO], eoff[MIX_MAXE];
+    V eval[MIX_MAXE];
+};
+// STG: the table's copy in LDS (nout <= MIX_MAXO, nnz <= MIX_MAXE), else global
+template <typename V, bool STG> struct MixView {
+    const int *optr, *osel, *esel;
+    const long *ooff, *eoff;
+    const V* eval;
+};
+template <typename V>
+__device__ __forceinline__ const V* mix_values(const MixTable& t)
 {
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= Bn) return;
-    const long x = blockIdx.y;
+    if constexpr (std::is_same<V, double>::value) return t.eval;
+    else return t.evalf;
+}
+template <typename V, bool STG>
+__device__ __forceinline__ MixView<V, STG> mix_view(const MixTable& t, MixLds<V>* l)
+{
+    if constexpr (!STG) {
+        return MixView<V, STG>{t.optr, t.osel, t.esel, t.ooff, t.eoff, mix_values<V>(t)};
+    } else {
+        const V* v = mix_values<V>(t);
+        const bool idt = t.esel != nullptr;
+        for (int i = threadIdx.x; i <= t.nout; i += 256) l->optr[i] = t.optr[i];
+        for (int i = threadIdx.x; i < t.nout; i += 256) {
+            l->ooff[i] = t.ooff[i];
+            l->osel[i] = idt ? t.osel[i] : 0;
+        }
+        for (int i = threadIdx.x; i < t.nnz; i += 256) {
+            l->eoff[i] = t.eoff[i];
+            l->eval[i] = v[i];
+            l->esel[i] = idt ? t.esel[i] : 0;
+        }
+        __syncthreads();
+        return MixView<V, STG>{l->optr, l->osel, l->esel, l->ooff, l->eoff, l->eval};
+    }
+}
+// grid z for nout outputs over xy workgroups
+static int mix_groups(long xy, int nout)
+{
+    const long z = (768 + xy - 1) / xy;
+    return (int)(z < nout ? z : nout);
+}
+
+// 64 b times 4 x per workgroup
+template <typename TI, typename TO, bool STG>
+__global__ void __launch_bounds__(256) wmix_k(const TI* __restrict__ in, long isx, TO* __restrict__ out, long osx,
+                                              int X, int Bn, MixTable t)
+{
+    typedef typename std::conditional<std::is_same<TI, double>::value, double, float>::type acc_t;
+    __shared__ typename std::conditional<STG, MixLds<acc_t>, int>::type lds;
+    const MixView<acc_t, STG> m = mix_view<acc_t, STG>(t, (MixLds<acc_t>*)&lds);
+    const int b = blockIdx.x * 64 + (threadIdx.x & 63);
+    const long x = (long)blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (b >= Bn || x >= X) return;
     const TI* ip = in + x * isx + b;
     TO* op = out + x * osx + b;
-    for (int o = 0; o < nout; o++) {
-        const int e0 = optr[o], e1 = optr[o + 1];
-        if constexpr (std::is_same<TI, double>::value) {
-            double acc = 0.0;
-            for (int e = e0; e < e1; e++) acc += eval[e] * to_d(ip[eoff[e]]);
-            op[ooff[o]] = cvt_from_d<TO>(acc);
-        } else {
-            float acc = 0.0f;
-            for (int e = e0; e < e1; e++) acc += evalf[e] * to_f(ip[eoff[e]]);
-            op[ooff[o]] = cvt_from_f<TO>(acc);
-        }
+    for (int o = blockIdx.z; o < t.nout; o += gridDim.z) {
+        const int e0 = m.optr[o], e1 = m.optr[o + 1];
+        acc_t acc = 0;
+#pragma unroll 4
+        for (int e = e0; e < e1; e++) acc += m.eval[e] * to_acc<acc_t>(ip[m.eoff[e]]);
+        if constexpr (std::is_same<TI, double>::value) op[m.ooff[o]] = cvt_from_d<TO>(acc);
+        else op[m.ooff[o]] = cvt_from_f<TO>(acc);
     }
 }
 
 hipError_t wmix(int tin, int tout, const void* in, long isx, void* out, long osx, int X, int Bn,
                 const MixTable& t, hipStream_t s)
 {
-    dim3 grid((Bn + 255) / 256, X);
-#define WM_CASE(TIc, TOc, TIt, TOt)                                                         \
-    if (tin == TIc && tout == TOc) {                                                        \
-        wmix_k<TIt, TOt><<<grid, 256, 0, s>>>((const TIt*)in, isx, (TOt*)out, osx, Bn,      \
-                                               t.nout, t.optr, t.ooff, t.eoff, t.eval,      \
-                                               t.evalf);                                    \
-        return hipGetLastError();                                                           \
+    dim3 grid((Bn + 63) / 64, (X + 3) / 4);
+    grid.z = mix_groups((long)grid.x * grid.y, t.nout);
+    const bool stg = t.nout <= MIX_MAXO && t.nnz <= MIX_MAXE;
+#define WM_CASE(TIc, TOc, TIt, TOt)                                                                             \
+    if (tin == TIc && tout == TOc) {                                                                            \
+        if (stg) wmix_k<TIt, TOt, true><<<grid, 256, 0, s>>>((const TIt*)in, isx, (TOt*)out, osx, X, Bn, t);    \
+        else wmix_k<TIt, TOt, false><<<grid, 256, 0, s>>>((const TIt*)in, isx, (TOt*)out, osx, X, Bn, t);       \
+        return hipGetLastError();                                                                               \
     }
     WM_CASE(T_F64, T_F64, double, double)
     WM_CASE(T_F32, T_F32, float, float)
@@ -57,17 +109,15 @@ hipError_t wmix(int tin, int tout, const void* in, long isx, void* out, long osx
     return hipErrorInvalidValue;
 }
 
-template <typename TI, typename TX, typename TO, bool X3 = false>
+template <typename TI, typename TX, typename TO, bool X3, bool STG>
 __global__ void __launch_bounds__(256) wmix_idt_k(const TI* __restrict__ in, long isx, const TX* __restrict__ in2,
                                                   long isx2, TO* __restrict__ out, long ldo, long ops,
-                                                  double* __restrict__ out2, long osx2, int Bn, int nout,
-                                                  const int* __restrict__ optr, const long* __restrict__ ooff,
-                                                  const long* __restrict__ eoff, const int* __restrict__ esel,
-                                                  const int* __restrict__ osel, const double* __restrict__ eval,
-                                                  const float* __restrict__ evalf)
+                                                  double* __restrict__ out2, long osx2, int Bn, MixTable t)
 {
     typedef typename std::conditional<std::is_same<TI, double>::value, double, float>::type acc_t;
     __shared__ acc_t tile[64][33];
+    __shared__ typename std::conditional<STG, MixLds<acc_t>, int>::type lds;
+    const MixView<acc_t, STG> m = mix_view<acc_t, STG>(t, (MixLds<acc_t>*)&lds);
     const int tb = threadIdx.x & 63, tr = threadIdx.x >> 6;  // b within the tile, row group of 8
     const int b = blockIdx.x * 64 + tb;
     const long x0 = (long)blockIdx.y * 32 + tr * 8;
@@ -75,16 +125,17 @@ __global__ void __launch_bounds__(256) wmix_idt_k(const TI* __restrict__ in, lon
     // writer role: row wb of the tile (b), columns wc..wc+7 (x)
     const int wb = threadIdx.x >> 2, wc = (threadIdx.x & 3) * 8;
     const bool wok = blockIdx.x * 64 + wb < Bn;
-    for (int o = 0; o < nout; o++) {
-        const int e0 = optr[o], e1 = optr[o + 1];
+    for (int o = blockIdx.z; o < t.nout; o += gridDim.z) {
+        const int e0 = m.optr[o], e1 = m.optr[o + 1];
         acc_t acc[8];
 #pragma unroll
         for (int r = 0; r < 8; r++) acc[r] = 0;
         if (bok) {
+#pragma unroll 2
             for (int e = e0; e < e1; e++) {
-                const acc_t v = std::is_same<TI, double>::value ? (acc_t)eval[e] : (acc_t)evalf[e];
-                const long off = eoff[e] + b;
-                if (esel[e]) {
+                const acc_t v = m.eval[e];
+                const long off = m.eoff[e] + b;
+                if (m.esel[e]) {
 #pragma unroll
                     for (int r = 0; r < 8; r++) acc[r] += v * to_acc<acc_t>(in2[(x0 + r) * isx2 + off]);
                 } else {
@@ -93,10 +144,10 @@ __global__ void __launch_bounds__(256) wmix_idt_k(const TI* __restrict__ in, lon
                 }
             }
         }
-        if (osel[o]) {  // identity channel of L: straight into y[x][m][b]
+        if (m.osel[o]) {  // identity channel of L: straight into y[x][m][b]
             if (bok) {
 #pragma unroll
-                for (int r = 0; r < 8; r++) out2[(x0 + r) * osx2 + ooff[o] + b] = (double)acc[r];
+                for (int r = 0; r < 8; r++) out2[(x0 + r) * osx2 + m.ooff[o] + b] = (double)acc[r];
             }
             continue;
         }
@@ -105,7 +156,7 @@ __global__ void __launch_bounds__(256) wmix_idt_k(const TI* __restrict__ in, lon
         for (int r = 0; r < 8; r++) tile[tb][tr * 8 + r] = acc[r];
         __syncthreads();
         if (wok) {
-            TO* dst = out + ooff[o] + (long)(blockIdx.x * 64 + wb) * ldo + (long)blockIdx.y * 32 + wc;
+            TO* dst = out + m.ooff[o] + (long)(blockIdx.x * 64 + wb) * ldo + (long)blockIdx.y * 32 + wc;
             if constexpr (X3) {
                 // three bfloat16 planes, one 16-byte store per plane (8 values;
                 // every offset here is a multiple of 8 elements)
@@ -143,23 +194,23 @@ hipError_t wmix_idt(int tin, int tx, int tout, const void* in, long isx, const v
 {
     if (!t.esel || !t.osel || X % 32) return hipErrorInvalidValue;
     dim3 grid((Bn + 63) / 64, X / 32);
-    if (tout == T_BF16X3) {
-        if (tin != T_F32 || tx != T_F64 || ops <= 0 || ops % 8 || ldo % 8) return hipErrorInvalidValue;
-        wmix_idt_k<float, double, bf16, true><<<grid, 256, 0, s>>>((const float*)in, isx, (const double*)in2, isx2,
-                                                                 (bf16*)out, ldo, ops, out2, osx2, Bn, t.nout, t.optr,
-                                                                 t.ooff, t.eoff, t.esel, t.osel, t.eval, t.evalf);
-        return hipGetLastError();
+    grid.z = mix_groups((long)grid.x * grid.y, t.nout);
+    const bool stg = t.nout <= MIX_MAXO && t.nnz <= MIX_MAXE;
+    if (tout == T_BF16X3 && (tin != T_F32 || tx != T_F64 || ops <= 0 || ops % 8 || ldo % 8)) return hipErrorInvalidValue;
+#define WT_CASE(TIc, TXc, TOc, TIt, TXt, TOt, X3)                                                               \
+    if (tin == TIc && tx == TXc && tout == TOc) {                                                               \
+        if (stg)                                                                                                \
+            wmix_idt_k<TIt, TXt, TOt, X3, true><<<grid, 256, 0, s>>>(                                           \
+                (const TIt*)in, isx, (const TXt*)in2, isx2, (TOt*)out, ldo, ops, out2, osx2, Bn, t);            \
+        else                                                                                                    \
+            wmix_idt_k<TIt, TXt, TOt, X3, false><<<grid, 256, 0, s>>>(                                          \
+                (const TIt*)in, isx, (const TXt*)in2, isx2, (TOt*)out, ldo, ops, out2, osx2, Bn, t);            \
+        return hipGetLastError();                                                                               \
     }
-#define WT_CASE(TIc, TXc, TOc, TIt, TXt, TOt)                                                              \
-    if (tin == TIc && tx == TXc && tout == TOc) {                                                          \
-        wmix_idt_k<TIt, TXt, TOt><<<grid, 256, 0, s>>>((const TIt*)in, isx, (const TXt*)in2, isx2,         \
-                                                       (TOt*)out, ldo, 0, out2, osx2, Bn, t.nout, t.optr,  \
-                                                       t.ooff, t.eoff, t.esel, t.osel, t.eval, t.evalf);   \
-        return hipGetLastError();                                                                          \
-    }
-    WT_CASE(T_F64, T_F64, T_F64, double, double, double)
-    WT_CASE(T_F32, T_F32, T_F32, float, float, float)
-    WT_CASE(T_F32, T_BF16, T_BF16, float, bf16, bf16)
+    WT_CASE(T_F32, T_F64, T_BF16X3, float, double, bf16, true)
+    WT_CASE(T_F64, T_F64, T_F64, double, double, double, false)
+    WT_CASE(T_F32, T_F32, T_F32, float, float, float, false)
+    WT_CASE(T_F32, T_BF16, T_BF16, float, bf16, bf16, false)
 #undef WT_CASE
     return hipErrorInvalidValue;
 }
@@ -310,46 +361,47 @@ hipError_t fill_value(double* p, double v, long n, hipStream_t s)
     return hipGetLastError();
 }
 
-// site tensor layouts: reference psi[m + d*(a + D1*b)] <-> internal [D1p][d][D2p]
-// (zero padding written on the internal side; grid-stride over the written side)
-__global__ void psi_r2i_k(const double* __restrict__ ref, double* __restrict__ out, int d, int D1, int D2, int D1p,
-                          int D2p)
+// out[c*ldo + r] = (r < R && c < C) ? in[r*ldi + c] : 0, for r < Ro, c < Co,
+// through a 32 x 32 LDS tile so that reads and writes are both coalesced
+// (D = 1024, d = 3, 50 MB moved: 23 and 17 us, read or written with a stride,
+// against 10.6 us tiled)
+__global__ void __launch_bounds__(256) transpose_k(const double* __restrict__ in, long ldi, int R, int C,
+                                                   double* __restrict__ out, long ldo, int Ro, int Co)
 {
-    const long n = (long)D1p * d * D2p;
-    for (long t = blockIdx.x * 256L + threadIdx.x; t < n; t += (long)gridDim.x * 256) {
-        const int b = (int)(t % D2p);
-        const long r = t / D2p;
-        const int m = (int)(r % d), a = (int)(r / d);
-        out[t] = (a < D1 && b < D2) ? ref[m + (long)d * (a + (long)D1 * b)] : 0.0;
+    __shared__ double tile[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
+#pragma unroll
+    for (int i = 0; i < 32; i += 8) {
+        const int r = r0 + ty + i, c = c0 + tx;
+        tile[ty + i][tx] = (r < R && c < C) ? in[(long)r * ldi + c] : 0.0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 32; i += 8) {
+        const int c = c0 + ty + i, r = r0 + tx;
+        if (r < Ro && c < Co) out[(long)c * ldo + r] = tile[tx][ty + i];
     }
 }
-__global__ void psi_i2r_k(const double* __restrict__ in, double* __restrict__ ref, int d, int D1, int D2, int D2p)
+static hipError_t transpose(const double* in, long ldi, int R, int C, double* out, long ldo, int Ro, int Co,
+                            hipStream_t s)
 {
-    const long n = (long)d * D1 * D2;
-    for (long t = blockIdx.x * 256L + threadIdx.x; t < n; t += (long)gridDim.x * 256) {
-        const int m = (int)(t % d);
-        const long r = t / d;
-        const int a = (int)(r % D1), b = (int)(r / D1);
-        ref[t] = in[((long)a * d + m) * D2p + b];
-    }
+    transpose_k<<<dim3((Co + 31) / 32, (Ro + 31) / 32), 256, 0, s>>>(in, ldi, R, C, out, ldo, Ro, Co);
+    return hipGetLastError();
 }
+
+// site tensor layouts: reference psi[m + d*(a + D1*b)] is the matrix (b, (a, m)),
+// internal [D1p][d][D2p] the matrix ((a, m), b): transposes of each other, with
+// zero padding on the internal side
 hipError_t psi_ref_to_int(const double* ref, double* out, int d, int D1, int D2, int D1p, int D2p, hipStream_t s)
 {
     if (d <= 0 || D1 <= 0 || D2 <= 0 || D1p < D1 || D2p < D2) return hipErrorInvalidValue;
-    const long n = (long)D1p * d * D2p;
-    long blocks = (n + 255) / 256;
-    if (blocks > 16384) blocks = 16384;
-    psi_r2i_k<<<blocks, 256, 0, s>>>(ref, out, d, D1, D2, D1p, D2p);
-    return hipGetLastError();
+    return transpose(ref, (long)d * D1, D2, d * D1, out, D2p, D2p, d * D1p, s);
 }
 hipError_t psi_int_to_ref(const double* in, double* ref, int d, int D1, int D2, int D2p, hipStream_t s)
 {
     if (d <= 0 || D1 <= 0 || D2 <= 0 || D2p < D2) return hipErrorInvalidValue;
-    const long n = (long)d * D1 * D2;
-    long blocks = (n + 255) / 256;
-    if (blocks > 16384) blocks = 16384;
-    psi_i2r_k<<<blocks, 256, 0, s>>>(in, ref, d, D1, D2, D2p);
-    return hipGetLastError();
+    return transpose(in, D2p, d * D1, D2, ref, (long)d * D1, d * D1, D2, s);
 }
 
 __global__ void copy3_k(const double* __restrict__ in, long si, long sj, long sk,
@@ -381,6 +433,8 @@ hipError_t copy2(const double* in, long si0, long si1, int r, int c, double* out
                  long so1, int ro, int co, hipStream_t s)
 {
     if (ro <= 0 || co <= 0) return hipSuccess;
+    if (si1 == 1 && so0 == 1 && so1 != 1) return transpose(in, si0, r, c, out, so1, ro, co, s);
+    if (si0 == 1 && so1 == 1 && si1 != 1) return transpose(in, si1, c, r, out, so0, co, ro, s);
     dim3 grid((co + 255) / 256, ro);
     copy2_k<<<grid, 256, 0, s>>>(in, si0, si1, r, c, out, so0, so1, co);
     return hipGetLastError();
@@ -2040,71 +2094,44 @@ hipError_t bconvert(const ConvJob* jobs, int n, long nmax, hipStream_t s)
     return hipGetLastError();
 }
 
-// MPO mixing (FP32 in, TO out) for many problems: grid (Bn blocks, X, problem).
-// The workgroup's mixing table (one problem's) is staged in LDS first when it
-// fits: read from global memory, every entry would be a chain of dependent
-// loads (offset, value, selector, then the data) per output.
-#define BW_MAXO 64
-#define BW_MAXE 512
-template <typename TO>
-__global__ void __launch_bounds__(256) bwmix_k(const MixJob* __restrict__ jobs)
+// MPO mixing (FP32 in, TO out) for many problems: the layout of wmix_k, the
+// problem in grid z
+template <typename TO, bool STG>
+__global__ void __launch_bounds__(256) bwmix_k(const MixJob* __restrict__ jobs, int groups)
 {
-    __shared__ int s_optr[BW_MAXO + 1];
-    __shared__ long s_ooff[BW_MAXO];
-    __shared__ int s_osel[BW_MAXO];
-    __shared__ long s_eoff[BW_MAXE];
-    __shared__ float s_eval[BW_MAXE];
-    __shared__ int s_esel[BW_MAXE];
-    const MixJob& j = jobs[blockIdx.z];
-    const long x = blockIdx.y;
-    if (x >= j.X) return;  // the whole workgroup
-    const MixTable& t = j.t;
-    const int nout = t.nout, nnz = t.nnz;
+    __shared__ typename std::conditional<STG, MixLds<float>, int>::type lds;
+    const MixJob& j = jobs[blockIdx.z / groups];
+    if (blockIdx.x * 64 >= j.Bn || (long)blockIdx.y * 4 >= j.X) return;  // the whole workgroup
+    const MixTable t = j.t;
     const bool idt = t.esel != nullptr;
-    const bool staged = nout <= BW_MAXO && nnz <= BW_MAXE;
-    if (staged) {
-        for (int i = threadIdx.x; i <= nout; i += 256) s_optr[i] = t.optr[i];
-        for (int i = threadIdx.x; i < nout; i += 256) {
-            s_ooff[i] = t.ooff[i];
-            s_osel[i] = idt ? t.osel[i] : 0;
-        }
-        for (int i = threadIdx.x; i < nnz; i += 256) {
-            s_eoff[i] = t.eoff[i];
-            s_eval[i] = t.evalf[i];
-            s_esel[i] = idt ? t.esel[i] : 0;
-        }
-        __syncthreads();
-    }
-    const int b = blockIdx.x * 256 + threadIdx.x;
-    if (b >= j.Bn) return;
+    const MixView<float, STG> m = mix_view<float, STG>(t, (MixLds<float>*)&lds);
+    const int b = blockIdx.x * 64 + (threadIdx.x & 63);
+    const long x = (long)blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (b >= j.Bn || x >= j.X) return;
     const float* ip = (const float*)j.in + x * j.isx + b;
     TO* op = (TO*)j.out + x * j.osx + b;
     const float* ip2 = idt ? j.in2 + x * j.isx2 + b : nullptr;
-    if (staged) {
-        for (int o = 0; o < nout; o++) {
-            const int e0 = s_optr[o], e1 = s_optr[o + 1];
-            float acc = 0.0f;
-#pragma unroll 4
-            for (int e = e0; e < e1; e++) acc += s_eval[e] * (s_esel[e] ? ip2[s_eoff[e]] : ip[s_eoff[e]]);
-            if (s_osel[o]) j.out2[x * j.osx2 + s_ooff[o] + b] = (double)acc;
-            else op[s_ooff[o]] = cvt_from_f<TO>(acc);
-        }
-        return;
-    }
-    for (int o = 0; o < nout; o++) {
-        const int e0 = t.optr[o], e1 = t.optr[o + 1];
+    for (int o = blockIdx.z % groups; o < t.nout; o += groups) {
+        const int e0 = m.optr[o], e1 = m.optr[o + 1];
         float acc = 0.0f;
-        for (int e = e0; e < e1; e++) acc += t.evalf[e] * (idt && t.esel[e] ? ip2[t.eoff[e]] : ip[t.eoff[e]]);
-        if (idt && t.osel[o]) j.out2[x * j.osx2 + t.ooff[o] + b] = (double)acc;
-        else op[t.ooff[o]] = cvt_from_f<TO>(acc);
+#pragma unroll 4
+        for (int e = e0; e < e1; e++)
+            acc += m.eval[e] * (idt && m.esel[e] ? ip2[m.eoff[e]] : ip[m.eoff[e]]);
+        if (idt && m.osel[o]) j.out2[x * j.osx2 + m.ooff[o] + b] = (double)acc;
+        else op[m.ooff[o]] = cvt_from_f<TO>(acc);
     }
 }
-hipError_t bwmix(int tout, const MixJob* jobs, int n, int Xmax, int Bnmax, hipStream_t s)
+hipError_t bwmix(int tout, const MixJob* jobs, int n, int Xmax, int Bnmax, int nout_max, int nnz_max, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    dim3 grid((Bnmax + 255) / 256, Xmax, n);
-    if (tout == T_F32) bwmix_k<float><<<grid, 256, 0, s>>>(jobs);
-    else if (tout == T_F64) bwmix_k<double><<<grid, 256, 0, s>>>(jobs);
+    dim3 grid((Bnmax + 63) / 64, (Xmax + 3) / 4);
+    const int groups = mix_groups((long)grid.x * grid.y * n, nout_max);
+    grid.z = n * groups;
+    const bool stg = nout_max <= MIX_MAXO && nnz_max <= MIX_MAXE;
+    if (tout == T_F32 && stg) bwmix_k<float, true><<<grid, 256, 0, s>>>(jobs, groups);
+    else if (tout == T_F32) bwmix_k<float, false><<<grid, 256, 0, s>>>(jobs, groups);
+    else if (tout == T_F64 && stg) bwmix_k<double, true><<<grid, 256, 0, s>>>(jobs, groups);
+    else if (tout == T_F64) bwmix_k<double, false><<<grid, 256, 0, s>>>(jobs, groups);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
