@@ -1129,13 +1129,11 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
     int* flag = c->svd_flag.as<int>();
     const double tol = std::max(1e-15, 4.4e-16 * std::sqrt((double)pj));
     int hflag = 1;
-    // one sweep of rotations on each pair's Gram matrix per visit: the pairs
+    // (each visit gives a pair's Gram matrix one sweep of rotations: the pairs
     // come back every outer sweep, and a round has only nb/2 pairs, so its
-    // latency (mostly the inner rounds) sets the cost.  Measured on the
-    // 512 x 512 two-site splits at D=256: one inner sweep halves the SVD time
-    // against diagonalising each pair (up to 20 inner sweeps), with more
-    // outer sweeps and the same singular values.
-    const int inner = 1;
+    // latency sets the cost.  On the 512 x 512 two-site splits at D=256 that
+    // halves the SVD time against diagonalising each pair, with more outer
+    // sweeps and the same singular values)
     // workgroups per pair, each rotating its own rows (about 256 in all, at
     // least 32 rows each); the iterate alternates between X and X2
     const int nchunk = std::max(1, std::min({16, 256 / std::max(1, nb / 2), std::max(1, pj / 32)}));
@@ -1146,7 +1144,7 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
         TN_HIP(set_int(flag, 0, s));
         for (int rd = 0; rd < nb - 1; rd++) {
             TN_HIP(jacobi_step(Xa, Xb, ldx, pj, V, qp, qp, c->svd_pairs.as<int>() + (size_t)rd * nb, nb / 2,
-                               nchunk, tol, flag, s, inner));
+                               nchunk, tol, flag, s));
             std::swap(Xa, Xb);
         }
         TN_HIP(hipMemcpyAsync(&hflag, flag, sizeof(int), hipMemcpyDeviceToHost, s));

@@ -971,60 +971,93 @@ hipError_t dsqrt_scalar(const double* src, double* dst, hipStream_t s)
 // spread over up to 16 times as many CUs; reading Xs and writing Xd keeps a
 // workgroup from seeing rows another has already rotated.  A pair that is
 // already orthogonal copies its rows to Xd.
+//
+// Bound by the latency of 31 dependent rotation rounds (three divisions and two
+// square roots each).  A round has one barrier: every 16 lanes form the round's
+// rotations themselves from the previous round's G (two buffers) instead of
+// waiting for 16 threads to publish them.  Measured per launch, that form (with
+// one thread per row in step 3) and this one: 45 and 31 us at p = q = 32, 50 and
+// 34 us at 192, 53 and 41 us at 512.
 #define JB 16
 #define JW 32
 #define JR 128  // rows per Gram chunk
 
+// the rotation that annihilates apq of [app apq; apq aqq] (no branch: the
+// discarded values of a skipped rotation may be infinite)
+__device__ __forceinline__ void jacobi_rot(double app, double aqq, double apq, double& c, double& s)
+{
+    const bool rot = fabs(apq) > 1e-300 && fabs(apq) > 1e-16 * sqrt(fabs(app * aqq));
+    const double theta = (aqq - app) / (2.0 * apq);
+    const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
+    const double cr = 1.0 / sqrt(t * t + 1.0);
+    c = rot ? cr : 1.0;
+    s = rot ? t * cr : 0.0;
+}
+
 __global__ void __launch_bounds__(256) jacobi_k(const double* __restrict__ Xs, double* __restrict__ Xd, long ldx,
                                                 int p, double* __restrict__ V, long ldv, int qv,
-                                                const int* __restrict__ pairs, double tol,
-                                                int* __restrict__ flag, int inner)
+                                                const int* __restrict__ pairs, double tol, int* __restrict__ flag)
 {
-    // even row strides: column pairs are 16-byte aligned for double2 reads
-    __shared__ double G[JW][JW + 1];
-    __shared__ __align__(16) double J[JW][JW + 2];
-    __shared__ __align__(16) double tile[JR][JW + 2];
-    __shared__ double rc[JW / 2], rs[JW / 2];
-    __shared__ int rp[JW / 2], rq[JW / 2];
-    __shared__ int any_rot;
+    __shared__ double G[2][JW][JW + 1];
+    __shared__ __align__(16) double J[JW][JW + 2];  // even stride: column pairs are 16-byte aligned
+    __shared__ double tile[JW][JR + 1];
     __shared__ int sh_off;
     const int tid = threadIdx.x;
     const int pb = pairs[2 * blockIdx.x], qb = pairs[2 * blockIdx.x + 1];
     auto colidx = [&](int j) { return j < JB ? pb * JB + j : qb * JB + (j - JB); };
+    // this workgroup's rows of the iterate and of V, 32 at a time: thread = row
+    // ar of the 32 and columns 4 ac .. 4 ac + 3 of the product
+    const int nch = gridDim.y, ch = blockIdx.y;
+    const int xrows = (p + nch - 1) / nch, vrows = (qv + nch - 1) / nch;
+    const int xr0 = ch * xrows, xr1 = min(p, xr0 + xrows);
+    const int vr0 = ch * vrows, vr1 = min(qv, vr0 + vrows);
+    const int ar = tid & 31, ac = tid >> 5;
 
-    // 1. Gram matrix over row chunks of JR rows staged in LDS (all loads of a
-    // chunk in flight together: few load-then-barrier rounds per launch), on
-    // the FP64 matrix cores: wave w forms the 16 x 16 block (w >> 1, w & 1)
-    // of G, one v_mfma_f64_16x16x4 per 4 rows (lane l reads row l/16 of the
-    // step and column l%16 of each of its two column blocks).
+    // 1. Gram matrix over row chunks of JR rows staged in LDS, on the FP64
+    // matrix cores: wave w forms the 16 x 16 block (w >> 1, w & 1) of G, one
+    // v_mfma_f64_16x16x4 per 4 rows (lane l reads row l/16 of the step and
+    // column l%16 of each of its two column blocks).
     const int lane = tid & 63, wv = tid >> 6;
     const int wi = wv >> 1, wj = wv & 1;
     v4d gacc = {0.0, 0.0, 0.0, 0.0};
-    for (int r0 = 0; r0 < p; r0 += JR) {
-        double ld[JR * JW / 256];
+    double ld[JR * JW / 256];
+    auto load_chunk = [&](int r0) {  // rows past the last one read as zero
 #pragma unroll
         for (int u = 0; u < JR * JW / 256; u++) {
             const int idx = tid + 256 * u;
-            const int row = idx % JR, c = idx / JR;
-            const int gr = r0 + row;
-            ld[u] = (gr < p) ? Xs[(long)colidx(c) * ldx + gr] : 0.0;
+            const int gr = r0 + idx % JR;
+            const double w = Xs[(long)colidx(idx / JR) * ldx + min(gr, p - 1)];
+            ld[u] = gr < p ? w : 0.0;
         }
+    };
+    load_chunk(0);
+    for (int r0 = 0; r0 < p; r0 += JR) {
 #pragma unroll
         for (int u = 0; u < JR * JW / 256; u++) {
             const int idx = tid + 256 * u;
-            tile[idx % JR][idx / JR] = ld[u];
+            tile[idx / JR][idx % JR] = ld[u];
         }
         __syncthreads();
+        if (r0 + JR < p) load_chunk(r0 + JR);
+        const int kn = min(JR, (p - r0 + 3) & ~3);
 #pragma unroll 8
-        for (int k0 = 0; k0 < JR; k0 += 4) {
-            const double a = tile[k0 + (lane >> 4)][16 * wi + (lane & 15)];
-            const double b = tile[k0 + (lane >> 4)][16 * wj + (lane & 15)];
+        for (int k0 = 0; k0 < kn; k0 += 4) {
+            const double a = tile[16 * wi + (lane & 15)][k0 + (lane >> 4)];
+            const double b = tile[16 * wj + (lane & 15)][k0 + (lane >> 4)];
             gacc = mma(a, b, gacc);
         }
         __syncthreads();
     }
+    // the first 32 rows of both products, in flight during the rotations (a row
+    // that does not exist repeats the last one and is not stored)
+    double x[JW], v[JW];
 #pragma unroll
-    for (int r = 0; r < 4; r++) G[16 * wi + (lane >> 4) + 4 * r][16 * wj + (lane & 15)] = gacc[r];
+    for (int c = 0; c < JW; c++) {
+        x[c] = Xs[(long)colidx(c) * ldx + min(xr0 + ar, p - 1)];
+        v[c] = V[(long)colidx(c) * ldv + min(vr0 + ar, qv - 1)];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) G[0][16 * wi + (lane >> 4) + 4 * r][16 * wj + (lane & 15)] = gacc[r];
 #pragma unroll
     for (int u = 0; u < 4; u++) {
         const int e = tid + 256 * u;
@@ -1038,16 +1071,11 @@ __global__ void __launch_bounds__(256) jacobi_k(const double* __restrict__ Xs, d
         const int e = tid + 256 * u;
         const int gi = e >> 5, gj = e & 31;
         if (gi < gj) {
-            const double dd = G[gi][gi] * G[gj][gj];
-            if (dd > 1e-300 && fabs(G[gi][gj]) > tol * sqrt(dd)) sh_off = 1;
+            const double dd = G[0][gi][gi] * G[0][gj][gj];
+            if (dd > 1e-300 && fabs(G[0][gi][gj]) > tol * sqrt(dd)) sh_off = 1;
         }
     }
     __syncthreads();
-    // this workgroup's rows of the iterate and of V
-    const int nch = gridDim.y, ch = blockIdx.y;
-    const int xrows = (p + nch - 1) / nch, vrows = (qv + nch - 1) / nch;
-    const int xr0 = ch * xrows, xr1 = min(p, xr0 + xrows);
-    const int vr0 = ch * vrows, vr1 = min(qv, vr0 + vrows);
     if (sh_off == 0) {  // already orthogonal: nothing to rotate
         for (int e = tid; e < JW * (xr1 > xr0 ? xr1 - xr0 : 0); e += 256) {
             const long off = (long)colidx(e / (xr1 - xr0)) * ldx + xr0 + e % (xr1 - xr0);
@@ -1057,104 +1085,91 @@ __global__ void __launch_bounds__(256) jacobi_k(const double* __restrict__ Xs, d
     }
     if (tid == 0) flag[0] = 1;
 
-    // 2. cyclic parallel Jacobi on G (tournament ordering, 31 rounds per sweep)
-    for (int sweep = 0; sweep < inner; sweep++) {
-        if (tid == 0) any_rot = 0;
-        __syncthreads();
-        for (int round = 0; round < JW - 1; round++) {
-            if (tid < JW / 2) {
-                auto elem = [&](int kpos) { return kpos == 0 ? 0 : ((kpos - 1 + round) % (JW - 1)) + 1; };
-                int a = elem(tid), b = elem(JW - 1 - tid);
-                int P = a < b ? a : b, Q = a < b ? b : a;
-                double app = G[P][P], aqq = G[Q][Q], apq = G[P][Q];
-                double c = 1.0, s = 0.0;
-                if (fabs(apq) > 1e-300 && fabs(apq) > 1e-16 * sqrt(fabs(app * aqq))) {
-                    double theta = (aqq - app) / (2.0 * apq);
-                    double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-                    c = 1.0 / sqrt(t * t + 1.0);
-                    s = t * c;
-                    any_rot = 1;
-                }
-                rc[tid] = c;
-                rs[tid] = s;
-                rp[tid] = P;
-                rq[tid] = Q;
-            }
-            __syncthreads();
-            // G <- R^T G R in one phase: the round's pairs are disjoint, so G
-            // splits into 16 x 16 independent 2 x 2 blocks (rows P1, Q1 of
-            // pair bi, columns P2, Q2 of pair bj), one per thread
-            {
-                const int bi = tid >> 4, bj = tid & 15;
-                const int P1 = rp[bi], Q1 = rq[bi], P2 = rp[bj], Q2 = rq[bj];
-                const double c1 = rc[bi], s1 = rs[bi], c2 = rc[bj], s2 = rs[bj];
-                const double g00 = G[P1][P2], g01 = G[P1][Q2], g10 = G[Q1][P2], g11 = G[Q1][Q2];
-                const double h00 = c1 * g00 - s1 * g10, h01 = c1 * g01 - s1 * g11;
-                const double h10 = s1 * g00 + c1 * g10, h11 = s1 * g01 + c1 * g11;
-                G[P1][P2] = c2 * h00 - s2 * h01;
-                G[P1][Q2] = s2 * h00 + c2 * h01;
-                G[Q1][P2] = c2 * h10 - s2 * h11;
-                G[Q1][Q2] = s2 * h10 + c2 * h11;
-            }
-            // J <- J R
-            for (int e = tid; e < (JW / 2) * JW; e += 256) {
-                const int pi = e / JW, row = e % JW;
-                const int P = rp[pi], Q = rq[pi];
-                const double c = rc[pi], s = rs[pi];
-                const double jp = J[row][P], jq = J[row][Q];
-                J[row][P] = c * jp - s * jq;
-                J[row][Q] = s * jp + c * jq;
-            }
-            __syncthreads();
-        }
-        if (any_rot == 0) break;
+    // 2. one sweep of cyclic parallel Jacobi on G (tournament ordering, 31
+    // rounds).  The round's pairs are disjoint, so G <- R^T G R splits into
+    // 16 x 16 independent 2 x 2 blocks (rows P1, Q1 of pair bi, columns P2, Q2
+    // of pair bj), one per thread; J <- J R in place, rows 2 bi and 2 bi + 1 of
+    // the columns P2, Q2.
+    const int bi = tid >> 4, bj = tid & 15;
+#pragma unroll 1
+    for (int round = 0; round < JW - 1; round++) {
+        auto elem = [&](int kpos) {
+            const int k = kpos - 1 + round;
+            return kpos == 0 ? 0 : (k >= JW - 1 ? k - (JW - 1) : k) + 1;
+        };
+        const int a1 = elem(bi), b1 = elem(JW - 1 - bi), a2 = elem(bj), b2 = elem(JW - 1 - bj);
+        const int P1 = min(a1, b1), Q1 = max(a1, b1), P2 = min(a2, b2), Q2 = max(a2, b2);
+        const double(*Gc)[JW + 1] = G[round & 1];
+        double(*Gn)[JW + 1] = G[(round & 1) ^ 1];
+        const double g00 = Gc[P1][P2], g01 = Gc[P1][Q2], g10 = Gc[Q1][P2], g11 = Gc[Q1][Q2];
+        const double p2 = Gc[P2][P2], q2 = Gc[Q2][Q2], o2 = Gc[P2][Q2];
+        const double j00 = J[2 * bi][P2], j01 = J[2 * bi][Q2], j10 = J[2 * bi + 1][P2], j11 = J[2 * bi + 1][Q2];
+        // lanes bj of every 16 hold the rotation of pair bj; that of pair bi
+        // comes from lane bi
+        double c2, s2;
+        jacobi_rot(p2, q2, o2, c2, s2);
+        const double c1 = __shfl(c2, bi, 64), s1 = __shfl(s2, bi, 64);
+        const double h00 = c1 * g00 - s1 * g10, h01 = c1 * g01 - s1 * g11;
+        const double h10 = s1 * g00 + c1 * g10, h11 = s1 * g01 + c1 * g11;
+        Gn[P1][P2] = c2 * h00 - s2 * h01;
+        Gn[P1][Q2] = s2 * h00 + c2 * h01;
+        Gn[Q1][P2] = c2 * h10 - s2 * h11;
+        Gn[Q1][Q2] = s2 * h10 + c2 * h11;
+        J[2 * bi][P2] = c2 * j00 - s2 * j01;
+        J[2 * bi][Q2] = s2 * j00 + c2 * j01;
+        J[2 * bi + 1][P2] = c2 * j10 - s2 * j11;
+        J[2 * bi + 1][Q2] = s2 * j10 + c2 * j11;
         __syncthreads();
     }
 
-    // 3. X[:, cols] <- X[:, cols] J ; V[:, cols] <- V[:, cols] J (J read in
-    // 16-byte column pairs, the same for every lane)
-    for (int row = xr0 + tid; row < xr1; row += 256) {
-        double x[JW];
+    // 3. X[:, cols] <- X[:, cols] J ; V[:, cols] <- V[:, cols] J
+    auto product = [&](const double (&x)[JW], double (&y)[4]) {
 #pragma unroll
-        for (int c = 0; c < JW; c++) x[c] = Xs[(long)colidx(c) * ldx + row];
-#pragma unroll 2
-        for (int c2 = 0; c2 < JW; c2 += 2) {
-            double s0 = 0.0, s1 = 0.0;
+        for (int u = 0; u < 4; u++) y[u] = 0.0;
 #pragma unroll
-            for (int c = 0; c < JW; c++) {
-                const double2 jj = *(const double2*)&J[c][c2];
-                s0 = fma(x[c], jj.x, s0);
-                s1 = fma(x[c], jj.y, s1);
-            }
-            Xd[(long)colidx(c2) * ldx + row] = s0;
-            Xd[(long)colidx(c2 + 1) * ldx + row] = s1;
+        for (int c = 0; c < JW; c++) {
+            const double2 ja = *(const double2*)&J[c][4 * ac], jb = *(const double2*)&J[c][4 * ac + 2];
+            y[0] = fma(x[c], ja.x, y[0]);
+            y[1] = fma(x[c], ja.y, y[1]);
+            y[2] = fma(x[c], jb.x, y[2]);
+            y[3] = fma(x[c], jb.y, y[3]);
+        }
+    };
+    for (int r0 = xr0; r0 < xr1; r0 += 32) {
+        const int row = r0 + ar;
+        if (r0 > xr0) {
+#pragma unroll
+            for (int c = 0; c < JW; c++) x[c] = Xs[(long)colidx(c) * ldx + min(row, p - 1)];
+        }
+        double y[4];
+        product(x, y);
+        if (row < xr1) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) Xd[(long)colidx(4 * ac + u) * ldx + row] = y[u];
         }
     }
-    for (int row = vr0 + tid; row < vr1; row += 256) {
-        double x[JW];
+    for (int r0 = vr0; r0 < vr1; r0 += 32) {
+        const int row = r0 + ar;
+        if (r0 > vr0) {
 #pragma unroll
-        for (int c = 0; c < JW; c++) x[c] = V[(long)colidx(c) * ldv + row];
-#pragma unroll 2
-        for (int c2 = 0; c2 < JW; c2 += 2) {
-            double s0 = 0.0, s1 = 0.0;
+            for (int c = 0; c < JW; c++) v[c] = V[(long)colidx(c) * ldv + min(row, qv - 1)];
+        }
+        double y[4];
+        product(v, y);
+        __syncthreads();  // in place: every thread of these rows has read them
+        if (row < vr1) {
 #pragma unroll
-            for (int c = 0; c < JW; c++) {
-                const double2 jj = *(const double2*)&J[c][c2];
-                s0 = fma(x[c], jj.x, s0);
-                s1 = fma(x[c], jj.y, s1);
-            }
-            V[(long)colidx(c2) * ldv + row] = s0;
-            V[(long)colidx(c2 + 1) * ldv + row] = s1;
+            for (int u = 0; u < 4; u++) V[(long)colidx(4 * ac + u) * ldv + row] = y[u];
         }
     }
 }
 
 hipError_t jacobi_step(const double* Xs, double* Xd, long ldx, int p, double* V, long ldv, int qv,
-                       const int* pairs, int npairs, int nchunk, double tol, int* flag, hipStream_t s, int inner)
+                       const int* pairs, int npairs, int nchunk, double tol, int* flag, hipStream_t s)
 {
     if (npairs <= 0) return hipSuccess;
     if (nchunk < 1 || nchunk > 64 || Xs == Xd) return hipErrorInvalidValue;
-    jacobi_k<<<dim3(npairs, nchunk), 256, 0, s>>>(Xs, Xd, ldx, p, V, ldv, qv, pairs, tol, flag, inner);
+    jacobi_k<<<dim3(npairs, nchunk), 256, 0, s>>>(Xs, Xd, ldx, p, V, ldv, qv, pairs, tol, flag);
     return hipGetLastError();
 }
 
