@@ -914,7 +914,6 @@ static hipError_t launch_x3(int code, const GemmX3Params& p, int batch, hipStrea
     return hipGetLastError();
 }
 
-static int choose_tile(int M, int N, int batch);
 // the split-bfloat16 product: K-major planes only, K a multiple of 32
 static hipError_t gemm_x3(const GemmDesc& g, hipStream_t s)
 {
@@ -926,7 +925,12 @@ static hipError_t gemm_x3(const GemmDesc& g, hipStream_t s)
     p.sA = g.sA; p.sB = g.sB; p.sC = g.sC;
     p.psA = g.psA; p.psB = g.psB;
     p.alpha = g.alpha; p.accumulate = g.accumulate;
-    const int code = g.tile > 0 ? g.tile - 1 : choose_tile(g.M, g.N, g.batch);
+    int code = g.tile - 1;
+    if (g.tile <= 0) {
+        int ks;
+        gemm_default(g.tin, g.M, g.N, g.K, g.batch, false, &code, &ks);
+        code--;
+    }
     if (code < 0 || code >= kNumTiles || g.M % kTiles[code].bm || g.N % kTiles[code].bn) return hipErrorInvalidValue;
     if (kTiles[code].deep && g.K % 64) return hipErrorInvalidValue;
     if (g.tout == T_F32) return launch_x3<float>(code, p, g.batch, s);
@@ -945,6 +949,7 @@ bool gemm_tile_ok(int code, int tin, int M, int N, int K)
 }
 int gemm_tile_bm(int code) { return (code >= 1 && code <= kNumTiles) ? kTiles[code - 1].bm : 0; }
 int gemm_tile_bn(int code) { return (code >= 1 && code <= kNumTiles) ? kTiles[code - 1].bn : 0; }
+static int choose_tile(int M, int N, int batch);
 int gemm_grouped_tile(int M, int N) { return choose_tile(M, N, 1) + 1; }
 int gemm_k_step(int tin, int K)
 {
@@ -965,7 +970,7 @@ hipError_t gemm_grouped(int tin, int tout, bool akm, bool bkm, int tile, int bk,
     return grouped_layout<false, true>(tin, tout, tile - 1, bk, probs, off, nprob, grid, s);
 }
 
-// bf16 and split bf16: pick the largest tile that divides the problem and still
+// bf16 and grouped launches: pick the largest tile that divides the problem and still
 // gives >= ~1.5 workgroups per CU (256 CUs); fall back to the tile with the
 // most blocks.
 static int choose_tile(int M, int N, int batch)
@@ -981,43 +986,50 @@ static int choose_tile(int M, int N, int batch)
     return best;
 }
 
-// FP64 / FP32 tile and k-split from a model of the time, in us, fitted to the
+// FP64, FP32 and split-bf16 tile and k-split from a model of the time, in us, fitted to the
 // tiles timed one by one (M x N x K from 32 x 96 x 128 to 3072 x 4096 x 1024, all
 // layouts; within 8 % of the measured time from 5 us up):
 //   3.7 + steps * max(n * busy, alone)   + for a split  3 + bytes / 10 TB/s
 // steps: K steps (16 FP64, 32 FP32 values) of one workgroup; n: workgroups on the
 // fullest CU; busy: matrix-pipe time of a workgroup's step; alone: the step of a
 // workgroup that has a CU to itself (copy, barrier and instruction latency).
-struct PipeCost { int code; float busy64, alone64, busy32, alone32; };
-static const PipeCost kPipeCost[] = {
-    {1, 0.933f, 1.05f, 1.016f, 1.15f},   // 128x64
-    {2, 0.933f, 1.05f, 1.016f, 1.15f},   // 64x128
-    {3, 0.485f, 0.53f, 0.608f, 0.70f},   // 64x64
-    {4, 0.259f, 0.30f, 0.353f, 0.45f},   // 32x64
-    {5, 0.259f, 0.30f, 0.353f, 0.45f},   // 64x32
-    {6, 0.138f, 0.235f, 0.205f, 0.355f}, // 32x32
-};
+struct StepCost { int code; float busy, alone; };
+static const StepCost kCostF64[] = {  // 128x64, 64x128, 64x64, 32x64, 64x32, 32x32
+    {1, 0.933f, 1.05f}, {2, 0.933f, 1.05f}, {3, 0.485f, 0.53f}, {4, 0.259f, 0.30f}, {5, 0.259f, 0.30f},
+    {6, 0.138f, 0.235f}};
+static const StepCost kCostF32[] = {
+    {1, 1.016f, 1.15f}, {2, 1.016f, 1.15f}, {3, 0.608f, 0.70f}, {4, 0.353f, 0.45f}, {5, 0.353f, 0.45f},
+    {6, 0.205f, 0.355f}};
+// split bf16 (steps of 32): 128x128 .. 32x32, 96x128, 128x96, 192x256, 256x192,
+// 192x128, 128x192.  1024 x 3072 x 4096: 208 us in the 128x64 tiles of the
+// block-count rule, 134 us in 128x192 with a 2-way split (1.15 PFLOP/s of bf16);
+// 512 x 1536 x 2048: 36 -> 32 us; 320 x 448 x 1280: 19 -> 12 us
+static const StepCost kCostX3[] = {
+    {0, 1.42f, 1.60f}, {1, 0.715f, 1.00f}, {2, 0.708f, 1.00f}, {3, 0.418f, 0.60f},  {4, 0.285f, 0.41f},
+    {5, 0.274f, 0.36f}, {6, 0.167f, 0.266f}, {10, 1.02f, 1.48f}, {11, 1.00f, 1.48f}, {12, 4.0f, 4.0f},
+    {13, 4.0f, 4.0f}, {14, 2.0f, 2.0f}, {15, 1.95f, 1.95f}};
 void gemm_default(int tin, int M, int N, int K, int batch, bool split, int* tile, int* ksplit)
 {
     *ksplit = 1;
-    if (tin != T_F64 && tin != T_F32) {
+    const StepCost* cost = tin == T_F64 ? kCostF64 : (tin == T_F32 ? kCostF32 : kCostX3);
+    const int ncost = tin == T_BF16X3 ? (int)(sizeof(kCostX3) / sizeof(kCostX3[0])) : 6;
+    if (tin == T_BF16) {
         *tile = choose_tile(M, N, batch) + 1;
         return;
     }
-    const bool f64 = tin == T_F64;
-    const int bk = f64 ? 16 : 32;
+    const int bk = tin == T_F64 ? 16 : 32, es = tin == T_F64 ? 8 : 4;
     float best = 1e30f;
     *tile = 7;
-    for (const PipeCost& c : kPipeCost) {
+    for (int q = 0; q < ncost; q++) {
+        const StepCost& c = cost[q];
         const TileCfg& t = kTiles[c.code];
         if (M % t.bm || N % t.bn) continue;
         for (int ks = 1; ks <= 4; ks *= 2) {
             if (ks > 1 && (!split || batch != 1 || K % (64 * ks))) break;
             const long blocks = (long)(M / t.bm) * (N / t.bn) * batch * ks;
-            const float n = (float)((blocks + 255) / 256);
-            const float busy = n * (f64 ? c.busy64 : c.busy32), alone = f64 ? c.alone64 : c.alone32;
-            float us = 3.7f + (float)(K / ks) / bk * (busy > alone ? busy : alone);
-            if (ks > 1) us += 3.0f + (float)M * N * (2 * ks * (f64 ? 8 : 4) + 8) * 1e-7f;
+            const float busy = (float)((blocks + 255) / 256) * c.busy;
+            float us = 3.7f + (float)(K / ks) / bk * (busy > c.alone ? busy : c.alone);
+            if (ks > 1) us += 3.0f + (float)M * N * (2 * ks * es + 8) * 1e-7f;
             if (us < best) {
                 best = us;
                 *tile = c.code + 1;

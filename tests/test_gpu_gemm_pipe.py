@@ -66,3 +66,19 @@ def test_heff_with_built_in_split(ctx, D1, D2, d, prec, u):
     size = contract(np.abs(W), np.abs(L), np.abs(R), np.abs(x))
     # one rounding per term of the three nested sums
     assert np.all(np.abs(y - ref) <= (D2 + 3 * d + 3 * D1 + 8) * u * size)
+
+
+@pytest.mark.parametrize("M,N,K", [(32, 64, 128), (192, 256, 256), (256, 192, 512), (320, 448, 1280), (1024, 384, 1024),
+                                   (192, 128, 448), (96, 32, 32)])
+def test_split_bf16_built_in_tile(ctx, M, N, K):
+    # tile 0: the built-in tile of the split product, with and without a k-split
+    rng = np.random.default_rng(M + N + K)
+    A, B = rng.uniform(-1.0, 1.0, (M, K)), rng.uniform(-1.0, 1.0, (K, N))
+    ref, size = A @ B, np.abs(A) @ np.abs(B)
+    for ksplit in (1, 2, 4):
+        if ksplit > 1 and K % (64 * ksplit):
+            continue
+        C = ctx.gemm_test(A, np.ascontiguousarray(B.T), tn.TN_BF16X3, 0 if ksplit > 1 else 1, True, True, M, N, K, 1,
+                          0, ksplit)[0]
+        # 24-bit operands, six products and one FP32 rounding per k
+        assert np.all(np.abs(C - ref) <= (7 * K + 8) * 2.0 ** -24 * size)
