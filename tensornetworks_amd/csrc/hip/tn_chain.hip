@@ -1125,8 +1125,12 @@ int tn_heff_apply_device(tn_ctx* c, const double* x, double* y, int64_t N)
     TN_REQUIRE(x && y && N == (int64_t)c->b_d * c->b_D1 * c->b_D2, TN_ERR_ARG,
                "tn_heff_apply_device: N != d*D1*D2");
     const int d = c->b_d, D1 = c->b_D1, D2 = c->b_D2, D1p = pad32(D1), D2p = pad32(D2);
-    TN_HIP(psi_ref_to_int(x, c->b_x.as<double>(), d, D1, D2, D1p, D2p, c->stream));
     HeffOp op = bound_op(c);
+    if (heff_apply_ref(c, op, D1, D2, x, y)) {
+        sync(c);
+        return TN_OK;
+    }
+    TN_HIP(psi_ref_to_int(x, c->b_x.as<double>(), d, D1, D2, D1p, D2p, c->stream));
     heff_apply(c, op, c->b_x.as<double>(), c->b_y.as<double>(), false);
     TN_HIP(psi_int_to_ref(c->b_y.as<double>(), y, d, D1, D2, D2p, c->stream));
     sync(c);
@@ -1153,6 +1157,10 @@ int tn_heff_apply_device_noalloc(tn_ctx* c, const double* x, double* y, int64_t 
     TN_REQUIRE(total <= kNoAllocBytes, TN_ERR_ARG,
                "tn_heff_apply_device_noalloc: this site needs " + std::to_string(total) +
                    " bytes of work space, above the fixed " + std::to_string(kNoAllocBytes) + " bytes");
+    if (heff_apply_ref(c, op, D1, D2, x, y)) {
+        sync(c);
+        return TN_OK;
+    }
     char* base = (char*)c->noalloc;
     double* xi = (double*)base;
     double* yi = (double*)(base + bv);
@@ -2015,10 +2023,10 @@ int tn_chain_heff_bench(tn_chain* ch, int site, int precision, int reps, int ski
     const long N = op.n();
     c->b_y.ensure((size_t)N * 8);
     double a = 0, b = 0, e = 0;
-    heff_apply(c, op, ch->A[site], c->b_y.as<double>(), true);  // warm
+    heff_apply(c, op, ch->A[site], c->b_y.as<double>(), true, nullptr, true);  // warm
     sync(c);
     for (int r = 0; r < reps; r++) {
-        heff_apply(c, op, ch->A[site], c->b_y.as<double>(), true);
+        heff_apply(c, op, ch->A[site], c->b_y.as<double>(), true, nullptr, true);
         double x1, x2, x3;
         heff_stage_times(c, &x1, &x2, &x3);
         a += x1;

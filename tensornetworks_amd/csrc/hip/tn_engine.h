@@ -109,6 +109,11 @@ struct tn_ctx {
     // factor (within its first pass over it) and resets it; set by the Lanczos
     // driver right before the apply of a new basis vector
     double x_prescale = 0.0;
+    // nonzero after heff_apply: the result is of the scaled input, but the input
+    // itself still has to be scaled by this factor (one-launch apply)
+    double x_postscale = 0.0;
+    // the last timed apply was one launch: only ev[0] and ev[4] were recorded
+    bool ev_single = false;
     // seam state (tn_site_bind)
     int b_d = 0, b_D1 = 0, b_D2 = 0, b_Dw1 = 0, b_Dw2 = 0, b_prec = 0;
     int b_wl = -1, b_wr = -1;  // identity channels of the bound environments
@@ -175,11 +180,16 @@ struct HeffScratch {
 size_t heff_scratch_bytes(const HeffOp& op, size_t* t1, size_t* t2, size_t* xlo);
 // GEMM with the table's tile (or the built-in one), one launch, no tuning
 void gemm_run_fixed(tn_ctx* c, const GemmDesc& g);
-// y = Heff x (fp64 in/out).  timed: HIP events around the stages (read by
-// heff_timing_read / heff_stage_times).  scr: caller work space (see HeffScratch),
-// nullptr = the context's buffers.
+// y = Heff x (fp64 in/out; x and y do not overlap).  timed: HIP events around the
+// stages (read by heff_timing_read / heff_stage_times).  scr: caller work space
+// (see HeffScratch), nullptr = the context's buffers.  stages: never the
+// one-launch form of small FP64 sites (whose stages have no times of their own).
 void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool timed,
-                const HeffScratch* scr = nullptr);
+                const HeffScratch* scr = nullptr, bool stages = false);
+// y = Heff x of a small FP64 site in one launch with x and y in the reference
+// layout (D1 x D2 logical); false when the site or the pointers (x and y
+// overlapping) do not allow it
+bool heff_apply_ref(tn_ctx* c, const HeffOp& op, int D1, int D2, const double* x, double* y);
 void heff_timing_read(tn_ctx* c, double* gemm_ms, double* total_ms);
 // per-stage times of the last timed apply (ms): s1, mix, s3
 void heff_stage_times(tn_ctx* c, double* s1, double* mix, double* s3);
@@ -217,7 +227,7 @@ typedef void (*ApplyFn)(tn_ctx* c, const void* op, const double* x, double* y);
 // against the whole basis every iteration
 //
 // prescale: fn applies the Heff through heff_apply, which honours
-// tn_ctx::x_prescale; the scaling v_{j+1} = w / beta_j is then left to the
+// tn_ctx::x_prescale (and leaves x_postscale); the scaling v_{j+1} = w / beta_j is then left to the
 // next apply's first pass over its input instead of a separate kernel
 LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, double tol,
                       int max_krylov, int max_restarts, double tol_rel = 0.0, bool partial = false,

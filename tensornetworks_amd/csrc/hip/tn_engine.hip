@@ -353,13 +353,40 @@ size_t heff_scratch_bytes(const HeffOp& op, size_t* t1, size_t* t2, size_t* xlo)
     return up(a) + up(b) + up(x);
 }
 
-void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool timed, const HeffScratch* scr)
+static HeffSmall small_apply(const HeffOp& op, const double* x, double* y)
+{
+    HeffSmall a{};
+    a.p = op.p; a.D1p = op.D1p; a.D2p = op.D2p; a.Dw1 = op.Dw1; a.wl = op.wl_id;
+    a.nR = op.Dw2 - (op.wr_id >= 0 ? 1 : 0);
+    a.nL = op.Dw1 - (op.wl_id >= 0 ? 1 : 0);
+    a.x = x; a.y = y; a.scale = 1.0;
+    a.L = op.L + (op.wl_id == 0 ? op.D1p : 0);
+    a.R = op.R + (op.wr_id == 0 ? (long)op.D2p * op.D2p : 0);
+    a.t = op.mix->t;
+    return a;
+}
+
+bool heff_apply_ref(tn_ctx* c, const HeffOp& op, int D1, int D2, const double* x, double* y)
+{
+    const size_t n = (size_t)op.p * D1 * D2;
+    if (op.precision != TN_FP64 || op.tile != 0 || (x < y + n && y < x + n)) return false;
+    HeffSmall a = small_apply(op, x, y);
+    a.D1 = D1;
+    a.D2 = D2;
+    if (!heff_small_ok(a)) return false;
+    TN_HIP(heff_small(a, c->stream));
+    return true;
+}
+
+void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool timed, const HeffScratch* scr,
+                bool stages)
 {
     // a pending Lanczos scaling of x (x is then the driver's own basis vector,
     // scaled in place within the first pass over it), taken before anything
     // can throw
     const double pre = c->x_prescale;
-    c->x_prescale = 0.0;
+    c->x_prescale = c->x_postscale = 0.0;
+    c->ev_single = false;
     double* const xs = pre != 0.0 ? const_cast<double*>(x) : nullptr;
     hipStream_t s = c->stream;
     const int p = op.p, D1p = op.D1p, D2p = op.D2p, Dw1 = op.Dw1, Dw2 = op.Dw2;
@@ -420,6 +447,19 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
         if (scr) gemm_run_fixed(c, g);
         else gemm_run(c, g, true);
     };
+    if (op.precision == TN_FP64 && op.tile == 0 && !stages) {
+        HeffSmall a = small_apply(op, x, y);
+        if (heff_small_ok(a)) {
+            if (xs) {  // H (pre x); the caller scales x with its next pass over it
+                a.scale = pre;
+                c->x_postscale = pre;
+            }
+            TN_HIP(heff_small(a, s));
+            if (timed) TN_HIP(hipEventRecord(c->ev[4], s));
+            c->ev_single = true;
+            return;
+        }
+    }
     if (op.precision == TN_FP64) {
         if (!scr) {
             c->T1.ensure(n1 * 8);
@@ -506,6 +546,12 @@ void heff_timing_read(tn_ctx* c, double* gemm_ms, double* total_ms)
 {
     float t01 = 0, t12 = 0, t23 = 0, t34 = 0;
     TN_HIP(hipEventSynchronize(c->ev[4]));
+    if (c->ev_single) {
+        TN_HIP(hipEventElapsedTime(&t01, c->ev[0], c->ev[4]));
+        if (gemm_ms) *gemm_ms += t01;
+        if (total_ms) *total_ms += t01;
+        return;
+    }
     TN_HIP(hipEventElapsedTime(&t01, c->ev[0], c->ev[1]));
     TN_HIP(hipEventElapsedTime(&t12, c->ev[1], c->ev[2]));
     TN_HIP(hipEventElapsedTime(&t23, c->ev[2], c->ev[3]));
@@ -860,21 +906,36 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
             try {
                 fn(c, op, vj, hv);
             } catch (...) {
-                c->x_prescale = 0.0;
+                c->x_prescale = c->x_postscale = 0.0;
                 throw;
             }
+            const double post = c->x_postscale;  // v_j still to be scaled by this
+            c->x_postscale = 0.0;
             res.n_matvec++;
             // three-term step with the exact alpha = v_j.w (h[0] on the device),
             // then one classical Gram-Schmidt pass against every Krylov vector
             // (h[1..j+1]) removes what rounding left; |w|^2 comes last
-            TN_HIP(lz_dot(vj, hv, N, part, s));
-            if (pro) {
-                // the same step and pass against v_{j-1}, v_j only
-                const int kk = j >= 1 ? 2 : 1;
-                const double* Vl = V + (long)(j + 1 - kk) * N;
-                TN_HIP(lz_step(hv, w, Vl, N, kk, true, j > 0 ? be[j - 1] : 0.0, N, h, part, s));
+            // (partial: the same step and pass against v_{j-1}, v_j only).  Short
+            // vectors take the whole step in one launch, which also divides w by
+            // |w| unless a pass against the whole basis may still follow.
+            const int kk = pro ? (j >= 1 ? 2 : 1) : j + 1;
+            double* Vl = V + (long)(j + 1 - kk) * N;
+            const double beta = j > 0 ? be[j - 1] : 0.0;
+            const bool tiny = lz_small_ok(N, kk);
+            if (tiny) {
+                const unsigned long long seq = ++c->sc.seq;
+                TN_HIP(lz_small(hv, Vl, N, kk, post != 0.0 ? post : 1.0, beta, !pro, N, c->sc.d, c->sc.flag_d, seq, s));
+                read_published(c, hh.data(), kk + 2, seq);
+            } else {
+                if (post != 0.0) TN_HIP(scale_copy(post, vj, vj, N, s));
+                TN_HIP(lz_dot(vj, hv, N, part, s));
+                // three-term step fused with the Gram-Schmidt dot products, then
+                // the Gram-Schmidt update fused with the norm
+                TN_HIP(lz_step(hv, w, Vl, N, kk, true, beta, N, h, part, s));
                 TN_HIP(lz_update(w, Vl, N, kk, N, h + 1, part, s));
                 read(hh.data(), kk + 1);
+            }
+            if (pro) {
                 al[j] = hh[0] + hh[kk];
                 be[j] = std::sqrt(std::max(hh[kk + 1], 0.0));
                 tnorm = std::max(tnorm, std::fabs(al[j]) + be[j] + (j > 0 ? be[j - 1] : 0.0));
@@ -908,11 +969,6 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
                 std::swap(om_old, om);
                 std::swap(om, om_new);
             } else {
-                // three-term step fused with the Gram-Schmidt dot products, then
-                // the Gram-Schmidt update fused with the norm
-                TN_HIP(lz_step(hv, w, V, N, j + 1, true, j > 0 ? be[j - 1] : 0.0, N, h, part, s));
-                TN_HIP(lz_update(w, V, N, j + 1, N, h + 1, part, s));
-                read(hh.data(), j + 2);
                 al[j] = hh[0] + hh[j + 1];
                 be[j] = std::sqrt(std::max(hh[j + 2], 0.0));
                 tnorm = std::max(tnorm, std::fabs(al[j]) + be[j] + (j > 0 ? be[j - 1] : 0.0));
@@ -933,7 +989,7 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
                 conv = true;
                 break;
             }
-            if (j + 1 < kmax) {
+            if (j + 1 < kmax && !(tiny && !pro)) {
                 if (prescale) pending = 1.0 / be[j];
                 else TN_HIP(scale_copy(1.0 / be[j], w, w, N, s));
             }

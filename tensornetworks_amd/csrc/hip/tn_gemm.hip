@@ -1407,4 +1407,205 @@ hipError_t x3_stage1_mix(int p, int nR, const bf16* X, long psX, const bf16* R, 
     return hipErrorInvalidValue;
 }
 
+// ---------------------------------------------------------------------------
+// The whole FP64 Heff apply of a small site in one launch (left bond padded to
+// 32, right bond to 32 or 64).  A workgroup owns 16 of the b columns of y: stage 1
+// for those b (T1 in LDS, one 16-column block per kept right channel, and x itself
+// as one more block for the identity channel), then stage 3, whose right operand
+// (the MPO stage's output) is formed in registers from T1 as the matrix
+// instruction needs it.  16 waves: stage 1 wave = (row tile, channel group), stage
+// 3 wave = (m, slice of the K sum over (w, a')), the slices summed through LDS.
+// Bound by the latency of its loads and of the two stages; the three-kernel path
+// pays that, a launch and a drain three times: D = 32, d = 2, four channels 9.4 us
+// here; a host call at D = 8 (padded to 32) took 28 us with the three kernels and
+// the two layout passes, 18.6 us with this one.  A left bond of 64 makes one
+// workgroup's share of the work too large (measured at D = 64, d = 2: 26 us against
+// 14 us of kernels and two launch gaps), so it keeps the three kernels.
+constexpr int HS_LDS = 116 * 1024;
+constexpr int HS_MAXO = 64, HS_MAXE = 256;
+
+static inline int hs_pad(int p) { return p == 2 ? 2 : (p == 3 ? 4 : 1); }  // spreads the four lane groups over the banks
+bool heff_small_ok(const HeffSmall& a)
+{
+    return a.p >= 2 && a.p <= 4 && a.D1p == 32 && (a.D2p == 32 || a.D2p == 64) && a.nR >= 1 && a.nL >= 1 &&
+           a.t.ocode && a.t.ecode && a.t.nout <= HS_MAXO && a.t.nnz <= HS_MAXE &&
+           32L * a.p * ((a.nR + 1) * 16 + hs_pad(a.p)) * 8 <= HS_LDS;
+}
+
+template <int P, int D2P, bool REF>
+__global__ void __launch_bounds__(1024) heff_small_k(HeffSmall q)
+{
+    typedef MT<double> T;
+    constexpr int NT = 1024, NW = 16, D1P = 32, RT = D1P * P / 16, KB = D2P / 16, AT = D1P / 16;
+    constexpr int CG = NW / RT;  // channel groups of stage 1
+    constexpr int PAD = P == 2 ? 2 : (P == 3 ? 4 : 1);
+    constexpr int SL = NW / P;   // K slices of stage 3
+    static_assert(SL * P * D1P * 16 * 8 <= HS_LDS, "partial sums");
+    __shared__ __attribute__((aligned(16))) double sm[HS_LDS / 8];
+    __shared__ int s_optr[HS_MAXO + 1], s_ecode[HS_MAXE];
+    __shared__ double s_val[HS_MAXE];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int r = lane & 15, kq = lane >> 4;
+    const int b0 = blockIdx.x * 16;
+    const int ld1 = (q.nR + 1) * 16 + PAD;
+    // element (row (a', n), b') of x
+    auto xat = [&](int row, int b) -> double {
+        if constexpr (REF) return row < P * q.D1 && b < q.D2 ? q.x[row + (long)P * q.D1 * b] : 0.0;
+        else return q.x[(long)row * D2P + b];
+    };
+    // K index of a block's value e of lane group kq: two 16-byte units per lane,
+    // the four groups side by side
+    auto kof = [&](int e) { return ((e >> 1) * 4 + kq) * 2 + (e & 1); };
+    // every first load is in flight before anything waits: the stage-1 operands,
+    // stage 3's first block of L, x's own columns, the table
+    double a[KB][4], bv[2][KB][4], la[AT][4];
+    const int rt = wid % RT, cg = wid / RT;  // stage 1: row tile, channels cg, cg + CG, ...
+    const int nkb = q.nL * AT;
+    const int m = wid % P, sl = wid / P;  // stage 3: column block m, K blocks sl, sl + SL, ...
+    auto loadR = [&](int ch, int h) {
+        const double* Rw = q.R + ((long)ch * D2P + b0 + r) * D2P;
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) bv[h][kb][e] = Rw[kb * 16 + kof(e)];
+    };
+    auto loadL = [&](int kb) {
+        const double* Lw = q.L + (long)(kb / AT) * D1P + (kb % AT) * 16;
+#pragma unroll
+        for (int i = 0; i < AT; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) la[i][e] = Lw[(long)(i * 16 + r) * q.Dw1 * D1P + kof(e)];
+    };
+    const bool s1 = cg < CG && cg < q.nR;
+    if (s1) {
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) a[kb][e] = xat(rt * 16 + r, kb * 16 + kof(e));
+        loadR(cg, 0);
+        if (cg + CG < q.nR) loadR(cg + CG, 1);
+    }
+    if (sl < SL && sl < nkb) loadL(sl);
+    constexpr int XN = (D1P * P * 16 + NT - 1) / NT;
+    double xs[XN];
+#pragma unroll
+    for (int u = 0; u < XN; u++) {
+        const int i = tid + u * NT;
+        const int row = REF ? i % (D1P * P) : i >> 4, b = REF ? i / (D1P * P) : i & 15;
+        if (i < D1P * P * 16) xs[u] = xat(row, b0 + b);
+    }
+    static_assert(HS_MAXO < NT && HS_MAXE <= NT, "one table entry per thread");
+    const int to = tid <= q.t.nout ? q.t.optr[tid] : 0, te = tid < q.t.nnz ? q.t.ecode[tid] : 0;
+    const double tv = tid < q.t.nnz ? q.t.eval[tid] : 0.0;
+    if (tid <= q.t.nout) s_optr[tid] = to;
+    if (tid < q.t.nnz) {
+        s_ecode[tid] = te;
+        s_val[tid] = tv;
+    }
+    // x's own 16 columns: the block after the kept channels
+#pragma unroll
+    for (int u = 0; u < XN; u++) {
+        const int i = tid + u * NT;
+        const int row = REF ? i % (D1P * P) : i >> 4, b = REF ? i / (D1P * P) : i & 15;
+        if (i < D1P * P * 16) sm[row * ld1 + q.nR * 16 + b] = xs[u];
+    }
+    // stage 1: T1[(a', n)][(w', b)]
+    auto step = [&](int ch, int h) {
+        v4d acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int kb = 0; kb < KB; kb++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc = mma(a[kb][e], bv[h][kb][e], acc);
+        if (ch + 2 * CG < q.nR) loadR(ch + 2 * CG, h);
+        double* d = sm + rt * 16 * ld1 + ch * 16 + r;
+#pragma unroll
+        for (int i = 0; i < 4; i++) d[T::crow(lane, i) * ld1] = acc[i];
+    };
+    if (s1) {
+        for (int ch = cg; ch < q.nR; ch += 2 * CG) {
+            step(ch, 0);
+            if (ch + CG < q.nR) step(ch + CG, 1);
+        }
+    }
+    __syncthreads();
+    v4d acc[AT];
+#pragma unroll
+    for (int i = 0; i < AT; i++) acc[i] = v4d{0.0, 0.0, 0.0, 0.0};
+    if (sl < SL) {
+        if (sl == 0 && q.wl >= 0) {  // the left identity channel: a' = a
+            const int o = q.wl * P + m;
+            for (int e = s_optr[o]; e < s_optr[o + 1]; e++) {
+                const int ec = s_ecode[e];
+                const int ch = ec >> 16 ? q.nR : (ec >> 8) & 255;
+                const double* src = sm + (ec & 255) * ld1 + ch * 16 + r;
+                const double v = s_val[e];
+#pragma unroll
+                for (int i = 0; i < AT; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) acc[i][j] += v * src[(i * 16 + T::crow(lane, j)) * P * ld1];
+            }
+        }
+        for (int kb = sl; kb < nkb; kb += SL) {
+            const int w = kb / AT;
+            const int o = (w + (q.wl == 0 ? 1 : 0)) * P + m;
+            double b3[4] = {0.0, 0.0, 0.0, 0.0};
+            const int a0 = (kb % AT) * 16;
+            for (int e = s_optr[o]; e < s_optr[o + 1]; e++) {
+                const int ec = s_ecode[e];
+                const int ch = ec >> 16 ? q.nR : (ec >> 8) & 255;
+                const double* src = sm + (ec & 255) * ld1 + ch * 16 + r;
+                const double v = s_val[e];
+#pragma unroll
+                for (int u = 0; u < 4; u++) b3[u] += v * src[(a0 + kof(u)) * P * ld1];
+            }
+            double ca[AT][4];
+#pragma unroll
+            for (int i = 0; i < AT; i++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) ca[i][u] = la[i][u];
+            if (kb + SL < nkb) loadL(kb + SL);
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int i = 0; i < AT; i++) acc[i] = mma(ca[i][u], b3[u], acc[i]);
+        }
+    }
+    __syncthreads();  // T1 is no longer read
+    if (sl < SL) {
+        double* d = sm + (sl * P + m) * D1P * 16 + r;
+#pragma unroll
+        for (int i = 0; i < AT; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) d[(i * 16 + T::crow(lane, j)) * 16] = acc[i][j];
+    }
+    __syncthreads();
+    for (int i = tid; i < D1P * P * 16; i += NT) {
+        const int row = REF ? i % (D1P * P) : i >> 4, b = REF ? i / (D1P * P) : i & 15;
+        const int mm = row % P, aa = row / P;
+        double s = 0.0;
+#pragma unroll
+        for (int z = 0; z < SL; z++) s += sm[((z * P + mm) * D1P + aa) * 16 + b];
+        if constexpr (REF) {
+            if (aa < q.D1 && b0 + b < q.D2) q.y[row + (long)P * q.D1 * (b0 + b)] = q.scale * s;
+        } else {
+            q.y[(long)row * D2P + b0 + b] = q.scale * s;
+        }
+    }
+}
+
+hipError_t heff_small(const HeffSmall& a, hipStream_t s)
+{
+    if (!heff_small_ok(a)) return hipErrorInvalidValue;
+    const dim3 grid(a.D2p / 16);
+#define HS_CASE(PP, B)                                                           \
+    if (a.p == PP && a.D2p == B) {                                               \
+        if (a.D1 > 0) heff_small_k<PP, B, true><<<grid, 1024, 0, s>>>(a);        \
+        else heff_small_k<PP, B, false><<<grid, 1024, 0, s>>>(a);                \
+        return hipGetLastError();                                                \
+    }
+    HS_CASE(2, 32) HS_CASE(2, 64) HS_CASE(3, 32) HS_CASE(3, 64) HS_CASE(4, 32) HS_CASE(4, 64)
+#undef HS_CASE
+    return hipErrorInvalidValue;
+}
+
 }  // namespace tn

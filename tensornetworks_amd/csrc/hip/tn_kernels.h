@@ -105,6 +105,21 @@ bool x3_stage1_mix_ok(int p, int nR, const MixTable& t, int D1p, int D2p);
 hipError_t x3_stage1_mix(int p, int nR, const bf16* X, long psX, const bf16* R, long psR, const double* x,
                          bf16* T2, long ps2, long ldo, double* y, int D1p, int D2p, const MixTable& t,
                          hipStream_t s);
+// The whole FP64 Heff apply of a small site (left bond padded to 32, right bond to
+// 32 or 64) in one launch: y = scale * H x.  R: the nR kept right channels [nR][D2p][D2p];
+// L: first kept left channel of [D1p][Dw1][D1p]; wl: identity channel of the
+// left side (0 or Dw1 - 1, -1 none), its slice mixed straight into y; t: the
+// MIX_HEFF_T table.  D1 > 0: x and y in the reference layout (D1 x D2 logical).
+struct HeffSmall {
+    int p, D1p, D2p, nR, nL, Dw1, wl;
+    const double *x, *L, *R;
+    double* y;
+    double scale;
+    int D1, D2;
+    MixTable t;
+};
+bool heff_small_ok(const HeffSmall& a);
+hipError_t heff_small(const HeffSmall& a, hipStream_t s);
 // The Heff mixing with a second input and a second output, its stage-3
 // operand written transposed: entries e with esel[e] read
 // in2[x*isx2 + eoff[e] + b] (type tx), outputs o with osel[o] write
@@ -179,6 +194,12 @@ hipError_t lz_dot(const double* v, const double* w, long n, double* part, hipStr
 hipError_t lz_step(const double* y, double* w, const double* V, long ldv, int k, bool three, double beta, long n,
                    double* h, double* part, hipStream_t s);
 hipError_t lz_update(double* w, const double* V, long ldv, int k, long n, double* coef, double* part, hipStream_t s);
+// the same step of a short vector in one launch: y = H v_j (v_j = V_{k-1}, scaled
+// by vscale first, in place, when that is not 1), the pass against V_0 .. V_{k-1}, w to V_k
+// (divided by |w| when unit), and (alpha, the k coefficients, |w|^2) to the host
+bool lz_small_ok(long n, int k);
+hipError_t lz_small(const double* y, double* V, long ldv, int k, double vscale, double beta, bool unit, long n,
+                    double* host_dst, unsigned long long* host_flag, unsigned long long seq, hipStream_t s);
 hipError_t lz_publish(const double* h, int nh, long n, const double* part, double* host_dst,
                       unsigned long long* host_flag, unsigned long long seq, hipStream_t s);
 // y = a x (y is not read; x and y may be the same buffer)

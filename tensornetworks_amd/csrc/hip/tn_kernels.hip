@@ -810,6 +810,145 @@ hipError_t lz_update(double* w, const double* V, long ldv, int k, long n, double
     return hipGetLastError();
 }
 
+// The whole step of a short vector in one workgroup: scales v_j = V_{k-1} by
+// vscale first when that is not 1 (in place), then alpha, the three-term step,
+// the pass against V_0 .. V_{k-1}, |w|^2, and the publication of (alpha,
+// coefficients, |w|^2).
+// w goes to V_k, divided by |w| when `unit`.  w stays in registers (PP pairs
+// per thread) and in LDS, where every wave takes whole vectors of the basis:
+// one lane reduction per vector instead of one per vector and wave.  Bound by
+// the one CU's reads of the basis (two passes), so it pays while that is small
+// (lz_small_ok).  n = 2048: 8.8 us at k = 1, 10.5 at 8, 15.6 at 30, 19.8 at 48; the
+// four launches take 14.3 us and three launch gaps of about 1.5 us at k ~ 28.
+// n = 12288 took 23 us at k = 2, more than the four launches.
+#define LZ_TINY_T 1024
+#define LZ_TINY_K 64
+#define LZ_TINY_N (6 * LZ_TINY_T)
+bool lz_small_ok(long n, int k) { return n > 0 && n % 128 == 0 && n <= LZ_TINY_N && k >= 1 && k <= LZ_TINY_K && n * k <= 65536; }
+
+template <int PP>
+__global__ void __launch_bounds__(LZ_TINY_T) lz_small_k(const double* __restrict__ y, double* __restrict__ V, long ldv,
+                                                        int k, double vscale, double beta, int unit, int n,
+                                                        double* host_dst, unsigned long long* host_flag,
+                                                        unsigned long long seq)
+{
+    constexpr int NW = LZ_TINY_T / 64;
+    __shared__ __attribute__((aligned(16))) double ws[2 * PP * LZ_TINY_T];
+    __shared__ double one[2][NW];
+    __shared__ double c[LZ_TINY_K];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    double* vj = V + (long)(k - 1) * ldv;
+    const double* vm = k >= 2 ? vj - ldv : vj;
+    const double b = k >= 2 ? beta : 0.0;
+    auto total = [&](double v, double* buf) {  // sum over the workgroup
+        v = wave_sum(v);
+        if (lane == 0) buf[wid] = v;
+        __syncthreads();
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < NW; q++) s += buf[q];
+        return s;
+    };
+    double2 x[PP], p[PP], q[PP];
+#pragma unroll
+    for (int e = 0; e < PP; e++) {
+        const int idx = 2 * (e * LZ_TINY_T + tid);
+        const bool in = idx < n;
+        x[e] = in ? *(const double2*)(y + idx) : make_double2(0.0, 0.0);
+        p[e] = in ? *(const double2*)(vj + idx) : make_double2(0.0, 0.0);
+        q[e] = in ? *(const double2*)(vm + idx) : make_double2(0.0, 0.0);
+    }
+    double dot = 0.0;
+#pragma unroll
+    for (int e = 0; e < PP; e++) {
+        const int idx = 2 * (e * LZ_TINY_T + tid);
+        if (vscale != 1.0) {
+            p[e].x *= vscale;
+            p[e].y *= vscale;
+            if (idx < n) *(double2*)(vj + idx) = p[e];
+        }
+        dot += x[e].x * p[e].x + x[e].y * p[e].y;
+    }
+    const double alpha = total(dot, one[0]);
+#pragma unroll
+    for (int e = 0; e < PP; e++) {
+        x[e].x -= alpha * p[e].x;
+        x[e].y -= alpha * p[e].y;
+        x[e].x -= b * q[e].x;
+        x[e].y -= b * q[e].y;
+        *(double2*)(ws + 2 * (e * LZ_TINY_T + tid)) = x[e];
+    }
+    __syncthreads();  // w in LDS; the scaled v_j is visible to every wave
+    for (int i = wid; i < k; i += NW) {
+        const double* vi = V + (long)i * ldv;
+        double s = 0.0;
+#pragma unroll 16
+        for (int e = 0; e < n / 128; e++) {
+            const int idx = 2 * (e * 64 + lane);
+            const double2 v = *(const double2*)(vi + idx), w = *(const double2*)(ws + idx);
+            s += v.x * w.x + v.y * w.y;
+        }
+        s = wave_sum(s);
+        if (lane == 0) {
+            c[i] = s;
+            host_dst[1 + i] = s;
+        }
+    }
+    __syncthreads();
+#pragma unroll 8
+    for (int i = 0; i < k; i++) {
+        const double* vi = V + (long)i * ldv;
+        const double ci = c[i];
+#pragma unroll
+        for (int e = 0; e < PP; e++) {
+            const int idx = 2 * (e * LZ_TINY_T + tid);
+            if (idx < n) {
+                const double2 v = *(const double2*)(vi + idx);
+                x[e].x -= ci * v.x;
+                x[e].y -= ci * v.y;
+            }
+        }
+    }
+    double sq = 0.0;
+#pragma unroll
+    for (int e = 0; e < PP; e++) sq += x[e].x * x[e].x + x[e].y * x[e].y;
+    const double nn = total(sq, one[1]);
+    const double f = unit ? 1.0 / sqrt(nn) : 1.0;  // infinite when the Krylov space is complete: w is not used then
+    double* w = vj + ldv;
+#pragma unroll
+    for (int e = 0; e < PP; e++) {
+        const int idx = 2 * (e * LZ_TINY_T + tid);
+        if (idx < n) *(double2*)(w + idx) = make_double2(f * x[e].x, f * x[e].y);
+    }
+    if (tid == 0) {
+        host_dst[0] = alpha;
+        host_dst[k + 1] = nn;
+    }
+    // the published values (each written by lane 0 of a wave) before the flag
+    __threadfence_system();
+    __syncthreads();
+    if (tid == 0) {
+        __threadfence_system();
+        *(volatile unsigned long long*)host_flag = seq;
+    }
+}
+
+hipError_t lz_small(const double* y, double* V, long ldv, int k, double vscale, double beta, bool unit, long n,
+                    double* host_dst, unsigned long long* host_flag, unsigned long long seq, hipStream_t s)
+{
+    if (!lz_small_ok(n, k)) return hipErrorInvalidValue;
+    const int pp = (int)((n + 2 * LZ_TINY_T - 1) / (2 * LZ_TINY_T));
+#define LZ_CASE(P)                                                                                             \
+    if (pp <= P) {                                                                                             \
+        lz_small_k<P><<<1, LZ_TINY_T, 0, s>>>(y, V, ldv, k, vscale, beta, unit, (int)n, host_dst, host_flag,   \
+                                              seq);                                                            \
+        return hipGetLastError();                                                                              \
+    }
+    LZ_CASE(1) LZ_CASE(2) LZ_CASE(3)
+#undef LZ_CASE
+    return hipErrorInvalidValue;
+}
+
 // h[0..nh) and then sum npart[0..G) (|w|^2) to the host, as publish does
 __global__ void __launch_bounds__(MD_BLOCK) lz_publish_k(const double* __restrict__ h, int nh,
                                                          const double* __restrict__ npart, int G, double* host_dst,
