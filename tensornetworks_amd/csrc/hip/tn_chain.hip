@@ -502,7 +502,7 @@ void svd_normalize(tn_chain* ch, int i, int dir, tn_sweep_stats* st, int gauge =
         std::vector<double> sv_pad(kp, 0.0);
         normalised_copy(sv, sv_pad);
         c->pack.ensure(kp * 8 + 64);
-        h2d(c, c->pack.p, sv_pad.data(), kp * 8);
+        h2d_small(c, c->pack.p, sv_pad.data(), kp * 8);
         TN_HIP(scale_rows(c->svd_Vt.as<double>(), D2p, kp, D2p, c->pack.as<double>(), s));
         GemmDesc g{};
         g.tin = T_F64; g.tout = T_F64; g.a_kmajor = true; g.b_kmajor = false;
@@ -531,7 +531,7 @@ void svd_normalize(tn_chain* ch, int i, int dir, tn_sweep_stats* st, int gauge =
         std::vector<double> sv_pad(kp, 0.0);
         normalised_copy(sv, sv_pad);
         c->pack.ensure(kp * 8 + 64);
-        h2d(c, c->pack.p, sv_pad.data(), kp * 8);
+        h2d_small(c, c->pack.p, sv_pad.data(), kp * 8);
         TN_HIP(scale_cols(c->svd_U.as<double>(), kp, D1p, kp, c->pack.as<double>(), s));
         GemmDesc g{};
         g.tin = T_F64; g.tout = T_F64; g.a_kmajor = true; g.b_kmajor = false;
@@ -773,7 +773,7 @@ int tn_ctx_destroy(tn_ctx* c)
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     tn::DBuf* bufs[] = {&c->T1, &c->T2, &c->xlo, &c->part, &c->krylov, &c->lanczos_small, &c->svd_X,
-                        &c->svd_V, &c->svd_U, &c->svd_Vt, &c->svd_s, &c->svd_perm, &c->svd_pairs,
+                        &c->svd_V, &c->svd_U, &c->svd_Vt, &c->svd_s, &c->svd_perm,
                         &c->svd_flag, &c->svd_A, &c->spare, &c->pack, &c->qr_W, &c->qr_G, &c->qr_L,
                         &c->qr_T, &c->qr_linv, &c->qr_Q, &c->tune_C, &c->splitk, &c->b_L, &c->b_R,
                         &c->b_Llo, &c->b_Rlo, &c->b_x, &c->b_y, &c->b_M, &c->dav_W, &c->dav_vec,
@@ -1979,7 +1979,7 @@ int tn_chain_sweep2(tn_chain* ch, int dir, int Dmax, double eps_sv, const tn_swe
         std::vector<double> scl(std::max(Dkp, 32), 0.0);
         for (int t = 0; t < Dk; t++) scl[t] = sk[t] / nr;
         c->pack.ensure((size_t)scl.size() * 8 + 64);
-        h2d(c, c->pack.p, scl.data(), scl.size() * 8);
+        h2d_small(c, c->pack.p, scl.data(), scl.size() * 8);
         if (dir == 0) {
             // A_i <- U[:, :Dk] ; A_j <- diag(s) Vt[:Dk]
             TN_HIP(copy2(c->svd_U.as<double>(), kp, 1, rr, Dk, ch->A[i], Dkp, 1, D1p * d, Dkp, s));

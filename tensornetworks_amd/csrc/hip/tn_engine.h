@@ -85,7 +85,7 @@ struct tn_ctx {
     std::string err;
     // scratch
     tn::DBuf T1, T2, xlo, part, krylov, lanczos_small, svd_X, svd_V, svd_U, svd_Vt, svd_s,
-        svd_perm, svd_pairs, svd_flag, svd_A, spare, pack, qr_W, qr_G, qr_L, qr_T, qr_linv, qr_Q;
+        svd_perm, svd_flag, svd_A, spare, pack, qr_W, qr_G, qr_L, qr_T, qr_linv, qr_Q;
     // preconditioned SVD: R, Q_h, reflectors (then Q_h J), T factors + GEMM work space
     tn::DBuf svd_R, svd_Q, svd_H, svd_W, svd_X2;
     tn::Scalars sc;
@@ -276,6 +276,13 @@ void d2h(tn_ctx* c, void* dst, const void* src, size_t bytes);
 // n (<= TN_PUBLISH_MAX) doubles device -> host through the published scalars
 // (no stream synchronisation: the host polls the completion flag)
 void d2h_small(tn_ctx* c, double* dst, const double* src, int n);
+// the same for any n (a copy and a wait above TN_PUBLISH_MAX) and for one int in
+// a buffer of at least 8 bytes
+void d2h_vec(tn_ctx* c, double* dst, const double* src, long n);
+int d2h_int(tn_ctx* c, const int* src);
+// host -> device within stream order, without waiting for it (src is copied before
+// the call returns); bytes % 4 == 0
+void h2d_small(tn_ctx* c, void* dst, const void* src, size_t bytes);
 // the n values a kernel published with sequence number seq (polls its flag)
 void read_published(tn_ctx* c, double* dst, int n, unsigned long long seq);
 

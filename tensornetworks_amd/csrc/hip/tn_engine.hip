@@ -71,6 +71,27 @@ void read_published(tn_ctx* c, double* dst, int n, unsigned long long seq)
     for (int i = 0; i < n; i++) dst[i] = ((volatile double*)c->sc.h)[i];
 }
 
+void d2h_vec(tn_ctx* c, double* dst, const double* src, long n)
+{
+    if (n <= TN_PUBLISH_MAX) d2h_small(c, dst, src, (int)n);
+    else d2h(c, dst, src, (size_t)n * 8);
+}
+
+int d2h_int(tn_ctx* c, const int* src)
+{
+    double w;
+    d2h_small(c, &w, (const double*)src, 1);
+    int v;
+    std::memcpy(&v, &w, sizeof(v));
+    return v;
+}
+
+void h2d_small(tn_ctx* c, void* dst, const void* src, size_t bytes)
+{
+    if (bytes <= 4096) TN_HIP(upload(dst, src, (long)bytes, c->stream));
+    else h2d(c, dst, src, bytes);
+}
+
 void d2h(tn_ctx* c, void* dst, const void* src, size_t bytes)
 {
     TN_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
@@ -995,7 +1016,7 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
             }
         }
         // Ritz vector x = sum_i z_i v_i, normalised
-        h2d(c, zd, z.data(), (size_t)k * 8);
+        h2d_small(c, zd, z.data(), (size_t)k * 8);
         TN_HIP(gemv_acc(V, N, k, zd, 1.0, 0.0, x, N, s));
         const double nr = norm_host(x);
         TN_HIP(scale_copy(1.0 / nr, x, x, N, s));
@@ -1089,8 +1110,8 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
     c->svd_V.ensure((size_t)qp * qp * 8);
     double* V = c->svd_V.as<double>();
     c->svd_s.ensure((size_t)(qp + 64) * 8 * 2 + 1024 * 8);
-    double* amax_d = c->svd_s.as<double>() + 2 * qp + 128;
     double* nd = c->svd_s.as<double>();
+    double* amax_d = nd + q;  // read together with the q norms or cosines before it
     c->part.ensure(1024 * 8);
     double amax = 0.0;
     // X0 (column j of X0 at B + j*ldb), scaled to max |entry| = 1 (Gram
@@ -1099,9 +1120,12 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
         if (tall) TN_HIP(copy2(A, cs, rs, q, p, B, ldb, 1, qp, rows_out, s));
         else TN_HIP(copy2(A, rs, cs, q, p, B, ldb, 1, qp, rows_out, s));
         TN_HIP(absmax(B, ldb * qp, amax_d, c->part.as<double>(), 1024, s));
-        d2h(c, &amax, amax_d, 8);
-        if (!std::isfinite(amax)) throw TnError{TN_ERR_STATE, "svd: non-finite matrix entries"};
-        if (amax > 0.0) TN_HIP(scale_by_inv(B, amax_d, ldb * qp, s));
+        TN_HIP(scale_by_inv(B, amax_d, ldb * qp, s, true));
+    };
+    // called before anything of the caller's is written
+    auto check_amax = [&](double a) {
+        if (!std::isfinite(a)) throw TnError{TN_ERR_STATE, "svd: non-finite matrix entries"};
+        amax = a;
     };
     // the Jacobi iterate X (pj rows, column j at X + j*ldx)
     double* X = nullptr;
@@ -1127,9 +1151,10 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
         g.A = Hb; g.lda = pp; g.B = Hb; g.ldb = pp; g.C = R; g.ldc = qp;
         TN_HIP(gemm(g, s));
         TN_HIP(max_cos(R, qp, q, nd, s));
-        std::vector<double> mc(q);
-        d2h(c, mc.data(), nd, (size_t)q * 8);
-        const double cmax = *std::max_element(mc.begin(), mc.end());
+        std::vector<double> mc(q + 1);
+        d2h_vec(c, mc.data(), nd, q + 1);
+        check_amax(mc[q]);
+        const double cmax = *std::max_element(mc.begin(), mc.begin() + q);
         pre = !(cmax < kSvdPlainCos);
         if (getenv("TN_SVD_TRACE")) fprintf(stderr, "# svdcos q=%d cmax=%.3e pre=%d\n", q, cmax, (int)pre);
         if (pre) {
@@ -1149,11 +1174,11 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
             // iteration)
             TN_HIP(col_norms(Hb, pp, p, q, nd, s));
             std::vector<double> cn(q);
-            d2h(c, cn.data(), nd, (size_t)q * 8);
+            d2h_vec(c, cn.data(), nd, q);
             std::vector<int> piv(qp);
             std::iota(piv.begin(), piv.end(), 0);
             std::stable_sort(piv.begin(), piv.begin() + q, [&](int a, int b) { return cn[a] > cn[b]; });
-            h2d(c, dpiv, piv.data(), (size_t)qp * sizeof(int));
+            h2d_small(c, dpiv, piv.data(), (size_t)qp * sizeof(int));
             TN_HIP(gather_cols(Hb, pp, R, pp, dpiv, pp, qp, s));
             house_qr(c, R, pp, qp, Qh, Hb, W + (size_t)2 * qp * 32, W, W + (size_t)qp * 32);
             // X0 P = Q_h R, so X0 = Q_h (P R^T)^T: X = P R^T,
@@ -1170,21 +1195,11 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
         load_scaled(X, ldx, p);
     }
     TN_HIP(set_identity(V, qp, qp, s));
-    // tournament pairs for nb = qp/16 column blocks
-    const int nb = qp / 16;
-    std::vector<int> pairs((size_t)(nb - 1) * nb);
-    for (int rd = 0; rd < nb - 1; rd++)
-        for (int i = 0; i < nb / 2; i++) {
-            auto elem = [&](int kp) { return kp == 0 ? 0 : ((kp - 1 + rd) % (nb - 1)) + 1; };
-            pairs[(size_t)rd * nb + 2 * i] = elem(i);
-            pairs[(size_t)rd * nb + 2 * i + 1] = elem(nb - 1 - i);
-        }
-    c->svd_pairs.ensure(pairs.size() * sizeof(int) + 64);
-    h2d(c, c->svd_pairs.p, pairs.data(), pairs.size() * sizeof(int));
+    const int nb = qp / 16;  // column blocks
     c->svd_flag.ensure(256);
     int* flag = c->svd_flag.as<int>();
     const double tol = std::max(1e-15, 4.4e-16 * std::sqrt((double)pj));
-    int hflag = 1;
+    const int max_sweeps = 80;
     // (each visit gives a pair's Gram matrix one sweep of rotations: the pairs
     // come back every outer sweep, and a round has only nb/2 pairs, so its
     // latency sets the cost.  On the 512 x 512 two-site splits at D=256 that
@@ -1194,25 +1209,29 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
     // least 32 rows each); the iterate alternates between X and X2
     const int nchunk = std::max(1, std::min({16, 256 / std::max(1, nb / 2), std::max(1, pj / 32)}));
     c->svd_X2.ensure((size_t)ldx * qp * 8);
-    double* Xa = X;
-    double* Xb = c->svd_X2.as<double>();
-    for (int sweep = 0; sweep < 80 && hflag; sweep++) {
+    // q >= 128 takes the rotations from reciprocal square roots; fewer columns keep
+    // the divisions, whose results callers have bit for bit
+    if (jacobi_all_ok(pj, qp)) {
+        TN_HIP(jacobi_all(X, c->svd_X2.as<double>(), ldx, pj, V, qp, qp, tol, max_sweeps, s));
+    } else {
+        double* Xa = X;
+        double* Xb = c->svd_X2.as<double>();
         TN_HIP(set_int(flag, 0, s));
-        for (int rd = 0; rd < nb - 1; rd++) {
-            TN_HIP(jacobi_step(Xa, Xb, ldx, pj, V, qp, qp, c->svd_pairs.as<int>() + (size_t)rd * nb, nb / 2,
-                               nchunk, tol, flag, s));
-            std::swap(Xa, Xb);
+        for (int sweep = 1; sweep <= max_sweeps; sweep++) {
+            for (int rd = 0; rd < nb - 1; rd++) {
+                TN_HIP(jacobi_step(Xa, Xb, ldx, pj, V, qp, qp, nb, rd, nchunk, tol, flag, sweep, big, s));
+                std::swap(Xa, Xb);
+            }
+            if (d2h_int(c, flag) != sweep) break;  // no pair rotated
         }
-        TN_HIP(hipMemcpyAsync(&hflag, flag, sizeof(int), hipMemcpyDeviceToHost, s));
-        sync(c);
+        X = Xa;
     }
-    X = Xa;
     // singular values = column norms; sort descending
     double* sd = c->svd_s.as<double>();
     TN_HIP(col_norms(X, ldx, pj, q, sd, s));
-    std::vector<double> sv(q);
-    TN_HIP(hipMemcpyAsync(sv.data(), sd, q * 8, hipMemcpyDeviceToHost, s));
-    sync(c);
+    std::vector<double> sv(q + 1);
+    d2h_vec(c, sv.data(), sd, q + 1);
+    check_amax(sv[q]);
     std::vector<int> perm(q);
     std::iota(perm.begin(), perm.end(), 0);
     std::stable_sort(perm.begin(), perm.end(), [&](int a, int b) { return sv[a] > sv[b]; });
@@ -1227,7 +1246,7 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
     }
     // normalise the good columns of X
     double* dinv = sd + qp + 32;
-    h2d(c, dinv, inv.data(), qp * 8);
+    h2d_small(c, dinv, inv.data(), qp * 8);
     TN_HIP(scale_rows(X, ldx, q, pj, dinv, s));
     // orthonormal completion of (exactly) zero columns, in the sorted order,
     // within the first pc rows (pre: the right factor lives in q dimensions;
@@ -1272,13 +1291,9 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
     // gather into U / Vt (zero padded first)
     if (zr > 0) TN_HIP(fill_zero(U, (long)zr * ldu * 8, s));
     if (zk > 0) TN_HIP(fill_zero(Vt, (long)zk * ldvt * 8, s));
-    int* dperm = (int*)(sd + 2 * qp + 64);
-    c->svd_perm.ensure((size_t)(q + 64) * 12);
-    dperm = c->svd_perm.as<int>();
-    double* ones = (double*)(dperm + ((q + 63) / 64) * 64);
-    std::vector<double> onev(k, 1.0);
-    h2d(c, dperm, perm.data(), k * sizeof(int));
-    h2d(c, ones, onev.data(), k * 8);
+    c->svd_perm.ensure((size_t)q * sizeof(int));
+    int* dperm = c->svd_perm.as<int>();
+    h2d_small(c, dperm, perm.data(), k * sizeof(int));
     // the factor with p-long columns (L, ld ldl) and the one with q-long
     // columns (Rt, ld qp): plain X and J, preconditioned Q_h J and X
     const double* Lf = X;
@@ -1319,14 +1334,13 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
     }
     if (tall) {
         // U (r x k) from the p-side factor, Vt (k x c) from the q-side one
-        TN_HIP(svd_gather(Lf, ldl, p, Rf, qp, q, dperm, ones, k, U, ldu, 1, Vt, ldvt, 1, s));
+        TN_HIP(svd_gather(Lf, ldl, p, Rf, qp, q, dperm, k, U, ldu, 1, Vt, ldvt, 1, s));
     } else {
         // Vt (k x c) from the p-side factor (columns of length c), U (r x k) from the q-side one
-        TN_HIP(svd_gather(Lf, ldl, p, Rf, qp, q, dperm, ones, k, Vt, 1, ldvt, U, 1, ldu, s));
+        TN_HIP(svd_gather(Lf, ldl, p, Rf, qp, q, dperm, k, Vt, 1, ldvt, U, 1, ldu, s));
     }
     s_out.resize(k);
     for (int j = 0; j < k; j++) s_out[j] = sv[perm[j]] * (amax > 0.0 ? amax : 1.0);
-    sync(c);
     return k;
 }
 
@@ -1529,14 +1543,11 @@ bool cholqr_device(tn_ctx* c, const double* A, long lda, int m, int n, int nl, d
         double* Lp = pass == 1 ? Lacc : Lk;
         TN_HIP(set_int(flag, 0, s));
         qr_factor(c, G, n, nl, 0.0, Lp, Linv, flag);
-        int hflag = 0;
-        d2h(c, &hflag, flag, sizeof(int));
-        if (hflag) {
+        if (d2h_int(c, flag)) {
             TN_HIP(set_int(flag, 0, s));
             qr_gram(c, X, ldx, m, n, G);
             qr_factor(c, G, n, nl, shift, Lp, Linv, flag);
-            d2h(c, &hflag, flag, sizeof(int));
-            if (hflag) return false;
+            if (d2h_int(c, flag)) return false;
             if (shifted) *shifted = 1;
         }
         double* Y = X == Q1 ? Q : Q1;

@@ -143,6 +143,10 @@ hipError_t wmix_idt(int tin, int tx, int tout, const void* in, long isx, const v
 hipError_t publish(const double* src, int n, double* host_dst, unsigned long long* host_flag,
                    unsigned long long seq, hipStream_t s);
 
+// Small host -> device transfer in the arguments of a launch (2 KB each): src is
+// copied before the call returns.  bytes % 4 == 0.
+hipError_t upload(void* dst, const void* src, long bytes, hipStream_t s);
+
 // elementwise
 hipError_t convert(int tin, const void* in, int tout, void* out, long n, hipStream_t s);
 // three bfloat16 planes of n values (T_F64 or T_F32 input): out[p*ps + i], p = 0..2
@@ -179,7 +183,7 @@ hipError_t gemv_acc(const double* V, long ldv, int k, const double* coef, double
 // out[0] = max_i |x[i]|  (part: >= 1024 doubles of scratch)
 hipError_t absmax(const double* x, long n, double* out, double* part, int part_cap, hipStream_t s);
 // v[n] *= 1/den[0] (den on device)
-hipError_t scale_by_inv(double* v, const double* den, long n, hipStream_t s);
+hipError_t scale_by_inv(double* v, const double* den, long n, hipStream_t s, bool keep_zero = false);
 hipError_t axpby(double a, const double* x, double b, double* y, long n, hipStream_t s);
 // Fused Lanczos step (n even, vectors 16-byte aligned, k <= 512), in this order
 // on one stream, part: lz_part_size(n, k) doubles of scratch, h: k + 1 doubles:
@@ -211,12 +215,18 @@ hipError_t dcopy_scalar(const double* src, double* dst, hipStream_t s);
 hipError_t dsqrt_scalar(const double* src, double* dst, hipStream_t s);
 
 // one-sided block Jacobi SVD round (fp64, column-major iterate with ldx,
-// q%32==0): the round's pairs rotate Xs into Xd (every column of the round's
-// pairs written, rotated or copied; Xs != Xd) and V in place, nchunk
-// workgroups per pair, each its own chunk of rows; each pair's 32 x 32 Gram
-// matrix gets one sweep of rotations
-hipError_t jacobi_step(const double* Xs, double* Xd, long ldx, int p, double* V, long ldv, int qv,
-                       const int* pairs, int npairs, int nchunk, double tol, int* flag, hipStream_t s);
+// q%32==0): round rd of the tournament of the nb = q/16 column blocks rotates Xs
+// into Xd (every column written, rotated or copied; Xs != Xd) and V in place,
+// nchunk workgroups per pair, each its own chunk of rows; each pair's 32 x 32
+// Gram matrix gets one sweep of rotations.  flag[0] = tag when a pair was not
+// orthogonal.  fast: rotations from reciprocal square roots (see jacobi_rot).
+hipError_t jacobi_step(const double* Xs, double* Xd, long ldx, int p, double* V, long ldv, int qv, int nb, int rd,
+                       int nchunk, double tol, int* flag, int tag, bool fast, hipStream_t s);
+// the whole iteration of q = 32 columns (one pair), at most max_sweeps visits:
+// X <- X J, V <- V J, X2 scratch of X's size
+bool jacobi_all_ok(int p, int qv);
+hipError_t jacobi_all(double* X, double* X2, long ldx, int p, double* V, long ldv, int qv, double tol, int max_sweeps,
+                      hipStream_t s);
 // Householder QR of the 32-column panel c0..c0+31 of the column-major A (pp
 // rows, ld lda), in place: R on and above the diagonal, zeros below; the
 // vectors in columns 0..31 of V (rows c0..pp-1, ld ldv) and the 32 x 32
@@ -233,10 +243,10 @@ hipError_t tr_scatter(const double* R, long ldr, double* X, long ldx, const int*
 hipError_t col_norms(const double* X, long ldx, int p, int q, double* s, hipStream_t st);
 hipError_t set_int(int* p, int v, hipStream_t s);
 hipError_t set_identity(double* V, long ldv, int n, hipStream_t s);
-// out1[i*s10 + j*s11] = X[perm[j]*ldx + i] * scl[j]   (i < p, j < k)
-// out2[j*s20 + i*s21] = V[perm[j]*ldv + i]            (i < q, j < k)
+// out1[i*s10 + j*s11] = X[perm[j]*ldx + i]   (i < p, j < k)
+// out2[j*s20 + i*s21] = V[perm[j]*ldv + i]   (i < q, j < k)
 hipError_t svd_gather(const double* X, long ldx, int p, const double* V, long ldv, int q,
-                      const int* perm, const double* scl, int k, double* out1, long s10, long s11,
+                      const int* perm, int k, double* out1, long s10, long s11,
                       double* out2, long s20, long s21, hipStream_t s);
 // unit vector e_pos in column j of X (length p)
 hipError_t set_unit_col(double* x, int p, int pos, hipStream_t s);

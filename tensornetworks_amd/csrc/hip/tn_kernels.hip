@@ -6,6 +6,9 @@
 // * jacobi_k   : one block pair of a one-sided block-Jacobi SVD (fp64).
 #include "tn_device.h"
 
+#include <algorithm>
+#include <cstring>
+
 namespace tn {
 
 // ---------------------------------------------------------------------------
@@ -236,6 +239,30 @@ hipError_t publish(const double* src, int n, double* host_dst, unsigned long lon
     if (n < 0 || n > TN_PUBLISH_MAX) return hipErrorInvalidValue;
     publish_k<<<1, 256, 0, s>>>(src, n, host_dst, host_flag, seq);
     return hipGetLastError();
+}
+
+// Words carried in the kernel's arguments: they are copied when the launch is
+// queued, so nothing has to wait for the stream (a pageable copy of 256 bytes
+// and the wait for it take about 20 us, this launch about 5).
+struct Words {
+    unsigned w[512];
+};
+__global__ void __launch_bounds__(256) upload_k(unsigned* __restrict__ dst, Words a, int n)
+{
+    for (int t = threadIdx.x; t < n; t += 256) dst[t] = a.w[t];
+}
+hipError_t upload(void* dst, const void* src, long bytes, hipStream_t s)
+{
+    if (bytes % 4 != 0) return hipErrorInvalidValue;
+    Words a;
+    for (long off = 0; off < bytes; off += (long)sizeof(a)) {
+        const int n = (int)std::min((long)sizeof(a), bytes - off);
+        memcpy(a.w, (const char*)src + off, n);
+        upload_k<<<1, 256, 0, s>>>((unsigned*)((char*)dst + off), a, n / 4);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 // ---------------------------------------------------------------------------
@@ -1043,16 +1070,16 @@ hipError_t absmax(const double* x, long n, double* out, double* part, int part_c
     return hipGetLastError();
 }
 
-__global__ void scale_by_inv_k(double* v, const double* den, long n)
+__global__ void scale_by_inv_k(double* v, const double* den, long n, bool keep_zero)
 {
-    const double f = 1.0 / den[0];
+    const double f = keep_zero && den[0] == 0.0 ? 1.0 : 1.0 / den[0];
     for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256) v[i] *= f;
 }
-hipError_t scale_by_inv(double* v, const double* den, long n, hipStream_t s)
+hipError_t scale_by_inv(double* v, const double* den, long n, hipStream_t s, bool keep_zero)
 {
     long blocks = (n + 255) / 256;
     if (blocks > 8192) blocks = 8192;
-    scale_by_inv_k<<<blocks, 256, 0, s>>>(v, den, n);
+    scale_by_inv_k<<<blocks, 256, 0, s>>>(v, den, n, keep_zero);
     return hipGetLastError();
 }
 __global__ void axpby_k(double a, const double* x, double b, double* y, long n)
@@ -1116,15 +1143,41 @@ hipError_t dsqrt_scalar(const double* src, double* dst, hipStream_t s)
 // rotations themselves from the previous round's G (two buffers) instead of
 // waiting for 16 threads to publish them.  Measured per launch, that form (with
 // one thread per row in step 3) and this one: 45 and 31 us at p = q = 32, 50 and
-// 34 us at 192, 53 and 41 us at 512.
+// 34 us at 192, 53 and 41 us at 512; with FAST rotations 25, 29 and 34 us.
 #define JB 16
 #define JW 32
 #define JR 128  // rows per Gram chunk
 
 // the rotation that annihilates apq of [app apq; apq aqq] (no branch: the
-// discarded values of a skipped rotation may be infinite)
+// discarded values of a skipped rotation may be infinite).  FAST forms c and s
+// from two reciprocal square roots instead of three divisions and two square
+// roots: with d = aqq - app, o = 2 apq (scaled by a power of two so that the
+// squares neither overflow nor vanish) and h = 1 / sqrt(d^2 + o^2),
+// c^2 = (1 + |d| h) / 2, s = sign(d) o h / (2 c).
+__device__ __forceinline__ double rsqrt_newton(double a)
+{
+    const double y = __builtin_amdgcn_rsq(a);  // to 2^-23
+    const double e = fma(-a * y, y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+template <bool FAST>
 __device__ __forceinline__ void jacobi_rot(double app, double aqq, double apq, double& c, double& s)
 {
+    if (FAST) {
+        const double w = fabs(app * aqq);
+        const bool rot = fabs(apq) > 1e-300 && !(fabs(apq) <= 1e-16 * (w * __builtin_amdgcn_rsq(w)));
+        double d = aqq - app, o = 2.0 * apq;
+        const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(d), fabs(o)));
+        d = __builtin_ldexp(d, ex);
+        o = __builtin_ldexp(o, ex);
+        const double h = rsqrt_newton(fma(d, d, o * o));
+        const double c2 = fma(0.5 * fabs(d), h, 0.5);
+        const double ic = rsqrt_newton(c2);
+        c = rot ? c2 * ic : 1.0;
+        s = rot ? copysign(0.5, d) * o * h * ic : 0.0;
+        return;
+    }
     const bool rot = fabs(apq) > 1e-300 && fabs(apq) > 1e-16 * sqrt(fabs(app * aqq));
     const double theta = (aqq - app) / (2.0 * apq);
     const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
@@ -1133,20 +1186,20 @@ __device__ __forceinline__ void jacobi_rot(double app, double aqq, double apq, d
     s = rot ? t * cr : 0.0;
 }
 
-__global__ void __launch_bounds__(256) jacobi_k(const double* __restrict__ Xs, double* __restrict__ Xd, long ldx,
-                                                int p, double* __restrict__ V, long ldv, int qv,
-                                                const int* __restrict__ pairs, double tol, int* __restrict__ flag)
+// One visit of a pair; false when it was orthogonal already (rows copied to Xd
+// unless COPY is off).
+template <bool FAST, bool COPY>
+__device__ __forceinline__ bool jacobi_pair(const double* Xs, double* Xd, long ldx, int p, double* V, long ldv, int qv,
+                                            int pb, int qb, double tol, int ch, int nch)
 {
     __shared__ double G[2][JW][JW + 1];
     __shared__ __align__(16) double J[JW][JW + 2];  // even stride: column pairs are 16-byte aligned
     __shared__ double tile[JW][JR + 1];
     __shared__ int sh_off;
     const int tid = threadIdx.x;
-    const int pb = pairs[2 * blockIdx.x], qb = pairs[2 * blockIdx.x + 1];
     auto colidx = [&](int j) { return j < JB ? pb * JB + j : qb * JB + (j - JB); };
     // this workgroup's rows of the iterate and of V, 32 at a time: thread = row
     // ar of the 32 and columns 4 ac .. 4 ac + 3 of the product
-    const int nch = gridDim.y, ch = blockIdx.y;
     const int xrows = (p + nch - 1) / nch, vrows = (qv + nch - 1) / nch;
     const int xr0 = ch * xrows, xr1 = min(p, xr0 + xrows);
     const int vr0 = ch * vrows, vr1 = min(qv, vr0 + vrows);
@@ -1216,13 +1269,12 @@ __global__ void __launch_bounds__(256) jacobi_k(const double* __restrict__ Xs, d
     }
     __syncthreads();
     if (sh_off == 0) {  // already orthogonal: nothing to rotate
-        for (int e = tid; e < JW * (xr1 > xr0 ? xr1 - xr0 : 0); e += 256) {
+        for (int e = tid; COPY && e < JW * (xr1 > xr0 ? xr1 - xr0 : 0); e += 256) {
             const long off = (long)colidx(e / (xr1 - xr0)) * ldx + xr0 + e % (xr1 - xr0);
             Xd[off] = Xs[off];
         }
-        return;
+        return false;
     }
-    if (tid == 0) flag[0] = 1;
 
     // 2. one sweep of cyclic parallel Jacobi on G (tournament ordering, 31
     // rounds).  The round's pairs are disjoint, so G <- R^T G R splits into
@@ -1246,7 +1298,7 @@ __global__ void __launch_bounds__(256) jacobi_k(const double* __restrict__ Xs, d
         // lanes bj of every 16 hold the rotation of pair bj; that of pair bi
         // comes from lane bi
         double c2, s2;
-        jacobi_rot(p2, q2, o2, c2, s2);
+        jacobi_rot<FAST>(p2, q2, o2, c2, s2);
         const double c1 = __shfl(c2, bi, 64), s1 = __shfl(s2, bi, 64);
         const double h00 = c1 * g00 - s1 * g10, h01 = c1 * g01 - s1 * g11;
         const double h10 = s1 * g00 + c1 * g10, h11 = s1 * g01 + c1 * g11;
@@ -1301,14 +1353,65 @@ __global__ void __launch_bounds__(256) jacobi_k(const double* __restrict__ Xs, d
             for (int u = 0; u < 4; u++) V[(long)colidx(4 * ac + u) * ldv + row] = y[u];
         }
     }
+    return true;
 }
 
-hipError_t jacobi_step(const double* Xs, double* Xd, long ldx, int p, double* V, long ldv, int qv,
-                       const int* pairs, int npairs, int nchunk, double tol, int* flag, hipStream_t s)
+// Round rd of the tournament of nb column blocks: gridDim.x = nb / 2 pairs,
+// gridDim.y workgroups each.  flag[0] = tag when a pair rotated.
+template <bool FAST>
+__global__ void __launch_bounds__(256) jacobi_k(const double* __restrict__ Xs, double* __restrict__ Xd, long ldx, int p,
+                                                double* __restrict__ V, long ldv, int qv, int nb, int rd, double tol,
+                                                int* __restrict__ flag, int tag)
 {
-    if (npairs <= 0) return hipSuccess;
-    if (nchunk < 1 || nchunk > 64 || Xs == Xd) return hipErrorInvalidValue;
-    jacobi_k<<<dim3(npairs, nchunk), 256, 0, s>>>(Xs, Xd, ldx, p, V, ldv, qv, pairs, tol, flag);
+    auto elem = [&](int kp) { return kp == 0 ? 0 : (kp - 1 + rd) % (nb - 1) + 1; };
+    const int i = blockIdx.x;
+    if (jacobi_pair<FAST, true>(Xs, Xd, ldx, p, V, ldv, qv, elem(i), elem(nb - 1 - i), tol, blockIdx.y, gridDim.y) &&
+        threadIdx.x == 0)
+        flag[0] = tag;
+}
+
+// The whole iteration of two column blocks (one pair, so no round depends on
+// another workgroup): sweeps until the pair is orthogonal, at most max_sweeps.
+// The result is in X.  A sweep of this kernel costs what a launch of jacobi_k
+// does (about 30 us at p = q = 32), without the launch, the flag's clearing and
+// the host's look at it that followed each (about 30 us more); one workgroup
+// takes every row, so the rule keeps to p <= 256, where the rows are a small
+// part of the rotations' time.
+__global__ void __launch_bounds__(256) jacobi_all_k(double* X, double* X2, long ldx, int p, double* V, long ldv, int qv,
+                                                    double tol, int max_sweeps)
+{
+    double *a = X, *b = X2;
+    for (int sweep = 0; sweep < max_sweeps; sweep++) {
+        if (!jacobi_pair<false, false>(a, b, ldx, p, V, ldv, qv, 0, 1, tol, 0, 1)) break;
+        double* t = a;
+        a = b;
+        b = t;
+        __syncthreads();  // the rotated rows, before the next Gram matrix reads them
+    }
+    if (a != X)
+        for (int e = threadIdx.x; e < JW * p; e += 256) {
+            const long off = (long)(e / p) * ldx + e % p;
+            X[off] = a[off];
+        }
+}
+
+bool jacobi_all_ok(int p, int qv) { return qv == JW && p > 0 && p <= 256; }
+hipError_t jacobi_all(double* X, double* X2, long ldx, int p, double* V, long ldv, int qv, double tol, int max_sweeps,
+                      hipStream_t s)
+{
+    if (!jacobi_all_ok(p, qv) || X == X2) return hipErrorInvalidValue;
+    jacobi_all_k<<<1, 256, 0, s>>>(X, X2, ldx, p, V, ldv, qv, tol, max_sweeps);
+    return hipGetLastError();
+}
+
+hipError_t jacobi_step(const double* Xs, double* Xd, long ldx, int p, double* V, long ldv, int qv, int nb, int rd,
+                       int nchunk, double tol, int* flag, int tag, bool fast, hipStream_t s)
+{
+    if (nb < 2) return hipSuccess;
+    if (nb % 2 != 0 || rd < 0 || rd >= nb - 1 || nchunk < 1 || nchunk > 64 || Xs == Xd) return hipErrorInvalidValue;
+    const dim3 grid(nb / 2, nchunk);
+    if (fast) jacobi_k<true><<<grid, 256, 0, s>>>(Xs, Xd, ldx, p, V, ldv, qv, nb, rd, tol, flag, tag);
+    else jacobi_k<false><<<grid, 256, 0, s>>>(Xs, Xd, ldx, p, V, ldv, qv, nb, rd, tol, flag, tag);
     return hipGetLastError();
 }
 
@@ -1562,13 +1665,12 @@ hipError_t set_identity(double* V, long ldv, int n, hipStream_t s)
 }
 
 __global__ void svd_gather1_k(const double* __restrict__ X, long ldx, int p,
-                              const int* __restrict__ perm, const double* __restrict__ scl,
-                              double* __restrict__ out, long s0, long s1)
+                              const int* __restrict__ perm, double* __restrict__ out, long s0, long s1)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
     const int j = blockIdx.y;
     if (i >= p) return;
-    out[(long)i * s0 + (long)j * s1] = X[(long)perm[j] * ldx + i] * scl[j];
+    out[(long)i * s0 + (long)j * s1] = X[(long)perm[j] * ldx + i];
 }
 __global__ void svd_gather2_k(const double* __restrict__ V, long ldv, int q,
                               const int* __restrict__ perm, double* __restrict__ out, long s0,
@@ -1580,12 +1682,12 @@ __global__ void svd_gather2_k(const double* __restrict__ V, long ldv, int q,
     out[(long)j * s0 + (long)i * s1] = V[(long)perm[j] * ldv + i];
 }
 hipError_t svd_gather(const double* X, long ldx, int p, const double* V, long ldv, int q,
-                      const int* perm, const double* scl, int k, double* out1, long s10, long s11,
+                      const int* perm, int k, double* out1, long s10, long s11,
                       double* out2, long s20, long s21, hipStream_t s)
 {
     if (k <= 0) return hipSuccess;
     dim3 g1((p + 255) / 256, k), g2((q + 255) / 256, k);
-    svd_gather1_k<<<g1, 256, 0, s>>>(X, ldx, p, perm, scl, out1, s10, s11);
+    svd_gather1_k<<<g1, 256, 0, s>>>(X, ldx, p, perm, out1, s10, s11);
     svd_gather2_k<<<g2, 256, 0, s>>>(V, ldv, q, perm, out2, s20, s21);
     return hipGetLastError();
 }
