@@ -1262,7 +1262,9 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
         c->pack.ensure((size_t)2 * q * 8 + 256);
         double* h = c->pack.as<double>();
         double* hc = h + q + 16;
-        for (int tries = 0; tries < pc && !good[j]; tries++) {
+        // the largest of the pc unit vectors' remainders is at least 1 / pc: a
+        // second round takes the first that is not far below it
+        for (int tries = 0; tries < 2 * pc && !good[j]; tries++) {
             TN_HIP(set_unit_col(xj, pc, (jj + tries) % pc, s));
             for (int pass = 0; pass < 2; pass++) {
                 std::vector<double> coef(q);
@@ -1278,7 +1280,7 @@ int svd_device(tn_ctx* c, const double* A, long rs, long cs, int r, int cc, doub
             TN_HIP(mdot(xj, pc, 1, xj, pc, h, c->part.as<double>(), (int)pcap, s));
             TN_HIP(hipMemcpyAsync(&nr2, h, 8, hipMemcpyDeviceToHost, s));
             sync(c);
-            if (nr2 > 0.25) {
+            if (nr2 > (tries < pc ? 0.25 : 0.5 / pc)) {
                 double f = 1.0 / std::sqrt(nr2);
                 std::vector<double> one(1, f);
                 h2d(c, hc, one.data(), 8);

@@ -72,3 +72,16 @@ def test_many_columns(ctx, m, n, kind):
     elif kind == "huge":
         A *= 1e290
     _check(ctx, A)
+
+
+# the completion of a zero column: in a square matrix no unit vector need have a
+# large part outside the other columns' span
+@pytest.mark.parametrize("m,n", [(2, 2), (32, 32), (40, 40), (100, 100), (50, 32), (20, 60)])
+def test_zero_column(ctx, m, n):
+    rng = np.random.default_rng(m + 3 * n)
+    A = rng.standard_normal((m, n))
+    if m >= n:
+        A[:, n // 2] = 0.0
+    else:
+        A[m // 2] = 0.0
+    _check(ctx, A)
