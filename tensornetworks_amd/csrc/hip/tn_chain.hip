@@ -26,7 +26,7 @@ int fail(tn_ctx* c, const TnError& e)
 {
     if (c) {
         c->err = e.msg;
-        c->heff_pending = nullptr;  // the caller's stats may not outlive the call
+        c->heff_pending[0] = c->heff_pending[1] = nullptr;  // the caller's stats may not outlive the call
     }
     return e.code;
 }
@@ -163,26 +163,35 @@ void env_update(tn_chain* ch, int i, int dir, const tn_sweep_opts& o, tn_sweep_s
 }
 
 // --- Heff apply callback for the Lanczos driver ---------------------------
+static void heff_timing_flush(tn_ctx* c, int set)
+{
+    tn_sweep_stats* st = c->heff_pending[set];
+    if (!st) return;
+    heff_timing_read(c, set, &st->heff_gemm_ms, &st->heff_ms);
+    c->heff_pending[set] = nullptr;
+}
 void heff_timing_flush(tn_ctx* c)
 {
-    if (!c->heff_pending) return;
-    heff_timing_read(c, &c->heff_pending->heff_gemm_ms, &c->heff_pending->heff_ms);
-    c->heff_pending = nullptr;
+    for (int set = 0; set < 2; set++) heff_timing_flush(c, set);
+}
+
+static void heff_count(const HeffCall* hc, int n)
+{
+    if (!hc->st) return;
+    hc->st->heff_flops += n * hc->op.flops_alg(hc->D1, hc->D2);
+    hc->st->heff_gemm_flops += n * hc->op.flops_gemm(hc->D1, hc->D2);
+    hc->st->n_matvec += n;
+    if (hc->op.precision == TN_FP64) hc->st->n_matvec_fp64 += n;
 }
 
 void heff_cb(tn_ctx* c, const void* vop, const double* x, double* y)
 {
     const HeffCall* hc = (const HeffCall*)vop;
     const bool timed = hc->st != nullptr && hc->timed;
-    heff_timing_flush(c);  // the events are reused below
+    if (timed) heff_timing_flush(c, c->ev_set ^ 1);  // the set is reused by this apply
     heff_apply(c, hc->op, x, y, timed);
-    if (timed) c->heff_pending = hc->st;
-    if (hc->st) {
-        hc->st->heff_flops += hc->op.flops_alg(hc->D1, hc->D2);
-        hc->st->heff_gemm_flops += hc->op.flops_gemm(hc->D1, hc->D2);
-        hc->st->n_matvec++;
-        if (hc->op.precision == TN_FP64) hc->st->n_matvec_fp64++;
-    }
+    if (timed) c->heff_pending[c->ev_set] = hc->st;
+    heff_count(hc, 1);
 }
 
 // Identity channels of the environments of site i: for the first and the last
@@ -301,6 +310,7 @@ void eigensolve(tn_chain* ch, int i, const tn_sweep_opts& o, tn_sweep_stats* st,
             if (st) st->n_precond_fallback++;
             LanczosResult r = lanczos(c, heff_cb, &hc, N, ch->A[i], o.eig_tol, o.max_krylov, o.max_restarts, 0.0,
                                       o.reorth == 1, unit_roundoff(TN_FP64), true);
+            heff_count(&hc, -r.n_unused);
             if (st) st->n_full_reorth += r.n_full;
             *e0 = r.e0;
             *e1 = r.e1;
@@ -315,6 +325,7 @@ void eigensolve(tn_chain* ch, int i, const tn_sweep_opts& o, tn_sweep_stats* st,
     const double rel = refining ? (o.precision == TN_BF16 ? 4e-3 : 4e-7) : 0.0;
     LanczosResult r = lanczos(c, heff_cb, &hc, N, ch->A[i], o.eig_tol, o.max_krylov, o.max_restarts, rel,
                               o.reorth == 1, unit_roundoff(o.precision), true);
+    heff_count(&hc, -r.n_unused);
     if (st) st->n_full_reorth += r.n_full;
     if (refining) {
         // polish the reduced-precision Ritz vector with a more accurate operator
@@ -322,6 +333,7 @@ void eigensolve(tn_chain* ch, int i, const tn_sweep_opts& o, tn_sweep_stats* st,
         hr.op = make_heff(ch, i, o.refine_precision, o.gemm_tile, wl, wr);
         LanczosResult r2 = lanczos(c, heff_cb, &hr, N, ch->A[i], o.refine_tol, o.max_krylov, o.max_restarts, 0.0,
                                    o.reorth == 1, unit_roundoff(o.refine_precision), true);
+        heff_count(&hr, -r2.n_unused);
         if (st) st->n_full_reorth += r2.n_full;
         r.e0 = r2.e0;
         r.e1 = r2.e1;
@@ -1932,6 +1944,7 @@ int tn_chain_sweep2(tn_chain* ch, int dir, int Dmax, double eps_sv, const tn_swe
         double tl = now_ms();
         LanczosResult r = lanczos(c, heff_cb, &hc, N, ch->theta.as<double>(), o.eig_tol, o.max_krylov, o.max_restarts,
                                   0.0, o.reorth == 1, unit_roundoff(o.precision), true);
+        heff_count(&hc, -r.n_unused);
         if (st) st->n_full_reorth += r.n_full;
         if (o.refine && o.refine_precision < o.precision) {
             HeffCall h64 = hc;
@@ -1940,6 +1953,7 @@ int tn_chain_sweep2(tn_chain* ch, int dir, int Dmax, double eps_sv, const tn_swe
             h64.op.Rlo = lo_right(ch, o.refine_precision, j);
             LanczosResult r2 = lanczos(c, heff_cb, &h64, N, ch->theta.as<double>(), o.refine_tol, o.max_krylov,
                                        o.max_restarts, 0.0, o.reorth == 1, unit_roundoff(o.refine_precision), true);
+            heff_count(&h64, -r2.n_unused);
             if (st) st->n_full_reorth += r2.n_full;
             r.e0 = r2.e0;
             r.e1 = r2.e1;

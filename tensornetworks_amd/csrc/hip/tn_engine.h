@@ -89,7 +89,8 @@ struct tn_ctx {
     // preconditioned SVD: R, Q_h, reflectors (then Q_h J), T factors + GEMM work space
     tn::DBuf svd_R, svd_Q, svd_H, svd_W, svd_X2;
     tn::Scalars sc;
-    hipEvent_t ev[8] = {};
+    hipEvent_t ev[16] = {};  // two sets of eight: timed applies alternate (ev_set)
+    int ev_set = 0;
     // GEMM autotuning (off unless requested): best (tile code, k-split) per
     // problem shape, measured on first use
     bool autotune = false;
@@ -104,7 +105,7 @@ struct tn_ctx {
     // device address of this device's fixed work space (allocation-free apply)
     void* noalloc = nullptr;
     // stats whose Heff event timings are recorded but not yet read
-    tn_sweep_stats* heff_pending = nullptr;
+    tn_sweep_stats* heff_pending[2] = {nullptr, nullptr};  // per event set
     // nonzero: the next heff_apply first scales its input in place by this
     // factor (within its first pass over it) and resets it; set by the Lanczos
     // driver right before the apply of a new basis vector
@@ -112,8 +113,8 @@ struct tn_ctx {
     // nonzero after heff_apply: the result is of the scaled input, but the input
     // itself still has to be scaled by this factor (one-launch apply)
     double x_postscale = 0.0;
-    // the last timed apply was one launch: only ev[0] and ev[4] were recorded
-    bool ev_single = false;
+    // the set's timed apply was one launch: only its events 0 and 4 were recorded
+    bool ev_single[2] = {false, false};
     // seam state (tn_site_bind)
     int b_d = 0, b_D1 = 0, b_D2 = 0, b_Dw1 = 0, b_Dw2 = 0, b_prec = 0;
     int b_wl = -1, b_wr = -1;  // identity channels of the bound environments
@@ -190,7 +191,7 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
 // layout (D1 x D2 logical); false when the site or the pointers (x and y
 // overlapping) do not allow it
 bool heff_apply_ref(tn_ctx* c, const HeffOp& op, int D1, int D2, const double* x, double* y);
-void heff_timing_read(tn_ctx* c, double* gemm_ms, double* total_ms);
+void heff_timing_read(tn_ctx* c, int set, double* gemm_ms, double* total_ms);
 // per-stage times of the last timed apply (ms): s1, mix, s3
 void heff_stage_times(tn_ctx* c, double* s1, double* mix, double* s3);
 
@@ -211,6 +212,7 @@ inline size_t lowprec_bytes(int prec) { return prec == TN_FP32 ? 4 : (prec == TN
 struct LanczosResult {
     double e0 = 0, e1 = 0, residual = 0;
     int n_matvec = 0;
+    int n_unused = 0;  // applies queued ahead of the convergence test and not used (not in n_matvec)
     int n_full = 0;  // iterations with a Gram-Schmidt pass against the whole basis
     bool converged = false;
 };

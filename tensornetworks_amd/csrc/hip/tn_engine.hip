@@ -407,7 +407,9 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
     // can throw
     const double pre = c->x_prescale;
     c->x_prescale = c->x_postscale = 0.0;
-    c->ev_single = false;
+    if (timed) c->ev_set ^= 1;
+    hipEvent_t* const ev = c->ev + 8 * c->ev_set;
+    if (timed) c->ev_single[c->ev_set] = false;
     double* const xs = pre != 0.0 ? const_cast<double*>(x) : nullptr;
     hipStream_t s = c->stream;
     const int p = op.p, D1p = op.D1p, D2p = op.D2p, Dw1 = op.Dw1, Dw2 = op.Dw2;
@@ -424,7 +426,7 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
     const long n = op.n();
     const long n1 = (long)D1p * p * nR * D2p;
     const long n2 = (long)nL * D1p * p * D2p;
-    if (timed) TN_HIP(hipEventRecord(c->ev[0], s));
+    if (timed) TN_HIP(hipEventRecord(ev[0], s));
     GemmDesc g1{}, g3{};
     g1.a_kmajor = true;
     g1.b_kmajor = true;
@@ -476,8 +478,8 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
                 c->x_postscale = pre;
             }
             TN_HIP(heff_small(a, s));
-            if (timed) TN_HIP(hipEventRecord(c->ev[4], s));
-            c->ev_single = true;
+            if (timed) TN_HIP(hipEventRecord(ev[4], s));
+            if (timed) c->ev_single[c->ev_set] = true;
             return;
         }
     }
@@ -489,13 +491,13 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
             T2 = c->T2.p;
         }
         if (xs) TN_HIP(scale_copy(pre, xs, xs, n, s));
-        if (timed) TN_HIP(hipEventRecord(c->ev[1], s));
+        if (timed) TN_HIP(hipEventRecord(ev[1], s));
         g1.tin = T_F64; g1.tout = T_F64; g1.A = x; g1.B = op.R + roff; g1.C = T1;
         run(g1);
-        if (timed) TN_HIP(hipEventRecord(c->ev[2], s));
+        if (timed) TN_HIP(hipEventRecord(ev[2], s));
         TN_HIP(wmix_idt(T_F64, T_F64, T_F64, T1, (long)p * nR * D2p, x, (long)p * D2p, T2,
                         (long)nL * D1p, y, (long)p * D2p, D1p, D2p, op.mix->t, s));
-        if (timed) TN_HIP(hipEventRecord(c->ev[3], s));
+        if (timed) TN_HIP(hipEventRecord(ev[3], s));
         g3.tin = T_F64; g3.tout = T_F64; g3.A = op.L + loff; g3.B = T2; g3.C = y;
         run(g3);
     } else if (op.precision == TN_BF16X3) {
@@ -517,22 +519,22 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
         TN_REQUIRE(op.Lps > 0 && op.Rps > 0, TN_ERR_STATE, "heff_apply: split-bfloat16 operator without plane strides");
         if (xs) TN_HIP(split3_scale(xs, pre, XL, n, n, s));
         else TN_HIP(split3(T_F64, x, XL, n, n, s));
-        if (timed) TN_HIP(hipEventRecord(c->ev[1], s));
+        if (timed) TN_HIP(hipEventRecord(ev[1], s));
         if (fuse) {
             TN_HIP(x3_stage1_mix(p, nR, (const bf16*)XL, n, (const bf16*)op.Rlo + roff, op.Rps, x, (bf16*)T2, n2,
                                  (long)nL * D1p, y, D1p, D2p, op.mix->t, s));
             if (timed) {
-                TN_HIP(hipEventRecord(c->ev[2], s));
-                TN_HIP(hipEventRecord(c->ev[3], s));
+                TN_HIP(hipEventRecord(ev[2], s));
+                TN_HIP(hipEventRecord(ev[3], s));
             }
         } else {
             g1.tin = T_BF16X3; g1.tout = T_F32; g1.A = XL; g1.psA = n;
             g1.B = (const bf16*)op.Rlo + roff; g1.psB = op.Rps; g1.C = T1;
             run(g1);
-            if (timed) TN_HIP(hipEventRecord(c->ev[2], s));
+            if (timed) TN_HIP(hipEventRecord(ev[2], s));
             TN_HIP(wmix_idt(T_F32, T_F64, T_BF16X3, T1, (long)p * nR * D2p, x, (long)p * D2p, T2, (long)nL * D1p,
                             y, (long)p * D2p, D1p, D2p, op.mix->t, s, n2));
-            if (timed) TN_HIP(hipEventRecord(c->ev[3], s));
+            if (timed) TN_HIP(hipEventRecord(ev[3], s));
         }
         g3.tin = T_BF16X3; g3.tout = T_F64; g3.A = (const bf16*)op.Llo + loff; g3.psA = op.Lps;
         g3.B = T2; g3.psB = n2; g3.C = y;
@@ -550,44 +552,46 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
         }
         if (xs) TN_HIP(convert_scale(xs, pre, tl, XL, n, s));
         else TN_HIP(convert(T_F64, x, tl, XL, n, s));
-        if (timed) TN_HIP(hipEventRecord(c->ev[1], s));
+        if (timed) TN_HIP(hipEventRecord(ev[1], s));
         g1.tin = tl; g1.tout = T_F32; g1.A = XL; g1.B = (const char*)op.Rlo + roff * es; g1.C = T1;
         run(g1);
-        if (timed) TN_HIP(hipEventRecord(c->ev[2], s));
+        if (timed) TN_HIP(hipEventRecord(ev[2], s));
         TN_HIP(wmix_idt(T_F32, tl, tl, T1, (long)p * nR * D2p, XL, (long)p * D2p, T2,
                         (long)nL * D1p, y, (long)p * D2p, D1p, D2p, op.mix->t, s));
-        if (timed) TN_HIP(hipEventRecord(c->ev[3], s));
+        if (timed) TN_HIP(hipEventRecord(ev[3], s));
         g3.tin = tl; g3.tout = T_F64; g3.A = (const char*)op.Llo + loff * es; g3.B = T2; g3.C = y;
         run(g3);
     }
-    if (timed) TN_HIP(hipEventRecord(c->ev[4], s));
+    if (timed) TN_HIP(hipEventRecord(ev[4], s));
 }
 
-void heff_timing_read(tn_ctx* c, double* gemm_ms, double* total_ms)
+void heff_timing_read(tn_ctx* c, int set, double* gemm_ms, double* total_ms)
 {
+    hipEvent_t* const ev = c->ev + 8 * set;
     float t01 = 0, t12 = 0, t23 = 0, t34 = 0;
-    TN_HIP(hipEventSynchronize(c->ev[4]));
-    if (c->ev_single) {
-        TN_HIP(hipEventElapsedTime(&t01, c->ev[0], c->ev[4]));
+    TN_HIP(hipEventSynchronize(ev[4]));
+    if (c->ev_single[set]) {
+        TN_HIP(hipEventElapsedTime(&t01, ev[0], ev[4]));
         if (gemm_ms) *gemm_ms += t01;
         if (total_ms) *total_ms += t01;
         return;
     }
-    TN_HIP(hipEventElapsedTime(&t01, c->ev[0], c->ev[1]));
-    TN_HIP(hipEventElapsedTime(&t12, c->ev[1], c->ev[2]));
-    TN_HIP(hipEventElapsedTime(&t23, c->ev[2], c->ev[3]));
-    TN_HIP(hipEventElapsedTime(&t34, c->ev[3], c->ev[4]));
+    TN_HIP(hipEventElapsedTime(&t01, ev[0], ev[1]));
+    TN_HIP(hipEventElapsedTime(&t12, ev[1], ev[2]));
+    TN_HIP(hipEventElapsedTime(&t23, ev[2], ev[3]));
+    TN_HIP(hipEventElapsedTime(&t34, ev[3], ev[4]));
     if (gemm_ms) *gemm_ms += (double)t12 + (double)t34;
     if (total_ms) *total_ms += (double)t01 + t12 + t23 + t34;
 }
 
 void heff_stage_times(tn_ctx* c, double* s1, double* mix, double* s3)
 {
+    hipEvent_t* const ev = c->ev + 8 * c->ev_set;
     float t12 = 0, t23 = 0, t34 = 0;
-    TN_HIP(hipEventSynchronize(c->ev[4]));
-    TN_HIP(hipEventElapsedTime(&t12, c->ev[1], c->ev[2]));
-    TN_HIP(hipEventElapsedTime(&t23, c->ev[2], c->ev[3]));
-    TN_HIP(hipEventElapsedTime(&t34, c->ev[3], c->ev[4]));
+    TN_HIP(hipEventSynchronize(ev[4]));
+    TN_HIP(hipEventElapsedTime(&t12, ev[1], ev[2]));
+    TN_HIP(hipEventElapsedTime(&t23, ev[2], ev[3]));
+    TN_HIP(hipEventElapsedTime(&t34, ev[3], ev[4]));
     *s1 = t12;
     *mix = t23;
     *s3 = t34;
@@ -880,6 +884,12 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
     // the scaling of the next basis vector not launched yet (prescale)
     double pending = 0.0;
     c->x_prescale = 0.0;
+    // Vectors up to 2 MB leave a full step at unit length (one pass over w more
+    // than a scaling inside the next apply's first pass, about 2 us at this
+    // length), so that the next apply can be queued before the host has seen the
+    // step's numbers: the host's answer takes about 12 us, a third of an iteration
+    // of a small site.  Longer applies hide none of their own time behind it.
+    const bool unit = !pro && N <= (1L << 18);
 
     // h[0..nh) and |w|^2 of the last lz_update
     auto read = [&](double* dst, int nh) {
@@ -916,6 +926,7 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
         bool conv = false;
         bool force = false;     // the previous vector had a full pass: this one gets one too
         double tnorm = 0.0;     // Gershgorin bound on |T|
+        bool ahead = false;     // the apply of v_j is queued already
         om[0] = 1.0;
         for (int j = 0; j < kmax; j++) {
             double* vj = V + (long)j * N;
@@ -925,11 +936,12 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
                 pending = 0.0;
             }
             try {
-                fn(c, op, vj, hv);
+                if (!ahead) fn(c, op, vj, hv);
             } catch (...) {
                 c->x_prescale = c->x_postscale = 0.0;
                 throw;
             }
+            ahead = false;
             const double post = c->x_postscale;  // v_j still to be scaled by this
             c->x_postscale = 0.0;
             res.n_matvec++;
@@ -942,11 +954,9 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
             const int kk = pro ? (j >= 1 ? 2 : 1) : j + 1;
             double* Vl = V + (long)(j + 1 - kk) * N;
             const double beta = j > 0 ? be[j - 1] : 0.0;
-            const bool tiny = lz_small_ok(N, kk);
-            if (tiny) {
-                const unsigned long long seq = ++c->sc.seq;
-                TN_HIP(lz_small(hv, Vl, N, kk, post != 0.0 ? post : 1.0, beta, !pro, N, c->sc.d, c->sc.flag_d, seq, s));
-                read_published(c, hh.data(), kk + 2, seq);
+            const unsigned long long seq = ++c->sc.seq;
+            if (lz_small_ok(N, kk)) {
+                TN_HIP(lz_small(hv, Vl, N, kk, post != 0.0 ? post : 1.0, beta, unit, N, c->sc.d, c->sc.flag_d, seq, s));
             } else {
                 if (post != 0.0) TN_HIP(scale_copy(post, vj, vj, N, s));
                 TN_HIP(lz_dot(vj, hv, N, part, s));
@@ -954,8 +964,17 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
                 // the Gram-Schmidt update fused with the norm
                 TN_HIP(lz_step(hv, w, Vl, N, kk, true, beta, N, h, part, s));
                 TN_HIP(lz_update(w, Vl, N, kk, N, h + 1, part, s));
-                read(hh.data(), kk + 1);
+                if (unit) TN_HIP(lz_publish_unit(h, kk + 1, w, N, part, c->sc.d, c->sc.flag_d, seq, s));
+                else TN_HIP(lz_publish(h, kk + 1, N, part, c->sc.d, c->sc.flag_d, seq, s));
             }
+            // the next apply ahead of this step's test, unless the last residual
+            // says that the test may end the iteration
+            if (unit && j >= 1 && j + 1 < kmax &&
+                res.residual > 100.0 * std::max(tol, tol_rel * std::fabs(res.e0))) {
+                fn(c, op, w, hv);
+                ahead = true;
+            }
+            read_published(c, hh.data(), kk + 2, seq);
             if (pro) {
                 al[j] = hh[0] + hh[kk];
                 be[j] = std::sqrt(std::max(hh[kk + 1], 0.0));
@@ -1007,10 +1026,11 @@ LanczosResult lanczos(tn_ctx* c, ApplyFn fn, const void* op, long N, double* x, 
             if (done || j + 1 == kmax)  // the second Ritz value is only reported
                 tridiag_lowest(j + 1, al.data(), be.data(), &res.e0, &res.e1, z.data(), true);
             if (done) {
+                res.n_unused += ahead;
                 conv = true;
                 break;
             }
-            if (j + 1 < kmax && !(tiny && !pro)) {
+            if (j + 1 < kmax && !unit) {
                 if (prescale) pending = 1.0 / be[j];
                 else TN_HIP(scale_copy(1.0 / be[j], w, w, N, s));
             }

@@ -192,7 +192,7 @@ hipError_t axpby(double a, const double* x, double b, double* y, long n, hipStre
 //              latter when k >= 2; y and w different buffers); not three: w as
 //              it is.  Then partial sums of V_i . w, i < k
 //  lz_update : coef[i] = V_i . w, w <- w - sum_{i<k} coef[i] V_i, partial |w|^2
-//  lz_publish: h[0..nh) and |w|^2 to the host (see publish)
+//  lz_publish: h[0..nh) and |w|^2 to the host (see publish); _unit: then w / |w|
 long lz_part_size(long n, int k);
 hipError_t lz_dot(const double* v, const double* w, long n, double* part, hipStream_t s);
 hipError_t lz_step(const double* y, double* w, const double* V, long ldv, int k, bool three, double beta, long n,
@@ -206,6 +206,8 @@ hipError_t lz_small(const double* y, double* V, long ldv, int k, double vscale, 
                     double* host_dst, unsigned long long* host_flag, unsigned long long seq, hipStream_t s);
 hipError_t lz_publish(const double* h, int nh, long n, const double* part, double* host_dst,
                       unsigned long long* host_flag, unsigned long long seq, hipStream_t s);
+hipError_t lz_publish_unit(const double* h, int nh, double* w, long n, const double* part, double* host_dst,
+                           unsigned long long* host_flag, unsigned long long seq, hipStream_t s);
 // y = a x (y is not read; x and y may be the same buffer)
 hipError_t scale_copy(double a, const double* x, double* y, long n, hipStream_t s);
 

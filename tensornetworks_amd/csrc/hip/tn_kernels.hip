@@ -993,6 +993,45 @@ __global__ void __launch_bounds__(MD_BLOCK) lz_publish_k(const double* __restric
     }
 }
 
+// The same with w <- w / |w|: every workgroup forms |w|^2 from npart as the first
+// one does for the host, so the next apply can be queued on w before the host has
+// seen |w| (one launch for the publication and the scaling: 4.8 us at n = 92160,
+// 6.8 us for the two; no wait between this step and the next apply).
+__global__ void __launch_bounds__(MD_BLOCK) lz_publish_unit_k(const double* __restrict__ h, int nh,
+                                                              const double* __restrict__ npart, int G,
+                                                              double* __restrict__ w, long n, double* host_dst,
+                                                              unsigned long long* host_flag, unsigned long long seq)
+{
+    __shared__ double red[4];
+    const long i = 2 * (blockIdx.x * (long)MD_BLOCK + threadIdx.x);
+    double2 x = i < n ? *(const double2*)(w + i) : make_double2(0.0, 0.0);
+    const double nn = block_sum(npart, G, red);
+    if (blockIdx.x == 0) {
+        for (int t = threadIdx.x; t < nh; t += MD_BLOCK) host_dst[t] = h[t];
+        if (threadIdx.x == 0) host_dst[nh] = nn;
+        __threadfence_system();  // every wave's stores before the flag (see publish_k)
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            __threadfence_system();
+            *(volatile unsigned long long*)host_flag = seq;
+        }
+    }
+    const double f = 1.0 / sqrt(nn);  // infinite when the Krylov space is complete: w is not used then
+    x.x *= f;
+    x.y *= f;
+    if (i < n) *(double2*)(w + i) = x;
+}
+
+hipError_t lz_publish_unit(const double* h, int nh, double* w, long n, const double* part, double* host_dst,
+                           unsigned long long* host_flag, unsigned long long seq, hipStream_t s)
+{
+    if (nh < 0 || nh >= TN_PUBLISH_MAX || n <= 0 || (n & 1)) return hipErrorInvalidValue;
+    const unsigned grid = (unsigned)((n + 2 * MD_BLOCK - 1) / (2 * MD_BLOCK));
+    lz_publish_unit_k<<<grid, MD_BLOCK, 0, s>>>(h, nh, part + lz_dot_blocks(n), (int)lz_norm_blocks(n), w, n, host_dst,
+                                                host_flag, seq);
+    return hipGetLastError();
+}
+
 hipError_t lz_publish(const double* h, int nh, long n, const double* part, double* host_dst,
                       unsigned long long* host_flag, unsigned long long seq, hipStream_t s)
 {
