@@ -1003,7 +1003,9 @@ static const StepCost kCostF32[] = {
 // split bf16 (steps of 32): 128x128 .. 32x32, 96x128, 128x96, 192x256, 256x192,
 // 192x128, 128x192.  1024 x 3072 x 4096: 208 us in the 128x64 tiles of the
 // block-count rule, 134 us in 128x192 with a 2-way split (1.15 PFLOP/s of bf16);
-// 512 x 1536 x 2048: 36 -> 32 us; 320 x 448 x 1280: 19 -> 12 us
+// 512 x 1536 x 2048: 36 -> 32 us; 320 x 448 x 1280: 19 -> 12 us.  Small tiles of
+// long products are bound by what they read from the caches, at most about 13 TB/s
+// (672 x 2688 x 2688: 162 us in 32x64, 97 us in 96x128, both in two K halves).
 static const StepCost kCostX3[] = {
     {0, 1.42f, 1.60f}, {1, 0.715f, 1.00f}, {2, 0.708f, 1.00f}, {3, 0.418f, 0.60f},  {4, 0.285f, 0.41f},
     {5, 0.274f, 0.36f}, {6, 0.167f, 0.266f}, {10, 1.02f, 1.48f}, {11, 1.00f, 1.48f}, {12, 4.0f, 4.0f},
@@ -1028,7 +1030,9 @@ void gemm_default(int tin, int M, int N, int K, int batch, bool split, int* tile
             if (ks > 1 && (!split || batch != 1 || K % (64 * ks))) break;
             const long blocks = (long)(M / t.bm) * (N / t.bn) * batch * ks;
             const float busy = (float)((blocks + 255) / 256) * c.busy;
-            float us = 3.7f + (float)(K / ks) / bk * (busy > c.alone ? busy : c.alone);
+            float us = (float)(K / ks) / bk * (busy > c.alone ? busy : c.alone);
+            if (tin == T_BF16X3) us = std::max(us, (float)blocks * (K / ks) * (t.bm + t.bn) * 6 / 13e6f);
+            us += 3.7f;
             if (ks > 1) us += 3.0f + (float)M * N * (2 * ks * es + 8) * 1e-7f;
             if (us < best) {
                 best = us;
