@@ -1136,14 +1136,13 @@ int tn_heff_apply_device(tn_ctx* c, const double* x, double* y, int64_t N)
     TN_REQUIRE(c->bound, TN_ERR_STATE, "tn_heff_apply_device: no site bound");
     TN_REQUIRE(x && y && N == (int64_t)c->b_d * c->b_D1 * c->b_D2, TN_ERR_ARG,
                "tn_heff_apply_device: N != d*D1*D2");
-    const int d = c->b_d, D1 = c->b_D1, D2 = c->b_D2, D1p = pad32(D1), D2p = pad32(D2);
+    const int d = c->b_d, D1 = c->b_D1, D2 = c->b_D2, D2p = pad32(D2);
     HeffOp op = bound_op(c);
     if (heff_apply_ref(c, op, D1, D2, x, y)) {
         sync(c);
         return TN_OK;
     }
-    TN_HIP(psi_ref_to_int(x, c->b_x.as<double>(), d, D1, D2, D1p, D2p, c->stream));
-    heff_apply(c, op, c->b_x.as<double>(), c->b_y.as<double>(), false);
+    heff_apply_from_ref(c, op, D1, D2, x, c->b_x.as<double>(), c->b_y.as<double>());
     TN_HIP(psi_int_to_ref(c->b_y.as<double>(), y, d, D1, D2, D2p, c->stream));
     sync(c);
     return TN_OK;
@@ -1158,7 +1157,7 @@ int tn_heff_apply_device_noalloc(tn_ctx* c, const double* x, double* y, int64_t 
     TN_REQUIRE(x && y && N == (int64_t)c->b_d * c->b_D1 * c->b_D2, TN_ERR_ARG,
                "tn_heff_apply_device_noalloc: N != d*D1*D2");
     TN_REQUIRE(c->noalloc != nullptr, TN_ERR_STATE, "tn_heff_apply_device_noalloc: no work space on this device");
-    const int d = c->b_d, D1 = c->b_D1, D2 = c->b_D2, D1p = pad32(D1), D2p = pad32(D2);
+    const int d = c->b_d, D1 = c->b_D1, D2 = c->b_D2, D2p = pad32(D2);
     HeffOp op = bound_op(c);
     // work space layout: x and y in the internal layout, then the stage buffers;
     // every byte a call reads is written earlier in the same call
@@ -1177,8 +1176,7 @@ int tn_heff_apply_device_noalloc(tn_ctx* c, const double* x, double* y, int64_t 
     double* xi = (double*)base;
     double* yi = (double*)(base + bv);
     HeffScratch scr{base + 2 * bv, b1, base + 2 * bv + b1, b2, bx ? base + 2 * bv + b1 + b2 : nullptr, bx};
-    TN_HIP(psi_ref_to_int(x, xi, d, D1, D2, D1p, D2p, c->stream));
-    heff_apply(c, op, xi, yi, false, &scr);
+    heff_apply_from_ref(c, op, D1, D2, x, xi, yi, &scr);
     TN_HIP(psi_int_to_ref(yi, y, d, D1, D2, D2p, c->stream));
     sync(c);
     return TN_OK;

@@ -187,6 +187,10 @@ void gemm_run_fixed(tn_ctx* c, const GemmDesc& g);
 // one-launch form of small FP64 sites (whose stages have no times of their own).
 void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool timed,
                 const HeffScratch* scr = nullptr, bool stages = false);
+// y = Heff x with x in the reference layout (D1 x D2 logical): its internal copy,
+// formed in xi, and its low-precision operand in one pass
+void heff_apply_from_ref(tn_ctx* c, const HeffOp& op, int D1, int D2, const double* x, double* xi, double* y,
+                         const HeffScratch* scr = nullptr);
 // y = Heff x of a small FP64 site in one launch with x and y in the reference
 // layout (D1 x D2 logical); false when the site or the pointers (x and y
 // overlapping) do not allow it

@@ -399,8 +399,10 @@ bool heff_apply_ref(tn_ctx* c, const HeffOp& op, int D1, int D2, const double* x
     return true;
 }
 
-void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool timed, const HeffScratch* scr,
-                bool stages)
+// lo_ready: x's low-precision operand is in the work space already (for FP32 and
+// BF16 x itself is then not read)
+static void apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool timed, const HeffScratch* scr,
+                  bool stages, bool lo_ready)
 {
     // a pending Lanczos scaling of x (x is then the driver's own basis vector,
     // scaled in place within the first pass over it), taken before anything
@@ -518,7 +520,7 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
         }
         TN_REQUIRE(op.Lps > 0 && op.Rps > 0, TN_ERR_STATE, "heff_apply: split-bfloat16 operator without plane strides");
         if (xs) TN_HIP(split3_scale(xs, pre, XL, n, n, s));
-        else TN_HIP(split3(T_F64, x, XL, n, n, s));
+        else if (!lo_ready) TN_HIP(split3(T_F64, x, XL, n, n, s));
         if (timed) TN_HIP(hipEventRecord(ev[1], s));
         if (fuse) {
             TN_HIP(x3_stage1_mix(p, nR, (const bf16*)XL, n, (const bf16*)op.Rlo + roff, op.Rps, x, (bf16*)T2, n2,
@@ -551,7 +553,7 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
             T2 = c->T2.p;
         }
         if (xs) TN_HIP(convert_scale(xs, pre, tl, XL, n, s));
-        else TN_HIP(convert(T_F64, x, tl, XL, n, s));
+        else if (!lo_ready) TN_HIP(convert(T_F64, x, tl, XL, n, s));
         if (timed) TN_HIP(hipEventRecord(ev[1], s));
         g1.tin = tl; g1.tout = T_F32; g1.A = XL; g1.B = (const char*)op.Rlo + roff * es; g1.C = T1;
         run(g1);
@@ -563,6 +565,28 @@ void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool ti
         run(g3);
     }
     if (timed) TN_HIP(hipEventRecord(ev[4], s));
+}
+
+void heff_apply(tn_ctx* c, const HeffOp& op, const double* x, double* y, bool timed, const HeffScratch* scr,
+                bool stages)
+{
+    apply(c, op, x, y, timed, scr, stages, false);
+}
+
+void heff_apply_from_ref(tn_ctx* c, const HeffOp& op, int D1, int D2, const double* x, double* xi, double* y,
+                         const HeffScratch* scr)
+{
+    if (op.precision == TN_FP64) {
+        TN_HIP(psi_ref_to_int(x, xi, op.p, D1, D2, op.D1p, op.D2p, c->stream));
+    } else {
+        size_t b1, b2, bx;
+        heff_scratch_bytes(op, &b1, &b2, &bx);
+        TN_REQUIRE(!scr || (scr->xlo && scr->xlo_bytes >= bx), TN_ERR_ARG, "heff_apply: work space too small");
+        if (!scr) c->xlo.ensure(bx);
+        const int tlo = op.precision == TN_BF16X3 ? (int)T_BF16X3 : (int)lo_type(op.precision);
+        TN_HIP(psi_ref_to_int_lo(x, tlo, xi, scr ? scr->xlo : c->xlo.p, op.p, D1, D2, op.D1p, op.D2p, c->stream));
+    }
+    apply(c, op, xi, y, false, scr, false, true);
 }
 
 void heff_timing_read(tn_ctx* c, int set, double* gemm_ms, double* total_ms)

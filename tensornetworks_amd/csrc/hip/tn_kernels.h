@@ -161,6 +161,10 @@ hipError_t fill_value(double* p, double v, long n, hipStream_t s);
 // site tensor layouts: reference psi[m + d*(a + D1*b)] <-> internal
 // out[(a*d + m)*D2p + b] over [D1p][d][D2p] (padding written as zero)
 hipError_t psi_ref_to_int(const double* ref, double* out, int d, int D1, int D2, int D1p, int D2p, hipStream_t s);
+// and the low-precision operand in the same pass: lo (T_F32, T_BF16 or T_BF16X3 with
+// planes d*D1p*D2p apart); out is written for T_BF16X3 only
+hipError_t psi_ref_to_int_lo(const double* ref, int tlo, double* out, void* lo, int d, int D1, int D2, int D1p, int D2p,
+                             hipStream_t s);
 hipError_t psi_int_to_ref(const double* in, double* ref, int d, int D1, int D2, int D2p, hipStream_t s);
 
 // copy a 3-index tensor with a strided view: out[(i*n1 + j)*n2o + k] = in[i*si + j*sj + k*sk]
