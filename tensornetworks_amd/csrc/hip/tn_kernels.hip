@@ -609,7 +609,9 @@ hipError_t mdot(const double* V, long ldv, int k, const double* w, long n, doubl
 // iteration with a pass against k vectors, that form (with a second launch per
 // reduction) and this one: n = 2048, k ~ 28: 58 and 15 us; n = 92160, k ~ 84:
 // 224 and 43 us (the 62 MB basis read twice: 2.9 TB/s); n = 196608, k = 2
-// (partial re-orthogonalisation): 33 and 22 us.
+// (partial re-orthogonalisation): 33 and 22 us.  lz_step has its first eight
+// vectors in flight while it sums alpha: 25 -> 19 us at n = 92160, k ~ 84, 9.5 ->
+// 5.9 us at n = 18432, k ~ 12.
 #define LZ_SMALL 131072  // entries up to which chunks are sized for latency
 
 // entry pairs per thread of lz_step: one while the vectors are short or few (a
@@ -637,15 +639,20 @@ long lz_part_size(long n, int k)
     return lz_dot_blocks(n) + lz_norm_blocks(n) + (few > all ? few : all);
 }
 
-// sum of v[0..n) over the workgroup (MD_BLOCK threads), the same on every thread
-__device__ __forceinline__ double block_sum(const double* __restrict__ v, int n, double* red)
+// sum of acc, or of v[0..n), over the workgroup (MD_BLOCK threads), the same on every
+// thread
+__device__ __forceinline__ double block_total(double acc, double* red)
 {
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < n; i += MD_BLOCK) acc += v[i];
     acc = wave_sum(acc);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
     __syncthreads();
     return (red[0] + red[1]) + (red[2] + red[3]);
+}
+__device__ __forceinline__ double block_sum(const double* __restrict__ v, int n, double* red)
+{
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += MD_BLOCK) acc += v[i];
+    return block_total(acc, red);
 }
 
 template <int P>
@@ -684,8 +691,25 @@ __global__ void __launch_bounds__(MD_BLOCK) lz_step_k(const double* __restrict__
     __shared__ double red[2][8][4];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const long c0 = (long)blockIdx.x * 2 * MD_BLOCK * P;
+    const int i1 = min(k, (int)(blockIdx.y + 1) * ng);
+    // eight vectors at a time: their loads and their lane reductions are
+    // independent (a vector past the last one repeats it and is dropped)
+    double2 v[8][P];
+    auto load = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const double* vi = V + (long)min(i0 + u, i1 - 1) * ldv;
+#pragma unroll
+            for (int e = 0; e < P; e++) {
+                const long idx = c0 + 2 * (e * MD_BLOCK + tid);
+                v[u][e] = idx < n ? *(const double2*)(vi + idx) : make_double2(0.0, 0.0);
+            }
+        }
+    };
     double2 x[P];
     if (na > 0) {
+        double asum = 0.0;
+        for (int i = tid; i < na; i += MD_BLOCK) asum += apart[i];
         const double* vj = V + (long)(k - 1) * ldv;
         const double* vm = k >= 2 ? V + (long)(k - 2) * ldv : vj;
         const double b = k >= 2 ? beta : 0.0;
@@ -698,7 +722,8 @@ __global__ void __launch_bounds__(MD_BLOCK) lz_step_k(const double* __restrict__
             p[e] = in ? *(const double2*)(vj + idx) : make_double2(0.0, 0.0);
             q[e] = in ? *(const double2*)(vm + idx) : make_double2(0.0, 0.0);
         }
-        const double a = block_sum(apart, na, ared);
+        load(blockIdx.y * ng);  // in flight while alpha is summed
+        const double a = block_total(asum, ared);
         if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) aout[0] = a;
 #pragma unroll
         for (int e = 0; e < P; e++) {
@@ -715,27 +740,19 @@ __global__ void __launch_bounds__(MD_BLOCK) lz_step_k(const double* __restrict__
             const long idx = c0 + 2 * (e * MD_BLOCK + tid);
             x[e] = idx < n ? *(const double2*)(w + idx) : make_double2(0.0, 0.0);
         }
+        load(blockIdx.y * ng);
     }
-    const int i1 = min(k, (int)(blockIdx.y + 1) * ng);
     int par = 0;
     for (int i0 = blockIdx.y * ng; i0 < i1; i0 += 8, par ^= 1) {
-        // eight vectors at a time: their loads and their lane reductions are
-        // independent (a vector past the last one repeats it and is dropped)
         double acc[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-            const double* vi = V + (long)min(i0 + u, i1 - 1) * ldv;
             double s = 0.0;
 #pragma unroll
-            for (int e = 0; e < P; e++) {
-                const long idx = c0 + 2 * (e * MD_BLOCK + tid);
-                if (idx < n) {
-                    const double2 v = *(const double2*)(vi + idx);
-                    s += v.x * x[e].x + v.y * x[e].y;
-                }
-            }
+            for (int e = 0; e < P; e++) s += v[u][e].x * x[e].x + v[u][e].y * x[e].y;
             acc[u] = s;
         }
+        if (i0 + 8 < i1) load(i0 + 8);
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1)
 #pragma unroll
