@@ -1870,7 +1870,11 @@ __device__ __forceinline__ double wave_bcast(double v, int lane)
 // are never read again.  The column and row buffers alternate between two
 // LDS slots by step parity, so one barrier per step orders them: a wave can
 // only overwrite a slot after every wave has passed the next barrier, that
-// is, after every wave has read it.
+// is, after every wave has read it.  Columns past nbk are the identity's and
+// are left out: a block of 32 takes 15 us, as one of 64 completed with the
+// identity it took 27.  (A wave factoring its 16 columns alone in registers, the
+// others updating theirs 16 columns at a time, took 29 us for 64 against 28: the
+// chain of square root and division per column is the bound, not the barriers.)
 __device__ __forceinline__ void chol_block(const double* __restrict__ G, long ldg, int k0, int nbk,
                                            double* __restrict__ L, long ldl, double* __restrict__ Linv, long ldi,
                                            int* __restrict__ flag, double (*Ls)[CB + 1], double (*col)[CB],
@@ -1899,7 +1903,7 @@ __device__ __forceinline__ void chol_block(const double* __restrict__ G, long ld
     }
     __syncthreads();  // every row is in registers before Ls takes L
     int bad = 0;
-    for (int jb = 0; jb < CB / CW; jb++) {
+    for (int jb = 0; jb * CW < nbk; jb++) {
 #pragma unroll
         for (int jj = 0; jj < CW; jj++) {
             const int j = jb * CW + jj, slot = jj & 1;
