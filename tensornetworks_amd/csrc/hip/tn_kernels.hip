@@ -680,7 +680,7 @@ __global__ void __launch_bounds__(MD_BLOCK) lz_dot_k(const double* __restrict__ 
 // part[i*gridDim.x + block] = V_i . w over the block's entries, for the ng
 // vectors i of block row blockIdx.y (w is formed by every block row, written
 // by the first: y and w are different buffers).
-template <int P>
+template <int P, int U>
 __global__ void __launch_bounds__(MD_BLOCK) lz_step_k(const double* __restrict__ y, double* __restrict__ w,
                                                       const double* __restrict__ V, long ldv, int k,
                                                       const double* __restrict__ apart, int na,
@@ -688,21 +688,20 @@ __global__ void __launch_bounds__(MD_BLOCK) lz_step_k(const double* __restrict__
                                                       double* __restrict__ part)
 {
     __shared__ double ared[4];
-    __shared__ double red[2][8][4];
+    __shared__ double red[2][U][4];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     const long c0 = (long)blockIdx.x * 2 * MD_BLOCK * P;
     const int i1 = min(k, (int)(blockIdx.y + 1) * ng);
-    // eight vectors at a time: their loads and their lane reductions are
-    // independent (a vector past the last one repeats it and is dropped)
-    double2 v[8][P];
+    // U vectors at a time: their loads and their lane reductions are independent
+    double2 v[U][P];
     auto load = [&](int i0) {
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const double* vi = V + (long)min(i0 + u, i1 - 1) * ldv;
+        for (int u = 0; u < U; u++) {
+            const double* vi = V + (long)(i0 + u) * ldv;
 #pragma unroll
             for (int e = 0; e < P; e++) {
                 const long idx = c0 + 2 * (e * MD_BLOCK + tid);
-                v[u][e] = idx < n ? *(const double2*)(vi + idx) : make_double2(0.0, 0.0);
+                v[u][e] = i0 + u < i1 && idx < n ? *(const double2*)(vi + idx) : make_double2(0.0, 0.0);
             }
         }
     };
@@ -743,26 +742,26 @@ __global__ void __launch_bounds__(MD_BLOCK) lz_step_k(const double* __restrict__
         load(blockIdx.y * ng);
     }
     int par = 0;
-    for (int i0 = blockIdx.y * ng; i0 < i1; i0 += 8, par ^= 1) {
-        double acc[8];
+    for (int i0 = blockIdx.y * ng; i0 < i1; i0 += U, par ^= 1) {
+        double acc[U];
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
+        for (int u = 0; u < U; u++) {
             double s = 0.0;
 #pragma unroll
             for (int e = 0; e < P; e++) s += v[u][e].x * x[e].x + v[u][e].y * x[e].y;
             acc[u] = s;
         }
-        if (i0 + 8 < i1) load(i0 + 8);
+        if (i0 + U < i1) load(i0 + U);
 #pragma unroll
         for (int o = 32; o >= 1; o >>= 1)
 #pragma unroll
-            for (int u = 0; u < 8; u++) acc[u] += __shfl_xor(acc[u], o, 64);
+            for (int u = 0; u < U; u++) acc[u] += __shfl_xor(acc[u], o, 64);
         if (lane == 0) {
 #pragma unroll
-            for (int u = 0; u < 8; u++) red[par][u][wid] = acc[u];
+            for (int u = 0; u < U; u++) red[par][u][wid] = acc[u];
         }
         __syncthreads();  // the other slot of red is read before the next round's barrier
-        if (tid < 8 && i0 + tid < i1)
+        if (tid < U && i0 + tid < i1)
             part[(long)(i0 + tid) * gridDim.x + blockIdx.x] =
                 (red[par][tid][0] + red[par][tid][1]) + (red[par][tid][2] + red[par][tid][3]);
     }
@@ -881,8 +880,12 @@ hipError_t lz_step(const double* y, double* w, const double* V, long ldv, int k,
     const int ng = 8 * ((groups + S - 1) / S);
     const dim3 grid(G, (k + ng - 1) / ng);
     const int nap = three ? (int)na : 0;
-    if (lz_step_pairs(n, k) == 1) lz_step_k<1><<<grid, MD_BLOCK, 0, s>>>(y, w, V, ldv, k, part, nap, h, beta, n, ng, dots);
-    else lz_step_k<4><<<grid, MD_BLOCK, 0, s>>>(y, w, V, ldv, k, part, nap, h, beta, n, ng, dots);
+    // one or two vectors (partial re-orthogonalisation): room for two only, so that
+    // more workgroups of the long streams fit on a CU (with room for eight a sweep at
+    // D = 1024, n = 3.1e6, took 2.15 s, with two 2.07 s)
+    if (lz_step_pairs(n, k) == 1) lz_step_k<1, 8><<<grid, MD_BLOCK, 0, s>>>(y, w, V, ldv, k, part, nap, h, beta, n, ng, dots);
+    else if (k <= 2) lz_step_k<4, 2><<<grid, MD_BLOCK, 0, s>>>(y, w, V, ldv, k, part, nap, h, beta, n, ng, dots);
+    else lz_step_k<4, 8><<<grid, MD_BLOCK, 0, s>>>(y, w, V, ldv, k, part, nap, h, beta, n, ng, dots);
     return hipGetLastError();
 }
 
