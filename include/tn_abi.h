@@ -316,6 +316,13 @@ int tn_chain_heff_bench(tn_chain* chain, int site, int precision, int reps, int 
  * (batch 1, K a multiple of 64 ksplit). */
 int tn_gemm_test(tn_ctx* ctx, int tin, int tout, int a_kmajor, int b_kmajor, int M, int N, int K,
                  int batch, const double* A, const double* B, double* C, int tile, int ksplit);
+/* GEMM diagnostic (host only, no device needed): the built-in tile code and, with
+ * split, the k-split of a batch of M x N x K products with operands of type tin,
+ * as a context without a tuning table takes them; *wide = 1 when the leading
+ * dimensions lda, ldb (elements) are too large for the tile's 32-bit copy offsets,
+ * so that the product runs in the 32x32 tile with 64-bit ones. */
+int tn_gemm_plan(int tin, int a_kmajor, int b_kmajor, int M, int N, int K, int64_t lda, int64_t ldb, int batch,
+                 int split, int* tile, int* ksplit, int* wide);
 
 /* ---- batched chains (no reference counterpart: the reference sweeps one
  * MPS at a time) ----

@@ -17,6 +17,7 @@ from ._abi import (  # noqa: F401
     SweepOpts,
     SweepStats,
     TnError,
+    gemm_plan,
     lib,
     mpo_reduce,
     read_checkpoint_mpo,
@@ -28,7 +29,8 @@ from .dmrg import FindVariationalGroundState, ScheduleLine  # noqa: F401
 
 __all__ = [
     "Context", "Chain", "Batch", "SweepOpts", "SweepStats", "TnError", "lib", "LIB_PATH",
-    "TN_FP64", "TN_FP32", "TN_BF16", "TN_BF16X3", "MLP_NP", "svcompress_rank", "mpo_reduce", "read_checkpoint_mpo",
+    "TN_FP64", "TN_FP32", "TN_BF16", "TN_BF16X3", "MLP_NP", "svcompress_rank", "gemm_plan", "mpo_reduce",
+    "read_checkpoint_mpo",
     "xxz_mpo", "tfim_mpo", "long_range_mpo", "three_body_mpo", "mpo_square", "identity_mpo", "mpo_contract",
     "FindVariationalGroundState", "ScheduleLine",
 ]

@@ -108,6 +108,7 @@ def _load():
         "tn_svd": (i, [v, i, i, _dp, _dp, _dp, _dp]),
         "tn_svcompress_rank": (i, [i, _dp, i, d, _dp, _dp]),
         "tn_gemm_test": (i, [v, i, i, i, i, i, i, i, i, _dp, _dp, _dp, i, i]),
+        "tn_gemm_plan": (i, [i, i, i, i, i, i, ctypes.c_int64, ctypes.c_int64, i, i, _ip, _ip, _ip]),
         "tn_cholqr_test": (i, [v, i, i, _dp, ctypes.c_double, _dp, _dp, _ip, i]),
         "tn_ctx_set_autotune": (i, [v, i]),
         "tn_copy_bench": (i, [v, ctypes.c_int64, _dp]),
@@ -176,6 +177,18 @@ def P(a):
 def IP(a):
     assert a.dtype == np.int32 and a.flags["C_CONTIGUOUS"]
     return a.ctypes.data_as(_ip)
+
+
+def gemm_plan(tin, a_kmajor, b_kmajor, M, N, K, lda=None, ldb=None, batch=1, split=False):
+    """Built-in (tile code, k-split, wide) of a GEMM; no device needed."""
+    out = [ctypes.c_int(), ctypes.c_int(), ctypes.c_int()]
+    lda = lda if lda else (K if a_kmajor else M)
+    ldb = ldb if ldb else (K if b_kmajor else N)
+    rc = lib.tn_gemm_plan(tin, int(a_kmajor), int(b_kmajor), M, N, K, lda, ldb, batch, int(split),
+                          *[ctypes.byref(x) for x in out])
+    if rc != TN_OK:
+        raise TnError(rc, "tn_gemm_plan")
+    return tuple(x.value for x in out)
 
 
 def svcompress_rank(s, Dmax, eps):

@@ -196,7 +196,7 @@ void readback(tn_batch* b, double* dst, const double* src, size_t n)
 struct GroupLaunch {
     int tin, tout;
     bool akm, bkm;
-    int tile, bk;
+    int tile;
     const GemmProb* probs;
     const int* off;
     int nprob, total;
@@ -207,7 +207,7 @@ std::vector<GroupLaunch> gemm_group_stage(tn_batch* b, const std::vector<GemmDes
     std::vector<GroupLaunch> out;
     if (list.empty()) return out;
     tn_ctx* c = b->ctx;
-    std::map<std::pair<int, int>, std::vector<int>> groups;
+    std::map<int, std::vector<int>> groups;
     for (int q = 0; q < (int)list.size(); q++) {
         const GemmDesc& g = list[q];
         TN_REQUIRE(g.batch == 1 && g.tin == list[0].tin && g.tout == list[0].tout &&
@@ -215,10 +215,14 @@ std::vector<GroupLaunch> gemm_group_stage(tn_batch* b, const std::vector<GemmDes
                    TN_ERR_ARG, "gemm_group: mixed problem types");
         int tile = gemm_choice(c, g).first;
         if (!gemm_tile_ok(tile, g.tin, g.M, g.N, g.K)) tile = gemm_grouped_tile(g.M, g.N);
-        groups[{tile, gemm_k_step(g.tin, g.K)}].push_back(q);
+        if (gemm_wide(tile, g.tin, g.a_kmajor, g.b_kmajor, g.lda, g.ldb)) tile = 7;  // 32x32
+        TN_REQUIRE(!gemm_wide(tile, g.tin, g.a_kmajor, g.b_kmajor, g.lda, g.ldb), TN_ERR_ARG,
+                   "gemm_group: leading dimension too large");
+        TN_REQUIRE(g.K % (128 / (int)dtype_size(g.tin)) == 0, TN_ERR_ARG, "gemm_group: K must be a multiple of 128 bytes");
+        groups[tile].push_back(q);
     }
     for (const auto& kv : groups) {
-        const int tile = kv.first.first, bk = kv.first.second;
+        const int tile = kv.first;
         const int bm = gemm_tile_bm(tile), bn = gemm_tile_bn(tile);
         std::vector<GemmProb> probs;
         std::vector<int> off{0};
@@ -230,7 +234,7 @@ std::vector<GroupLaunch> gemm_group_stage(tn_batch* b, const std::vector<GemmDes
         }
         const GemmProb* dp = stage(b, probs);
         const int* doff = stage(b, off);
-        out.push_back(GroupLaunch{list[0].tin, list[0].tout, list[0].a_kmajor, list[0].b_kmajor, tile, bk, dp, doff,
+        out.push_back(GroupLaunch{list[0].tin, list[0].tout, list[0].a_kmajor, list[0].b_kmajor, tile, dp, doff,
                                   (int)probs.size(), off.back()});
     }
     return out;
@@ -239,8 +243,7 @@ std::vector<GroupLaunch> gemm_group_stage(tn_batch* b, const std::vector<GemmDes
 void gemm_group_launch(tn_batch* b, const std::vector<GroupLaunch>& L)
 {
     for (const GroupLaunch& g : L)
-        TN_HIP(gemm_grouped(g.tin, g.tout, g.akm, g.bkm, g.tile, g.bk, g.probs, g.off, g.nprob, g.total,
-                            b->ctx->stream));
+        TN_HIP(gemm_grouped(g.tin, g.tout, g.akm, g.bkm, g.tile, g.probs, g.off, g.nprob, g.total, b->ctx->stream));
 }
 
 void gemm_group(tn_batch* b, const std::vector<GemmDesc>& list)

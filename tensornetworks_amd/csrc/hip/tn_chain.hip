@@ -2104,6 +2104,17 @@ int tn_gemm_test(tn_ctx* c, int tin, int tout, int akm, int bkm, int M, int N, i
     ABI_END(c)
 }
 
+int tn_gemm_plan(int tin, int akm, int bkm, int M, int N, int K, int64_t lda, int64_t ldb, int batch, int split,
+                 int* tile, int* ksplit, int* wide)
+{
+    if (tin < T_F64 || tin > T_BF16X3 || M <= 0 || N <= 0 || K <= 0 || M % 32 || N % 32 || K % 16 || lda <= 0 ||
+        ldb <= 0 || batch <= 0 || !tile || !ksplit || !wide)
+        return TN_ERR_ARG;
+    gemm_default(tin, M, N, K, batch, split != 0, tile, ksplit);
+    *wide = gemm_wide(*tile, tin, akm != 0, bkm != 0, lda, ldb);
+    return TN_OK;
+}
+
 int tn_copy_bench(tn_ctx* c, int64_t n, double* ms)
 {
     if (!c || n <= 0) return TN_ERR_ARG;

@@ -218,13 +218,20 @@ __device__ __forceinline__ uint32_t lds_offset(const void* p)
 {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
 }
-// 64 lanes copy 16 bytes each from base + off (off per lane) to LDS address
-// dst + 16 * lane (dst uniform)
+// 64 lanes copy 16 bytes each from base + off (off per lane, 32 bits unsigned) to
+// LDS address dst + 16 * lane (dst uniform)
 __device__ __forceinline__ void copy_to_lds(const void* base, uint32_t off, uint32_t dst)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
                  : "s"(dst), "v"(off), "s"(base)
+                 : "memory");
+}
+__device__ __forceinline__ void copy_to_lds(const void* base, uint64_t off, uint32_t dst)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :
+                 : "s"(dst), "v"((const char*)base + off)
                  : "memory");
 }
 // all but the last N copies have arrived and every LDS read has returned
@@ -250,14 +257,14 @@ template <typename TI, int ROWS, int BK, bool KM> struct Stage {
     }
     // byte offset, from the operand's first row and K index of the step, of the
     // unit that slot `slot` holds
-    static __device__ __forceinline__ uint32_t goff(int slot, long ld)
+    static __device__ __forceinline__ uint64_t goff(int slot, long ld)
     {
         if constexpr (KM) {
             const int row = slot / UPK, u = (slot % UPK) ^ rsw(row);
-            return (uint32_t)((row * ld + u * E) * (long)sizeof(TI));
+            return (row * ld + u * E) * (long)sizeof(TI);
         } else {
             const int k = slot / UPR, u = (slot % UPR) ^ ksw(k);
-            return (uint32_t)((k * ld + u * E) * (long)sizeof(TI));
+            return (k * ld + u * E) * (long)sizeof(TI);
         }
     }
     // values between the starts of consecutive K steps
@@ -289,7 +296,11 @@ template <int BM, int BN, int BK, int S, typename TI> constexpr int stage_bytes(
 // Sums over k in increasing order for every tile shape and operand layout (a
 // 16-byte FP64 fragment read, two k per lane, would give another order and only
 // 2-4 % more speed at 3072 x 4096 x 1024).
-template <typename TI, typename TO, int BM, int BN, int BK, int WGM, int WGN, int S, bool AKM, bool BKM>
+//
+// A lane keeps its copies' offsets as 32-bit registers beside a uniform base;
+// WIDE holds them in 64 bits, for operands whose rows lie too far apart (see
+// gemm_wide).
+template <typename TI, typename TO, int BM, int BN, int BK, int WGM, int WGN, int S, bool AKM, bool BKM, bool WIDE>
 __device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __restrict__ B, TO* __restrict__ C,
                                           long lda, long ldb, long ldc, int K, float alpha, int accumulate, int m0,
                                           int n0, TI* __restrict__ sm)
@@ -310,11 +321,12 @@ __device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __
 
     const TI* Ab = AKM ? A + (long)m0 * lda : A + m0;
     const TI* Bb = BKM ? B + (long)n0 * ldb : B + n0;
-    uint32_t off[L];
+    typedef typename std::conditional<WIDE, uint64_t, uint32_t>::type off_t;
+    off_t off[L];
 #pragma unroll
     for (int i = 0; i < L; i++) {
         const int c = wid * L + i;
-        off[i] = c < CA ? SA::goff(c * 64 + lane, lda) : SB::goff((c - CA) * 64 + lane, ldb);
+        off[i] = (off_t)(c < CA ? SA::goff(c * 64 + lane, lda) : SB::goff((c - CA) * 64 + lane, ldb));
     }
     const uint32_t base = __builtin_amdgcn_readfirstlane(lds_offset(sm));
     const long ka = SA::kstep(lda), kb = SB::kstep(ldb);
@@ -405,16 +417,17 @@ __device__ __forceinline__ void tile_of_block(int bid, int ntm, int ntn, int& tm
     tn = local / rows;
 }
 
-template <typename TI, typename TO, int BM, int BN, int BK, int WGM, int WGN, int S, int OCC, bool AKM, bool BKM>
+template <typename TI, typename TO, int BM, int BN, int BK, int WGM, int WGN, int S, int OCC, bool AKM, bool BKM,
+          bool WIDE = false>
 __global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_pipe_k(GemmParams p)
 {
     __shared__ __attribute__((aligned(1024))) TI sm[stage_bytes<BM, BN, BK, S, TI>() / sizeof(TI)];
     int tm, tn;
     tile_of_block(blockIdx.x, p.M / BM, p.N / BN, tm, tn);
     const long bz = blockIdx.y;
-    pipe_tile<TI, TO, BM, BN, BK, WGM, WGN, S, AKM, BKM>((const TI*)p.A + bz * p.sA, (const TI*)p.B + bz * p.sB,
-                                                         (TO*)p.C + bz * p.sC, p.lda, p.ldb, p.ldc, p.K, p.alpha,
-                                                         p.accumulate, tm * BM, tn * BN, sm);
+    pipe_tile<TI, TO, BM, BN, BK, WGM, WGN, S, AKM, BKM, WIDE>(
+        (const TI*)p.A + bz * p.sA, (const TI*)p.B + bz * p.sB, (TO*)p.C + bz * p.sC, p.lda, p.ldb, p.ldc, p.K,
+        p.alpha, p.accumulate, tm * BM, tn * BN, sm);
 }
 
 // Split-product LDS layout for BK = 32: rows of 64 bytes without padding,
@@ -779,8 +792,9 @@ __global__ void __launch_bounds__(256, OCC) gemm_grouped_k(const GemmProb* __res
         const int local = t - off[lo], ntn = q.N / BN;
         const int tm = local / ntn, tn = local - tm * ntn;
         __syncthreads();  // LDS of the previous tile is free
-        pipe_tile<TI, TO, BM, BN, BK, WGM, WGN, S, AKM, BKM>((const TI*)q.A, (const TI*)q.B, (TO*)q.C, q.lda, q.ldb,
-                                                             q.ldc, q.K, q.alpha, q.accumulate, tm * BM, tn * BN, sm);
+        pipe_tile<TI, TO, BM, BN, BK, WGM, WGN, S, AKM, BKM, false>((const TI*)q.A, (const TI*)q.B, (TO*)q.C, q.lda,
+                                                                    q.ldb, q.ldc, q.K, q.alpha, q.accumulate, tm * BM,
+                                                                    tn * BN, sm);
     }
 }
 
@@ -824,6 +838,18 @@ static hipError_t launch_bf16(int code, const GemmParams& p, int batch, hipStrea
     return hipGetLastError();
 }
 
+// Whether the rows of one tile (K-major: its BM or BN rows, else the rows of a K
+// step) span more than 32-bit byte offsets reach: with 128 rows of FP64 from a
+// leading dimension of 4.2 million on.  Such a problem takes the 32x32 tile with
+// 64-bit offsets (the same sums: every tile adds over k in order).
+bool gemm_wide(int code, int tin, bool akm, bool bkm, long lda, long ldb)
+{
+    if ((tin != T_F64 && tin != T_F32) || code < 1 || code > kNumTiles) return false;
+    const long es = tin == T_F64 ? 8 : 4, bk = 128 / es;
+    auto far = [&](bool km, int rows, long ld) { return ld > 0 && (km ? rows : bk) * es > (1L << 32) / ld; };
+    return far(akm, kTiles[code - 1].bm, lda) || far(bkm, kTiles[code - 1].bn, ldb);
+}
+
 // FP64 / FP32: waves, LDS stages and workgroups per CU of every tile.  The
 // small tiles have little work between barriers and take four stages; the
 // "deep" codes take one stage more than their plain form.
@@ -836,14 +862,18 @@ template <typename TI, typename TO, bool AKM, bool BKM>
 static hipError_t launch_pipe(int code, const GemmParams& p, int batch, hipStream_t s)
 {
     constexpr int BK = 128 / sizeof(TI);
+    const dim3 grid32((p.M / 32) * (p.N / 32), batch);
     if (p.K % BK) {
         // FP32 with K an odd multiple of 16: the smallest tile on 64-byte rows
         if constexpr (std::is_same<TI, float>::value) {
-            const dim3 grid((p.M / 32) * (p.N / 32), batch);
-            gemm_pipe_k<TI, TO, 32, 32, 16, 2, 2, 4, 4, AKM, BKM><<<grid, 256, 0, s>>>(p);
+            gemm_pipe_k<TI, TO, 32, 32, 16, 2, 2, 4, 4, AKM, BKM, true><<<grid32, 256, 0, s>>>(p);
             return hipGetLastError();
         }
         return hipErrorInvalidValue;
+    }
+    if (gemm_wide(code + 1, sizeof(TI) == 8 ? T_F64 : T_F32, AKM, BKM, p.lda, p.ldb)) {
+        gemm_pipe_k<TI, TO, 32, 32, BK, 2, 2, 4, 4, AKM, BKM, true><<<grid32, 256, 0, s>>>(p);
+        return hipGetLastError();
     }
     const TileCfg& t = kTiles[code];
     const dim3 grid((p.M / t.bm) * (p.N / t.bn), batch);
@@ -858,11 +888,9 @@ static hipError_t launch_pipe(int code, const GemmParams& p, int batch, hipStrea
 }
 
 template <typename TI, typename TO, bool AKM, bool BKM>
-static hipError_t launch_grouped(int code, int bk, const GemmProb* probs, const int* off, int nprob, int grid,
-                                 hipStream_t s)
+static hipError_t launch_grouped(int code, const GemmProb* probs, const int* off, int nprob, int grid, hipStream_t s)
 {
     constexpr int BK = 128 / sizeof(TI);
-    if (bk != BK) return hipErrorInvalidValue;
     switch (code) {
 #define PIPE_CASE(c, bm, bn, wm, wn, st, occ)                                                                       \
     case c:                                                                                                         \
@@ -876,12 +904,12 @@ static hipError_t launch_grouped(int code, int bk, const GemmProb* probs, const 
 }
 
 template <bool AKM, bool BKM>
-static hipError_t grouped_layout(int tin, int tout, int code, int bk, const GemmProb* probs, const int* off,
-                                 int nprob, int grid, hipStream_t s)
+static hipError_t grouped_layout(int tin, int tout, int code, const GemmProb* probs, const int* off, int nprob,
+                                 int grid, hipStream_t s)
 {
-    if (tin == T_F64 && tout == T_F64) return launch_grouped<double, double, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
-    if (tin == T_F32 && tout == T_F32) return launch_grouped<float, float, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
-    if (tin == T_F32 && tout == T_F64) return launch_grouped<float, double, AKM, BKM>(code, bk, probs, off, nprob, grid, s);
+    if (tin == T_F64 && tout == T_F64) return launch_grouped<double, double, AKM, BKM>(code, probs, off, nprob, grid, s);
+    if (tin == T_F32 && tout == T_F32) return launch_grouped<float, float, AKM, BKM>(code, probs, off, nprob, grid, s);
+    if (tin == T_F32 && tout == T_F64) return launch_grouped<float, double, AKM, BKM>(code, probs, off, nprob, grid, s);
     return hipErrorInvalidValue;
 }
 
@@ -958,16 +986,16 @@ int gemm_k_step(int tin, int K)
     return K % 64 == 0 ? 64 : 32;
 }
 
-hipError_t gemm_grouped(int tin, int tout, bool akm, bool bkm, int tile, int bk, const GemmProb* probs,
-                        const int* off, int nprob, int total_tiles, hipStream_t s)
+hipError_t gemm_grouped(int tin, int tout, bool akm, bool bkm, int tile, const GemmProb* probs, const int* off,
+                         int nprob, int total_tiles, hipStream_t s)
 {
     if (nprob <= 0 || total_tiles <= 0) return hipSuccess;
     if (tile < 1 || tile > kNumTiles || kTiles[tile - 1].x3only) return hipErrorInvalidValue;
     const int grid = total_tiles < 2048 ? total_tiles : 2048;
-    if (akm && bkm) return grouped_layout<true, true>(tin, tout, tile - 1, bk, probs, off, nprob, grid, s);
-    if (akm && !bkm) return grouped_layout<true, false>(tin, tout, tile - 1, bk, probs, off, nprob, grid, s);
-    if (!akm && !bkm) return grouped_layout<false, false>(tin, tout, tile - 1, bk, probs, off, nprob, grid, s);
-    return grouped_layout<false, true>(tin, tout, tile - 1, bk, probs, off, nprob, grid, s);
+    if (akm && bkm) return grouped_layout<true, true>(tin, tout, tile - 1, probs, off, nprob, grid, s);
+    if (akm && !bkm) return grouped_layout<true, false>(tin, tout, tile - 1, probs, off, nprob, grid, s);
+    if (!akm && !bkm) return grouped_layout<false, false>(tin, tout, tile - 1, probs, off, nprob, grid, s);
+    return grouped_layout<false, true>(tin, tout, tile - 1, probs, off, nprob, grid, s);
 }
 
 // bf16 and grouped launches: pick the largest tile that divides the problem and still

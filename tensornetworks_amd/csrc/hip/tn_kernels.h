@@ -53,10 +53,10 @@ struct GemmProb {
 };
 // One persistent launch over all output tiles of nprob problems; off (device,
 // nprob+1) is the prefix sum of per-problem tile counts (M/BM)*(N/BN) for the
-// tile code; bk the K step (gemm_k_step).  M, N of every problem must be
-// multiples of the tile, K of bk.
-hipError_t gemm_grouped(int tin, int tout, bool akm, bool bkm, int tile, int bk, const GemmProb* probs,
-                        const int* off, int nprob, int total_tiles, hipStream_t s);
+// tile code.  FP64 or FP32 operands within 32-bit offsets (not gemm_wide); M, N
+// of every problem must be multiples of the tile, K of 128 bytes.
+hipError_t gemm_grouped(int tin, int tout, bool akm, bool bkm, int tile, const GemmProb* probs, const int* off,
+                        int nprob, int total_tiles, hipStream_t s);
 int gemm_tile_bm(int code);
 // tile code usable for an M x N x K problem of input type tin
 bool gemm_tile_ok(int code, int tin, int M, int N, int K);
@@ -66,6 +66,9 @@ void gemm_default(int tin, int M, int N, int K, int batch, bool split, int* tile
 // built-in tile code of one problem of a grouped launch
 int gemm_grouped_tile(int M, int N);
 int gemm_k_step(int tin, int K);
+// FP64 / FP32 operands too long for the tile's 32-bit copy offsets: gemm takes its
+// 32x32 tile with 64-bit ones
+bool gemm_wide(int code, int tin, bool akm, bool bkm, long lda, long ldb);
 // split-K epilogue: C[i*ldc + j] = (accumulate ? C : 0) + sum_{z<ks} W[z][i][j]
 // (W: ks x M x N of type tacc, T_F64 or T_F32)
 hipError_t splitk_reduce(int tacc, const void* W, int ks, int M, int N, int tout, void* C, long ldc, int accumulate,

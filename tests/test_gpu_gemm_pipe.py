@@ -82,3 +82,19 @@ def test_split_bf16_built_in_tile(ctx, M, N, K):
                           0, ksplit)[0]
         # 24-bit operands, six products and one FP32 rounding per k
         assert np.all(np.abs(C - ref) <= (7 * K + 8) * 2.0 ** -24 * size)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 4, 7])
+def test_rows_too_far_apart_for_32_bit_offsets(ctx, tile):
+    # 128 rows of 34 MB: the last row of a 128-row tile starts 4.3e9 bytes after its
+    # first.  Only the two ends of the rows are not zero, so the sums (in increasing
+    # k) are those of the ends alone, bit for bit.
+    M, K = 128, 4259840
+    rng = np.random.default_rng(3)
+    ends = rng.uniform(-1.0, 1.0, (M, 64))
+    A = np.zeros((M, K))  # pages that are never written stay unallocated
+    A[:, :32] = ends[:, :32]
+    A[:, -32:] = ends[:, 32:]
+    C = ctx.gemm_test(A, A, tn.TN_FP64, tn.TN_FP64, True, True, M, M, K, 1, tile)[0]
+    ref = ctx.gemm_test(ends, ends, tn.TN_FP64, tn.TN_FP64, True, True, M, M, 64, 1, 7)[0]
+    assert np.array_equal(C, ref)
