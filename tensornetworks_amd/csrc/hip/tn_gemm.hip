@@ -219,18 +219,24 @@ __device__ __forceinline__ uint32_t lds_offset(const void* p)
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
 }
 // 64 lanes copy 16 bytes each from base + off (off per lane, 32 bits unsigned) to
-// LDS address dst + 16 * lane (dst uniform)
+// LDS address dst + 16 * lane (dst uniform).  The instruction takes dst from M0,
+// which the compiler owns (it is no register that inline assembly may declare as
+// clobbered): its value is put back.
 __device__ __forceinline__ void copy_to_lds(const void* base, uint32_t off, uint32_t dst)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
+    uint32_t m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
+                 : "=&s"(m0)
                  : "s"(dst), "v"(off), "s"(base)
                  : "memory");
 }
 __device__ __forceinline__ void copy_to_lds(const void* base, uint64_t off, uint32_t dst)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-                 :
+    uint32_t m0;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
+                 "global_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(m0)
                  : "s"(dst), "v"((const char*)base + off)
                  : "memory");
 }
@@ -359,6 +365,7 @@ __device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __
         if (t + S - 2 < nk) wait_copies<(S - 2) * L>();
         else wait_copies<0>();
         __builtin_amdgcn_s_barrier();
+        asm volatile("" : : : "memory");  // no LDS read of this step moves above the barrier
         if (t + S - 1 < nk) issue(st == 0 ? S - 1 : st - 1);
         const TI* As = sm + st * STG;
         const TI* Bs = As + BM * BK;
@@ -376,7 +383,7 @@ __device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __
                     for (int j = 0; j < FN; j++) acc[i][j] = mma(a[i], b[j], acc[i][j]);
             }
         __builtin_amdgcn_s_setprio(0);
-        asm volatile("" : : : "memory");
+        asm volatile("" : : : "memory");  // nor below the next one's wait
         st = st + 1 == S ? 0 : st + 1;
     }
     wait_copies<0>();
