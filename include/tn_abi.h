@@ -226,8 +226,10 @@ typedef struct tn_sweep_stats {
     int64_t n_env;             /* environment updates */
     int64_t n_svd;             /* bond SVDs */
     double heff_flops;         /* algorithmic flops of all Heff applies */
-    double heff_ms;            /* device time of all Heff applies (HIP events) */
-    double heff_gemm_ms;       /* device time of the two GEMM stages only */
+    double heff_ms;            /* device time of the n_matvec Heff applies (HIP events) */
+    double heff_gemm_ms;       /* device time of the two GEMM stages only; of an FP64 apply
+                                  that runs as one launch (left bond up to 32, right bond up
+                                  to 64) all of it, the MPO stage included */
     double heff_gemm_flops;    /* flops of the two GEMM stages as launched (identity
                                   environment channels excluded) */
     double env_flops, env_ms;
@@ -323,6 +325,10 @@ int tn_gemm_test(tn_ctx* ctx, int tin, int tout, int a_kmajor, int b_kmajor, int
  * so that the product runs in the 32x32 tile with 64-bit ones. */
 int tn_gemm_plan(int tin, int a_kmajor, int b_kmajor, int M, int N, int K, int64_t lda, int64_t ldb, int batch,
                  int split, int* tile, int* ksplit, int* wide);
+
+/* Heff applies whose device time has gone into a tn_sweep_stats of this context's
+ * chains so far (one per counted apply with time_heff = 1). */
+int tn_ctx_heff_timings(tn_ctx* ctx, int64_t* n);
 
 /* ---- batched chains (no reference counterpart: the reference sweeps one
  * MPS at a time) ----

@@ -108,6 +108,7 @@ def _load():
         "tn_svd": (i, [v, i, i, _dp, _dp, _dp, _dp]),
         "tn_svcompress_rank": (i, [i, _dp, i, d, _dp, _dp]),
         "tn_gemm_test": (i, [v, i, i, i, i, i, i, i, i, _dp, _dp, _dp, i, i]),
+        "tn_ctx_heff_timings": (i, [v, ctypes.POINTER(ctypes.c_int64)]),
         "tn_gemm_plan": (i, [i, i, i, i, i, i, ctypes.c_int64, ctypes.c_int64, i, i, _ip, _ip, _ip]),
         "tn_cholqr_test": (i, [v, i, i, _dp, ctypes.c_double, _dp, _dp, _ip, i]),
         "tn_ctx_set_autotune": (i, [v, i]),
@@ -276,6 +277,12 @@ class Context:
         ms = ctypes.c_double(0.0)
         self.check(lib.tn_copy_bench(self.h, int(n), ctypes.byref(ms)), "tn_copy_bench")
         return ms.value
+
+    def heff_timings(self):
+        """Number of Heff applies whose device time has gone into a SweepStats."""
+        n = ctypes.c_int64()
+        self.check(lib.tn_ctx_heff_timings(self.h, ctypes.byref(n)), "tn_ctx_heff_timings")
+        return n.value
 
     def tune_report(self):
         buf = ctypes.create_string_buffer(1 << 16)

@@ -169,6 +169,7 @@ static void heff_timing_flush(tn_ctx* c, int set)
     if (!st) return;
     heff_timing_read(c, set, &st->heff_gemm_ms, &st->heff_ms);
     c->heff_pending[set] = nullptr;
+    c->n_heff_timed++;
 }
 void heff_timing_flush(tn_ctx* c)
 {
@@ -192,6 +193,15 @@ void heff_cb(tn_ctx* c, const void* vop, const double* x, double* y)
     heff_apply(c, hc->op, x, y, timed);
     if (timed) c->heff_pending[c->ev_set] = hc->st;
     heff_count(hc, 1);
+}
+
+// Takes back the counts and the times of the solve's applies that were queued ahead
+// and not used: at most the last one, whose events have not been read yet.
+static void heff_unused(tn_ctx* c, const HeffCall* hc, int n)
+{
+    if (n == 0) return;
+    heff_count(hc, -n);
+    if (hc->st && hc->timed) c->heff_pending[c->ev_set] = nullptr;
 }
 
 // Identity channels of the environments of site i: for the first and the last
@@ -310,7 +320,7 @@ void eigensolve(tn_chain* ch, int i, const tn_sweep_opts& o, tn_sweep_stats* st,
             if (st) st->n_precond_fallback++;
             LanczosResult r = lanczos(c, heff_cb, &hc, N, ch->A[i], o.eig_tol, o.max_krylov, o.max_restarts, 0.0,
                                       o.reorth == 1, unit_roundoff(TN_FP64), true);
-            heff_count(&hc, -r.n_unused);
+            heff_unused(c, &hc, r.n_unused);
             if (st) st->n_full_reorth += r.n_full;
             *e0 = r.e0;
             *e1 = r.e1;
@@ -325,7 +335,7 @@ void eigensolve(tn_chain* ch, int i, const tn_sweep_opts& o, tn_sweep_stats* st,
     const double rel = refining ? (o.precision == TN_BF16 ? 4e-3 : 4e-7) : 0.0;
     LanczosResult r = lanczos(c, heff_cb, &hc, N, ch->A[i], o.eig_tol, o.max_krylov, o.max_restarts, rel,
                               o.reorth == 1, unit_roundoff(o.precision), true);
-    heff_count(&hc, -r.n_unused);
+    heff_unused(c, &hc, r.n_unused);
     if (st) st->n_full_reorth += r.n_full;
     if (refining) {
         // polish the reduced-precision Ritz vector with a more accurate operator
@@ -333,7 +343,7 @@ void eigensolve(tn_chain* ch, int i, const tn_sweep_opts& o, tn_sweep_stats* st,
         hr.op = make_heff(ch, i, o.refine_precision, o.gemm_tile, wl, wr);
         LanczosResult r2 = lanczos(c, heff_cb, &hr, N, ch->A[i], o.refine_tol, o.max_krylov, o.max_restarts, 0.0,
                                    o.reorth == 1, unit_roundoff(o.refine_precision), true);
-        heff_count(&hr, -r2.n_unused);
+        heff_unused(c, &hr, r2.n_unused);
         if (st) st->n_full_reorth += r2.n_full;
         r.e0 = r2.e0;
         r.e1 = r2.e1;
@@ -1942,7 +1952,7 @@ int tn_chain_sweep2(tn_chain* ch, int dir, int Dmax, double eps_sv, const tn_swe
         double tl = now_ms();
         LanczosResult r = lanczos(c, heff_cb, &hc, N, ch->theta.as<double>(), o.eig_tol, o.max_krylov, o.max_restarts,
                                   0.0, o.reorth == 1, unit_roundoff(o.precision), true);
-        heff_count(&hc, -r.n_unused);
+        heff_unused(c, &hc, r.n_unused);
         if (st) st->n_full_reorth += r.n_full;
         if (o.refine && o.refine_precision < o.precision) {
             HeffCall h64 = hc;
@@ -1951,7 +1961,7 @@ int tn_chain_sweep2(tn_chain* ch, int dir, int Dmax, double eps_sv, const tn_swe
             h64.op.Rlo = lo_right(ch, o.refine_precision, j);
             LanczosResult r2 = lanczos(c, heff_cb, &h64, N, ch->theta.as<double>(), o.refine_tol, o.max_krylov,
                                        o.max_restarts, 0.0, o.reorth == 1, unit_roundoff(o.refine_precision), true);
-            heff_count(&h64, -r2.n_unused);
+            heff_unused(c, &h64, r2.n_unused);
             if (st) st->n_full_reorth += r2.n_full;
             r.e0 = r2.e0;
             r.e1 = r2.e1;
@@ -2112,6 +2122,13 @@ int tn_gemm_plan(int tin, int akm, int bkm, int M, int N, int K, int64_t lda, in
         return TN_ERR_ARG;
     gemm_default(tin, M, N, K, batch, split != 0, tile, ksplit);
     *wide = gemm_wide(*tile, tin, akm != 0, bkm != 0, lda, ldb);
+    return TN_OK;
+}
+
+int tn_ctx_heff_timings(tn_ctx* c, int64_t* n)
+{
+    if (!c || !n) return TN_ERR_ARG;
+    *n = c->n_heff_timed;
     return TN_OK;
 }
 

@@ -106,6 +106,7 @@ struct tn_ctx {
     void* noalloc = nullptr;
     // stats whose Heff event timings are recorded but not yet read
     tn_sweep_stats* heff_pending[2] = {nullptr, nullptr};  // per event set
+    long n_heff_timed = 0;  // event timings read into stats so far
     // nonzero: the next heff_apply first scales its input in place by this
     // factor (within its first pass over it) and resets it; set by the Lanczos
     // driver right before the apply of a new basis vector

@@ -63,3 +63,27 @@ def test_capped_solve_matches_numpy(ctx, d, D1, D2, steps):
     assert abs(ev[0] - ref) <= tol, (ev[0], ref)
     assert abs(np.linalg.norm(x) - 1.0) <= 1e-13
     assert abs(x @ apply(x) - ev[0]) <= tol
+
+
+# one site in one launch, three kernels per apply; one- and two-site sweeps; refined
+@pytest.mark.parametrize("L,d,D,kw", [(4, 2, 4, {}), (6, 3, 40, {}), (4, 2, 4, {"reorth": 1}),
+                                      (6, 2, 8, {"precision": tn.TN_FP32, "refine": 1, "refine_precision": tn.TN_FP64,
+                                                 "refine_tol": 1e-12})])
+@pytest.mark.parametrize("two", [False, True])
+def test_timed_applies_are_the_counted_ones(ctx, L, d, D, kw, two):
+    # an apply that was queued ahead of the convergence test and not used goes
+    # neither into the counts nor into the times
+    opts = tn.SweepOpts.default(eig_tol=1e-11, **kw)
+    ch = tn.Chain(ctx, tn.xxz_mpo(L, 0.5 * (d - 1)), D)
+    ch.initialize(1, 5)
+    ch.normalize_qr(1)
+    ch.load_caches(opts)
+    st = tn.SweepStats()
+    before = ctx.heff_timings()
+    for direction in (0, 1):
+        if two:
+            ch.sweep2(direction, D, 0.0, opts, st)
+        else:
+            ch.sweep(direction, opts, st)
+    assert st.n_matvec > 0 and st.heff_ms > 0
+    assert ctx.heff_timings() - before == st.n_matvec
