@@ -409,13 +409,15 @@ __device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __
 }
 
 // XCD-aware tile order: consecutive block ids land on different XCDs, so each
-// XCD gets a contiguous range of tiles, and inside it 8 tile rows at a time go
+// XCD gets a contiguous range of tiles (also when their number is no multiple of
+// 8: FP32 992 x 2976 x 3968 in 32x32, 2883 tiles, 280 us in launch order, 264 so;
+// 1504 x 4512 x 6016 870 and 821), and inside it 8 tile rows at a time go
 // column by column (tiles resident together share 8 row blocks of A and a few
 // column blocks of B)
 __device__ __forceinline__ void tile_of_block(int bid, int ntm, int ntn, int& tm, int& tn)
 {
-    const int nblk = ntm * ntn;
-    if ((nblk & 7) == 0) bid = (bid & 7) * (nblk >> 3) + (bid >> 3);
+    const int nblk = ntm * ntn, xcd = bid & 7, rest = nblk & 7;
+    bid = xcd * (nblk >> 3) + (xcd < rest ? xcd : rest) + (bid >> 3);
     constexpr int GM = 8;
     const int gsz = GM * ntn, g = bid / gsz, first = g * GM;
     const int rows = ntm - first < GM ? ntm - first : GM;
@@ -857,13 +859,25 @@ bool gemm_wide(int code, int tin, bool akm, bool bkm, long lda, long ldb)
     return far(akm, kTiles[code - 1].bm, lda) || far(bkm, kTiles[code - 1].bn, ldb);
 }
 
-// FP64 / FP32: waves, LDS stages and workgroups per CU of every tile.  The
-// small tiles have little work between barriers and take four stages; the
-// "deep" codes take one stage more than their plain form.
-#define PIPE_TILES(X)                                                                                       \
-    X(0, 128, 128, 2, 2, 2, 2) X(1, 128, 64, 2, 2, 2, 3) X(2, 64, 128, 2, 2, 2, 3) X(3, 64, 64, 2, 2, 2, 4) \
-    X(4, 32, 64, 1, 4, 4, 3) X(5, 64, 32, 2, 2, 4, 3) X(6, 32, 32, 2, 2, 4, 4) X(7, 128, 128, 2, 2, 3, 1)   \
-    X(8, 128, 64, 2, 2, 3, 2) X(9, 64, 128, 2, 2, 3, 2)
+// FP64 / FP32: K values of a step, waves, LDS stages and workgroups per CU of
+// every tile.  The small FP64 tiles have little work between barriers and take
+// four stages; the "deep" codes take one stage more than their plain form.
+// FP32 tiles want workgroups on the CU more than stages.  Operands from memory
+// (a dozen buffers in turn), 4512 x 6016 x 1504, in 32x64: 805 us with three
+// workgroups of four stages, 760 with six of two (register-staged loop 783); 1504 x
+// 4512 x 6016 in 32x32: 888 with four of four stages, 810 with eight of two
+// (846).  3072 x 4096 x 1024 in 128x128: 199 us with two workgroups on 128-byte
+// rows, 190 with three on 64-byte rows (195).
+#define PIPE_F64(X)                                                                                       \
+    X(0, 128, 128, 16, 2, 2, 2, 2) X(1, 128, 64, 16, 2, 2, 2, 3) X(2, 64, 128, 16, 2, 2, 2, 3)            \
+    X(3, 64, 64, 16, 2, 2, 2, 4) X(4, 32, 64, 16, 1, 4, 4, 3) X(5, 64, 32, 16, 2, 2, 4, 3)                \
+    X(6, 32, 32, 16, 2, 2, 4, 4) X(7, 128, 128, 16, 2, 2, 3, 1) X(8, 128, 64, 16, 2, 2, 3, 2)             \
+    X(9, 64, 128, 16, 2, 2, 3, 2)
+#define PIPE_F32(X)                                                                                       \
+    X(0, 128, 128, 16, 2, 2, 2, 3) X(1, 128, 64, 32, 2, 2, 2, 3) X(2, 64, 128, 32, 2, 2, 2, 3)            \
+    X(3, 64, 64, 32, 2, 2, 2, 4) X(4, 32, 64, 32, 1, 4, 2, 6) X(5, 64, 32, 32, 2, 2, 2, 6)                \
+    X(6, 32, 32, 32, 2, 2, 2, 8) X(7, 128, 128, 32, 2, 2, 3, 1) X(8, 128, 64, 32, 2, 2, 3, 2)             \
+    X(9, 64, 128, 32, 2, 2, 3, 2)
 
 template <typename TI, typename TO, bool AKM, bool BKM>
 static hipError_t launch_pipe(int code, const GemmParams& p, int batch, hipStream_t s)
@@ -884,29 +898,53 @@ static hipError_t launch_pipe(int code, const GemmParams& p, int batch, hipStrea
     }
     const TileCfg& t = kTiles[code];
     const dim3 grid((p.M / t.bm) * (p.N / t.bn), batch);
-    switch (code) {
-#define PIPE_CASE(c, bm, bn, wm, wn, st, occ)                                                      \
-    case c: gemm_pipe_k<TI, TO, bm, bn, BK, wm, wn, st, occ, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-        PIPE_TILES(PIPE_CASE)
-#undef PIPE_CASE
-    default: return hipErrorInvalidValue;
+    if constexpr (std::is_same<TI, float>::value) {
+        // FP32 128x64 and 64x128: three workgroups per CU on 128-byte rows while that
+        // takes all of them at once (1024 x 3072 x 4096 in two K halves, 64x128: 197
+        // us, four on 64-byte rows 201), else four on 64-byte rows (1984 x 3968 x 992,
+        // 961 workgroups: 138 -> 132 us; 3072 x 4096 x 1024, 128x64: 199 -> 193)
+        if ((long)grid.x * batch > 768 && (code == 1 || code == 2)) {
+            if (code == 1) gemm_pipe_k<TI, TO, 128, 64, 16, 2, 2, 2, 4, AKM, BKM><<<grid, 256, 0, s>>>(p);
+            else gemm_pipe_k<TI, TO, 64, 128, 16, 2, 2, 2, 4, AKM, BKM><<<grid, 256, 0, s>>>(p);
+            return hipGetLastError();
+        }
     }
+#define PIPE_CASE(c, bm, bn, bk, wm, wn, st, occ)                                                  \
+    case c: gemm_pipe_k<TI, TO, bm, bn, bk, wm, wn, st, occ, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    if constexpr (std::is_same<TI, double>::value) {
+        switch (code) {
+            PIPE_F64(PIPE_CASE)
+        default: return hipErrorInvalidValue;
+        }
+    } else {
+        switch (code) {
+            PIPE_F32(PIPE_CASE)
+        default: return hipErrorInvalidValue;
+        }
+    }
+#undef PIPE_CASE
     return hipGetLastError();
 }
 
 template <typename TI, typename TO, bool AKM, bool BKM>
 static hipError_t launch_grouped(int code, const GemmProb* probs, const int* off, int nprob, int grid, hipStream_t s)
 {
-    constexpr int BK = 128 / sizeof(TI);
-    switch (code) {
-#define PIPE_CASE(c, bm, bn, wm, wn, st, occ)                                                                       \
+#define PIPE_CASE(c, bm, bn, bk, wm, wn, st, occ)                                                                  \
     case c:                                                                                                         \
-        gemm_grouped_k<TI, TO, bm, bn, BK, wm, wn, st, occ, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); \
+        gemm_grouped_k<TI, TO, bm, bn, bk, wm, wn, st, occ, AKM, BKM><<<grid, 256, 0, s>>>(probs, off, nprob); \
         break;
-        PIPE_TILES(PIPE_CASE)
-#undef PIPE_CASE
-    default: return hipErrorInvalidValue;
+    if constexpr (std::is_same<TI, double>::value) {
+        switch (code) {
+            PIPE_F64(PIPE_CASE)
+        default: return hipErrorInvalidValue;
+        }
+    } else {
+        switch (code) {
+            PIPE_F32(PIPE_CASE)
+        default: return hipErrorInvalidValue;
+        }
     }
+#undef PIPE_CASE
     return hipGetLastError();
 }
 
@@ -1032,8 +1070,8 @@ struct StepCost { int code; float busy, alone; };
 static const StepCost kCostF64[] = {  // 128x64, 64x128, 64x64, 32x64, 64x32, 32x32
     {1, 0.933f, 1.05f}, {2, 0.933f, 1.05f}, {3, 0.485f, 0.53f}, {4, 0.259f, 0.30f}, {5, 0.259f, 0.30f},
     {6, 0.138f, 0.235f}};
-static const StepCost kCostF32[] = {
-    {1, 1.016f, 1.15f}, {2, 1.016f, 1.15f}, {3, 0.608f, 0.70f}, {4, 0.353f, 0.45f}, {5, 0.353f, 0.45f},
+static const StepCost kCostF32[] = {  // and 128x128
+    {0, 1.95f, 2.40f}, {1, 1.016f, 1.15f}, {2, 1.016f, 1.15f}, {3, 0.608f, 0.70f}, {4, 0.353f, 0.45f}, {5, 0.353f, 0.45f},
     {6, 0.205f, 0.355f}};
 // split bf16 (steps of 32): 128x128 .. 32x32, 96x128, 128x96, 192x256, 256x192,
 // 192x128, 128x192.  1024 x 3072 x 4096: 208 us in the 128x64 tiles of the
@@ -1049,7 +1087,7 @@ void gemm_default(int tin, int M, int N, int K, int batch, bool split, int* tile
 {
     *ksplit = 1;
     const StepCost* cost = tin == T_F64 ? kCostF64 : (tin == T_F32 ? kCostF32 : kCostX3);
-    const int ncost = tin == T_BF16X3 ? (int)(sizeof(kCostX3) / sizeof(kCostX3[0])) : 6;
+    const int ncost = tin == T_BF16X3 ? (int)(sizeof(kCostX3) / sizeof(kCostX3[0])) : (tin == T_F32 ? 7 : 6);
     if (tin == T_BF16) {
         *tile = choose_tile(M, N, batch) + 1;
         return;

@@ -37,6 +37,15 @@ def test_every_tile_gives_the_same_bits(ctx, tin, akm, bkm, K):
         assert np.array_equal(_product(ctx, tin, akm, bkm, M, N, K, tile), ref), tile
 
 
+# numbers of tiles that are no multiple of the eight XCDs (117, 35, 961), and more
+# than 768 of 128x64 and 64x128, whose FP32 form then changes
+@pytest.mark.parametrize("tin", [tn.TN_FP64, tn.TN_FP32])
+@pytest.mark.parametrize("M,N,tile", [(288, 416, 7), (320, 448, 4), (1984, 3968, 3), (3968, 1984, 2), (3968, 3968, 1)])
+def test_any_number_of_tiles(ctx, tin, M, N, tile):
+    C = _product(ctx, tin, True, True, M, N, 96, tile)
+    assert np.array_equal(C, _product(ctx, tin, True, True, M, N, 96, 7 if tile != 7 else 0))
+
+
 @pytest.mark.parametrize("tin", [tn.TN_FP64, tn.TN_FP32])
 @pytest.mark.parametrize("akm,bkm", [(True, True), (True, False), (False, False), (False, True)])
 @pytest.mark.parametrize("M,N,K", [(32, 32, 16), (64, 32, 48), (96, 160, 112), (128, 128, 16)])
