@@ -19,8 +19,11 @@ namespace tn {
 // workgroups per CU exist.  Before (one workgroup walking all outputs with the
 // table in global memory) and after: transposed FP64 form, D = 8: 11.5 and
 // 4.1 us; 320 x 224, d = 2: 15.5 and 7.5 us; D = 256, d = 3: 21.7 and 6.9 us;
-// FP32 512 x 448, d = 3: 16.5 and 10.7 us; plain FP64 form, D = 256, d = 2: 6.9
-// and 6.4 us.  Sums keep the table's order.
+// FP32 512 x 448, d = 3: 16.5 and 8.9 us; plain FP64 form, D = 256, d = 2: 6.9
+// and 6.4 us.  What comes from LDS is the same for every lane and goes back to
+// scalar registers, so that the eight addresses of an entry are one scalar sum
+// each (with the offsets left in vector registers FP32 D = 2048, d = 3 took 160 us,
+// D = 1500 78; now 114 and 63).  Sums keep the table's order.
 #define MIX_MAXO 64
 #define MIX_MAXE 512
 template <typename V> struct MixLds {
@@ -30,9 +33,26 @@ template <typename V> struct MixLds {
 };
 // STG: the table's copy in LDS (nout <= MIX_MAXO, nnz <= MIX_MAXE), else global
 template <typename V, bool STG> struct MixView {
-    const int *optr, *osel, *esel;
-    const long *ooff, *eoff;
-    const V* eval;
+    const int *optr_, *osel_, *esel_;
+    const long *ooff_, *eoff_;
+    const V* eval_;
+    static __device__ __forceinline__ int uni(int v)
+    {
+        if constexpr (STG) return __builtin_amdgcn_readfirstlane(v);
+        else return v;
+    }
+    static __device__ __forceinline__ long uni(long v)
+    {
+        if constexpr (STG)
+            return (long)(uint32_t)uni((int)v) | ((long)uni((int)(v >> 32)) << 32);
+        else return v;
+    }
+    __device__ __forceinline__ int optr(int o) const { return uni(optr_[o]); }
+    __device__ __forceinline__ int osel(int o) const { return uni(osel_[o]); }
+    __device__ __forceinline__ int esel(int e) const { return uni(esel_[e]); }
+    __device__ __forceinline__ long ooff(int o) const { return uni(ooff_[o]); }
+    __device__ __forceinline__ long eoff(int e) const { return uni(eoff_[e]); }
+    __device__ __forceinline__ V eval(int e) const { return eval_[e]; }
 };
 template <typename V>
 __device__ __forceinline__ const V* mix_values(const MixTable& t)
@@ -83,12 +103,12 @@ __global__ void __launch_bounds__(256) wmix_k(const TI* __restrict__ in, long is
     const TI* ip = in + x * isx + b;
     TO* op = out + x * osx + b;
     for (int o = blockIdx.z; o < t.nout; o += gridDim.z) {
-        const int e0 = m.optr[o], e1 = m.optr[o + 1];
+        const int e0 = m.optr(o), e1 = m.optr(o + 1);
         acc_t acc = 0;
 #pragma unroll 4
-        for (int e = e0; e < e1; e++) acc += m.eval[e] * to_acc<acc_t>(ip[m.eoff[e]]);
-        if constexpr (std::is_same<TI, double>::value) op[m.ooff[o]] = cvt_from_d<TO>(acc);
-        else op[m.ooff[o]] = cvt_from_f<TO>(acc);
+        for (int e = e0; e < e1; e++) acc += m.eval(e) * to_acc<acc_t>(ip[m.eoff(e)]);
+        if constexpr (std::is_same<TI, double>::value) op[m.ooff(o)] = cvt_from_d<TO>(acc);
+        else op[m.ooff(o)] = cvt_from_f<TO>(acc);
     }
 }
 
@@ -129,16 +149,16 @@ __global__ void __launch_bounds__(256) wmix_idt_k(const TI* __restrict__ in, lon
     const int wb = threadIdx.x >> 2, wc = (threadIdx.x & 3) * 8;
     const bool wok = blockIdx.x * 64 + wb < Bn;
     for (int o = blockIdx.z; o < t.nout; o += gridDim.z) {
-        const int e0 = m.optr[o], e1 = m.optr[o + 1];
+        const int e0 = m.optr(o), e1 = m.optr(o + 1);
         acc_t acc[8];
 #pragma unroll
         for (int r = 0; r < 8; r++) acc[r] = 0;
         if (bok) {
 #pragma unroll 2
             for (int e = e0; e < e1; e++) {
-                const acc_t v = m.eval[e];
-                const long off = m.eoff[e] + b;
-                if (m.esel[e]) {
+                const acc_t v = m.eval(e);
+                const long off = m.eoff(e) + b;
+                if (m.esel(e)) {
 #pragma unroll
                     for (int r = 0; r < 8; r++) acc[r] += v * to_acc<acc_t>(in2[(x0 + r) * isx2 + off]);
                 } else {
@@ -147,10 +167,10 @@ __global__ void __launch_bounds__(256) wmix_idt_k(const TI* __restrict__ in, lon
                 }
             }
         }
-        if (m.osel[o]) {  // identity channel of L: straight into y[x][m][b]
+        if (m.osel(o)) {  // identity channel of L: straight into y[x][m][b]
             if (bok) {
 #pragma unroll
-                for (int r = 0; r < 8; r++) out2[(x0 + r) * osx2 + m.ooff[o] + b] = (double)acc[r];
+                for (int r = 0; r < 8; r++) out2[(x0 + r) * osx2 + m.ooff(o) + b] = (double)acc[r];
             }
             continue;
         }
@@ -159,7 +179,7 @@ __global__ void __launch_bounds__(256) wmix_idt_k(const TI* __restrict__ in, lon
         for (int r = 0; r < 8; r++) tile[tb][tr * 8 + r] = acc[r];
         __syncthreads();
         if (wok) {
-            TO* dst = out + m.ooff[o] + (long)(blockIdx.x * 64 + wb) * ldo + (long)blockIdx.y * 32 + wc;
+            TO* dst = out + m.ooff(o) + (long)(blockIdx.x * 64 + wb) * ldo + (long)blockIdx.y * 32 + wc;
             if constexpr (X3) {
                 // three bfloat16 planes, one 16-byte store per plane (8 values;
                 // every offset here is a multiple of 8 elements)
@@ -2482,13 +2502,13 @@ __global__ void __launch_bounds__(256) bwmix_k(const MixJob* __restrict__ jobs, 
     TO* op = (TO*)j.out + x * j.osx + b;
     const float* ip2 = idt ? j.in2 + x * j.isx2 + b : nullptr;
     for (int o = blockIdx.z % groups; o < t.nout; o += groups) {
-        const int e0 = m.optr[o], e1 = m.optr[o + 1];
+        const int e0 = m.optr(o), e1 = m.optr(o + 1);
         float acc = 0.0f;
 #pragma unroll 4
         for (int e = e0; e < e1; e++)
-            acc += m.eval[e] * (idt && m.esel[e] ? ip2[m.eoff[e]] : ip[m.eoff[e]]);
-        if (idt && m.osel[o]) j.out2[x * j.osx2 + m.ooff[o] + b] = (double)acc;
-        else op[m.ooff[o]] = cvt_from_f<TO>(acc);
+            acc += m.eval(e) * (idt && m.esel(e) ? ip2[m.eoff(e)] : ip[m.eoff(e)]);
+        if (idt && m.osel(o)) j.out2[x * j.osx2 + m.ooff(o) + b] = (double)acc;
+        else op[m.ooff(o)] = cvt_from_f<TO>(acc);
     }
 }
 hipError_t bwmix(int tout, const MixJob* jobs, int n, int Xmax, int Bnmax, int nout_max, int nnz_max, hipStream_t s)
