@@ -54,27 +54,73 @@ def test_odd_multiples_of_sixteen(ctx, tin, akm, bkm, M, N, K):
         _product(ctx, tin, akm, bkm, M, N, K, tile)
 
 
-@pytest.mark.parametrize("D1,D2,d", [(30, 30, 2), (320, 64, 2), (64, 320, 3), (288, 224, 2)])
-@pytest.mark.parametrize("prec,u", [(tn.TN_FP64, 2.0 ** -53), (tn.TN_FP32, 2.0 ** -24)])
-def test_heff_with_built_in_split(ctx, D1, D2, d, prec, u):
-    # stage 3 sums over (w, a'): split over K for the wide left environments
+def _pad(D):
+    return (D + 31) // 32 * 32
+
+
+def _heff(W, L, R, x):
+    T = np.einsum("anb,cwb->anwc", x, R, optimize=True)
+    T = np.einsum("anwc,vwmn->vamc", T, W, optimize=True)
+    return np.einsum("eva,vamc->emc", L, T, optimize=True)
+
+
+def _flat(F):  # (bra, w, ket) -> F[w + Dw*(i + D*j)]
+    return np.ascontiguousarray(F.transpose(2, 0, 1)).ravel()
+
+
+# (d, Dw, D1, D2) and the k-split of stage 3 (sum over (w, a')) in FP64, FP32 and
+# split bf16: none, by two and by four
+@pytest.mark.parametrize("d,Dw,D1,D2,splits", [(2, 3, 30, 30, (1, 1, 1)), (2, 3, 320, 64, (1, 1, 1)),
+                                               (3, 3, 64, 320, (1, 1, 1)), (2, 3, 288, 224, (1, 1, 1)),
+                                               (3, 4, 160, 96, (2, 2, 1)), (2, 4, 128, 64, (4, 4, 4)),
+                                               (2, 4, 320, 224, (4, 4, 4)), (2, 4, 250, 20, (4, 4, 4))])
+@pytest.mark.parametrize("k,prec", enumerate([tn.TN_FP64, tn.TN_FP32, tn.TN_BF16X3]))
+def test_heff_with_built_in_split(ctx, d, Dw, D1, D2, splits, k, prec):
+    D1p, D2p = _pad(D1), _pad(D2)
+    assert tn.gemm_plan(prec, True, True, D1p, d * D2p, Dw * D1p, split=True)[1] == splits[k]
     rng = np.random.default_rng(D1 + D2)
-    W = np.ascontiguousarray(rng.uniform(-1.0, 1.0, (3, 3, d, d)))
-    L, R = rng.uniform(-1.0, 1.0, (D1, 3, D1)), rng.uniform(-1.0, 1.0, (D2, 3, D2))
+    W = np.ascontiguousarray(rng.uniform(-1.0, 1.0, (Dw, Dw, d, d)))
+    L, R = rng.uniform(-1.0, 1.0, (D1, Dw, D1)), rng.uniform(-1.0, 1.0, (D2, Dw, D2))
     x = rng.uniform(-1.0, 1.0, (D1, d, D2))
-
-    def contract(W, L, R, x):
-        T = np.einsum("anb,cwb->anwc", x, R, optimize=True)
-        T = np.einsum("anwc,vwmn->vamc", T, W, optimize=True)
-        return np.einsum("eva,vamc->emc", L, T, optimize=True)
-
-    ctx.site_bind(W, np.ascontiguousarray(L.transpose(2, 0, 1)).ravel(),
-                  np.ascontiguousarray(R.transpose(2, 0, 1)).ravel(), d, D1, D2, prec)
+    ctx.site_bind(W, _flat(L), _flat(R), d, D1, D2, prec)
     y = ctx.heff_apply(np.ascontiguousarray(x.transpose(2, 0, 1)).ravel()).reshape(D2, D1, d).transpose(1, 2, 0)
-    ref = contract(W, L, R, x)
-    size = contract(np.abs(W), np.abs(L), np.abs(R), np.abs(x))
-    # one rounding per term of the three nested sums
-    assert np.all(np.abs(y - ref) <= (D2 + 3 * d + 3 * D1 + 8) * u * size)
+    ref = _heff(W, L, R, x)
+    size = _heff(np.abs(W), np.abs(L), np.abs(R), np.abs(x))
+    # one rounding per term of the three nested sums; split bf16: six products and
+    # one rounding per term
+    u = 2.0 ** -53 if prec == tn.TN_FP64 else 2.0 ** -24
+    terms = 7 if prec == tn.TN_BF16X3 else 1
+    assert np.all(np.abs(y - ref) <= (terms * (D2 + Dw * D1) + Dw * d + 8 * terms) * u * size)
+
+
+# FP64 environments: left with its last sum (a, m) split, right with its first (b')
+@pytest.mark.parametrize("direction,d,Dw,D1,D2,split", [(0, 2, 4, 250, 20, 4), (0, 2, 4, 320, 20, 2), (1, 2, 4, 20, 640, 2),
+                                                        (1, 2, 3, 20, 512, 4)])
+def test_environment_with_built_in_split(ctx, direction, d, Dw, D1, D2, split):
+    D1p, D2p = _pad(D1), _pad(D2)
+    shape = (D2p, Dw * D2p, D1p * d) if direction == 0 else (D1p * d, Dw * D2p, D2p)
+    assert tn.gemm_plan(tn.TN_FP64, direction == 1, direction == 1, *shape, split=True)[1] == split
+    rng = np.random.default_rng(D1 + 3 * D2)
+    W = np.ascontiguousarray(rng.uniform(-1.0, 1.0, (Dw, Dw, d, d)))
+    L, R = rng.uniform(-1.0, 1.0, (D1, Dw, D1)), rng.uniform(-1.0, 1.0, (D2, Dw, D2))
+    A = rng.uniform(-1.0, 1.0, (D1, d, D2))
+
+    def update(W, L, R, A):
+        if direction == 0:
+            T = np.einsum("eva,anb->evnb", L, A, optimize=True)
+            T = np.einsum("evnb,vwmn->emwb", T, W, optimize=True)
+            return np.einsum("emc,emwb->cwb", A, T, optimize=True)
+        T = np.einsum("anb,cwb->anwc", A, R, optimize=True)
+        T = np.einsum("anwc,vwmn->avmc", T, W, optimize=True)
+        return np.einsum("emc,avmc->eva", A, T, optimize=True)
+
+    ctx.site_bind(W, _flat(L), _flat(R), d, D1, D2, tn.TN_FP64)
+    D = D2 if direction == 0 else D1
+    F = ctx.env_update(direction, np.ascontiguousarray(A.transpose(2, 0, 1)).ravel(), D * D * Dw)
+    F = F.reshape(D, D, Dw).transpose(1, 2, 0)
+    size = update(np.abs(W), np.abs(L), np.abs(R), np.abs(A))
+    n = (D1 if direction == 0 else D2) * (1 + d) + Dw * d + 8  # terms of the three nested sums
+    assert np.all(np.abs(F - update(W, L, R, A)) <= n * 2.0 ** -53 * size)
 
 
 @pytest.mark.parametrize("M,N,K", [(32, 64, 128), (192, 256, 256), (256, 192, 512), (320, 448, 1280), (1024, 384, 1024),
