@@ -66,30 +66,24 @@ __device__ __forceinline__ void split3_val(float v, bf16& h0, bf16& h1, bf16& h2
 // MFMA traits: 16x16 output block per wave instruction
 //   A frag: lane l holds A[l%16][kbase + (l/16)*KPL + 0..KPL-1]
 //   B frag: lane l holds B[kbase + (l/16)*KPL + ..][l%16]
+//          (KPL = 1 for f64 and f32)
 //   C    : lane l holds C[row(l, r)][l%16], r = 0..3, with
 //          row = (l/16)*4 + r for the f32/bf16 instructions and
 //          row = (l/16) + 4*r for f64 (measured on gfx950 with a one-wave probe)
 template <typename TI> struct MT;
 template <> struct MT<double> {
-    static constexpr int KPL = 1, MK = 4, VEC = 2, PAD = 2;
     static __device__ __forceinline__ int crow(int lane, int r) { return (lane >> 4) + 4 * r; }
-    typedef double frag_t;
     typedef v4d acc_t;
-    typedef double acc_e;
 };
 template <> struct MT<float> {
-    static constexpr int KPL = 1, MK = 4, VEC = 4, PAD = 4;
     static __device__ __forceinline__ int crow(int lane, int r) { return (lane >> 4) * 4 + r; }
-    typedef float frag_t;
     typedef v4f acc_t;
-    typedef float acc_e;
 };
 template <> struct MT<bf16> {
     static constexpr int KPL = 8, MK = 32, VEC = 8, PAD = 8;
     static __device__ __forceinline__ int crow(int lane, int r) { return (lane >> 4) * 4 + r; }
     typedef v8bf frag_t;
     typedef v4f acc_t;
-    typedef float acc_e;
 };
 
 __device__ __forceinline__ v4d mma(double a, double b, v4d c)

@@ -23,31 +23,21 @@ struct GemmParams {
     int accumulate;
 };
 
-// element j of a 16-byte vector holding VEC values of type TI
-template <typename TI> __device__ __forceinline__ TI vec_elem(const u32x4& v, int j);
-template <> __device__ __forceinline__ double vec_elem<double>(const u32x4& v, int j)
-{
-    return j == 0 ? __hiloint2double((int)v.y, (int)v.x) : __hiloint2double((int)v.w, (int)v.z);
-}
-template <> __device__ __forceinline__ float vec_elem<float>(const u32x4& v, int j)
-{
-    const uint32_t w = j == 0 ? v.x : (j == 1 ? v.y : (j == 2 ? v.z : v.w));
-    return __uint_as_float(w);
-}
-template <> __device__ __forceinline__ bf16 vec_elem<bf16>(const u32x4& v, int j)
+// element j of a 16-byte vector of bfloat16 values
+__device__ __forceinline__ bf16 vec_elem(const u32x4& v, int j)
 {
     const uint32_t w = (j >> 1) == 0 ? v.x : ((j >> 1) == 1 ? v.y : ((j >> 1) == 2 ? v.z : v.w));
     return (bf16)((j & 1) ? (w >> 16) : (w & 0xffffu));
 }
 
-// global -> registers for one operand tile (ROWS x BK, K-major in LDS)
+// global -> registers for one bfloat16 operand tile (ROWS x BK, K-major in LDS)
 //   KM  : operand(row, k) = G[row*ld + k]   (vector loads along k)
 //   !KM : operand(row, k) = G[k*ld + row]   (vector loads along row)
-template <typename TI, int ROWS, int BK, bool KM, int R>
-__device__ __forceinline__ void tile_gload(u32x4 (&rg)[R], const TI* __restrict__ G, long ld,
+template <int ROWS, int BK, bool KM, int R>
+__device__ __forceinline__ void tile_gload(u32x4 (&rg)[R], const bf16* __restrict__ G, long ld,
                                            int r0, int k0, int tid)
 {
-    constexpr int VEC = MT<TI>::VEC;
+    constexpr int VEC = MT<bf16>::VEC;
     constexpr int TOT = ROWS * BK / VEC;
 #pragma unroll
     for (int r = 0; r < R; r++) {
@@ -63,12 +53,12 @@ __device__ __forceinline__ void tile_gload(u32x4 (&rg)[R], const TI* __restrict_
         }
     }
 }
-template <typename TI, int ROWS, int BK, bool KM, int R>
-__device__ __forceinline__ void tile_sstore(const u32x4 (&rg)[R], TI* __restrict__ S, int tid)
+template <int ROWS, int BK, bool KM, int R>
+__device__ __forceinline__ void tile_sstore(const u32x4 (&rg)[R], bf16* __restrict__ S, int tid)
 {
-    constexpr int VEC = MT<TI>::VEC;
+    constexpr int VEC = MT<bf16>::VEC;
     constexpr int TOT = ROWS * BK / VEC;
-    constexpr int LDK = BK + MT<TI>::PAD;
+    constexpr int LDK = BK + MT<bf16>::PAD;
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const int v = tid + r * 256;
@@ -79,21 +69,21 @@ __device__ __forceinline__ void tile_sstore(const u32x4 (&rg)[R], TI* __restrict
             } else {
                 const int kk = v / (ROWS / VEC), rv = v % (ROWS / VEC);
 #pragma unroll
-                for (int j = 0; j < VEC; j++) S[(rv * VEC + j) * LDK + kk] = vec_elem<TI>(rg[r], j);
+                for (int j = 0; j < VEC; j++) S[(rv * VEC + j) * LDK + kk] = vec_elem(rg[r], j);
             }
         }
     }
 }
 
-// One BM x BN output tile: 256 threads = 4 waves in a 2x2 arrangement, wave
-// tile (BM/2) x (BN/2); operand tiles staged through LDS (As, Bs) with the
-// next K-slice prefetched into registers.
-template <typename TI, typename TO, int BM, int BN, int BK, bool AKM, bool BKM>
-__device__ __forceinline__ void gemm_tile(const TI* __restrict__ A, const TI* __restrict__ B, TO* __restrict__ C,
+// One BM x BN output tile of a bfloat16 product: 256 threads = 4 waves in a 2x2
+// arrangement, wave tile (BM/2) x (BN/2); operand tiles staged through LDS (As,
+// Bs) with the next K-slice prefetched into registers.
+template <typename TO, int BM, int BN, int BK, bool AKM, bool BKM>
+__device__ __forceinline__ void gemm_tile(const bf16* __restrict__ A, const bf16* __restrict__ B, TO* __restrict__ C,
                                           long lda, long ldb, long ldc, int K, float alpha, int accumulate,
-                                          int m0, int n0, TI* __restrict__ As, TI* __restrict__ Bs)
+                                          int m0, int n0, bf16* __restrict__ As, bf16* __restrict__ Bs)
 {
-    typedef MT<TI> T;
+    typedef MT<bf16> T;
     typedef typename T::frag_t frag_t;
     typedef typename T::acc_t acc_t;
     constexpr int LDK = BK + T::PAD;
@@ -117,15 +107,15 @@ __device__ __forceinline__ void gemm_tile(const TI* __restrict__ A, const TI* __
             for (int r = 0; r < 4; r++) acc[i][j][r] = 0;
 
     const int nk = K / BK;
-    tile_gload<TI, BM, BK, AKM>(ra, A, lda, m0, 0, tid);
-    tile_gload<TI, BN, BK, BKM>(rb, B, ldb, n0, 0, tid);
-    tile_sstore<TI, BM, BK, AKM>(ra, As, tid);
-    tile_sstore<TI, BN, BK, BKM>(rb, Bs, tid);
+    tile_gload<BM, BK, AKM>(ra, A, lda, m0, 0, tid);
+    tile_gload<BN, BK, BKM>(rb, B, ldb, n0, 0, tid);
+    tile_sstore<BM, BK, AKM>(ra, As, tid);
+    tile_sstore<BN, BK, BKM>(rb, Bs, tid);
     __syncthreads();
     for (int t = 0; t < nk; t++) {
         if (t + 1 < nk) {
-            tile_gload<TI, BM, BK, AKM>(ra, A, lda, m0, (t + 1) * BK, tid);
-            tile_gload<TI, BN, BK, BKM>(rb, B, ldb, n0, (t + 1) * BK, tid);
+            tile_gload<BM, BK, AKM>(ra, A, lda, m0, (t + 1) * BK, tid);
+            tile_gload<BN, BK, BKM>(rb, B, ldb, n0, (t + 1) * BK, tid);
         }
         // the MFMA section of a slice at raised wave priority: a wave that has
         // its operands in LDS issues ahead of waves still loading or storing
@@ -147,8 +137,8 @@ __device__ __forceinline__ void gemm_tile(const TI* __restrict__ A, const TI* __
         __builtin_amdgcn_s_setprio(0);
         __syncthreads();
         if (t + 1 < nk) {
-            tile_sstore<TI, BM, BK, AKM>(ra, As, tid);
-            tile_sstore<TI, BN, BK, BKM>(rb, Bs, tid);
+            tile_sstore<BM, BK, AKM>(ra, As, tid);
+            tile_sstore<BN, BK, BKM>(rb, Bs, tid);
             __syncthreads();
         }
     }
@@ -173,12 +163,12 @@ __device__ __forceinline__ void gemm_tile(const TI* __restrict__ A, const TI* __
             }
 }
 
-template <typename TI, typename TO, int BM, int BN, int BK, bool AKM, bool BKM>
+template <typename TO, int BM, int BN, int BK, bool AKM, bool BKM>
 __global__ void __launch_bounds__(256) gemm_k(GemmParams p)
 {
-    constexpr int LDK = BK + MT<TI>::PAD;
-    __shared__ __attribute__((aligned(16))) TI As[BM * LDK];
-    __shared__ __attribute__((aligned(16))) TI Bs[BN * LDK];
+    constexpr int LDK = BK + MT<bf16>::PAD;
+    __shared__ __attribute__((aligned(16))) bf16 As[BM * LDK];
+    __shared__ __attribute__((aligned(16))) bf16 Bs[BN * LDK];
     const int ntn = p.N / BN, ntm = p.M / BM;
     const int nblk = ntn * ntm;
     int bid = blockIdx.x;
@@ -194,7 +184,7 @@ __global__ void __launch_bounds__(256) gemm_k(GemmParams p)
     const int local = bid - g * gsz;
     const int tm = first + local % rows, tn = local / rows;
     const long bz = blockIdx.y;
-    gemm_tile<TI, TO, BM, BN, BK, AKM, BKM>((const TI*)p.A + bz * p.sA, (const TI*)p.B + bz * p.sB,
+    gemm_tile<TO, BM, BN, BK, AKM, BKM>((const bf16*)p.A + bz * p.sA, (const bf16*)p.B + bz * p.sB,
                                             (TO*)p.C + bz * p.sC, p.lda, p.ldb, p.ldc, p.K, p.alpha,
                                             p.accumulate, tm * BM, tn * BN, As, Bs);
 }
@@ -281,12 +271,6 @@ template <typename TI, int ROWS, int BK, bool KM> struct Stage {
         if constexpr (KM) return S[row * BK + (((k / E) ^ rsw(row)) * E) + k % E];
         else return S[k * ROWS + ((row / E) ^ ksw(k)) * E + row % E];
     }
-    // FP64: operand(row, 2u) and operand(row, 2u + 1)
-    static __device__ __forceinline__ double2 pair(const TI* S, int row, int u)
-    {
-        if constexpr (KM) return *(const double2*)(S + row * BK + ((u ^ rsw(row)) * E));
-        else return make_double2(at(S, row, 2 * u), at(S, row, 2 * u + 1));
-    }
 };
 
 template <int BM, int BN, int BK, int S, typename TI> constexpr int stage_bytes()
@@ -371,17 +355,17 @@ __device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __
         const TI* Bs = As + BM * BK;
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int kk = 0; kk < BK; kk += 4) {
-                TI a[FM], b[FN];
+        for (int kk = 0; kk < BK; kk += 4) {
+            TI a[FM], b[FN];
 #pragma unroll
-                for (int i = 0; i < FM; i++) a[i] = SA::at(As, wm0 + i * 16 + r, kk + kq);
+            for (int i = 0; i < FM; i++) a[i] = SA::at(As, wm0 + i * 16 + r, kk + kq);
 #pragma unroll
-                for (int j = 0; j < FN; j++) b[j] = SB::at(Bs, wn0 + j * 16 + r, kk + kq);
+            for (int j = 0; j < FN; j++) b[j] = SB::at(Bs, wn0 + j * 16 + r, kk + kq);
 #pragma unroll
-                for (int i = 0; i < FM; i++)
+            for (int i = 0; i < FM; i++)
 #pragma unroll
-                    for (int j = 0; j < FN; j++) acc[i][j] = mma(a[i], b[j], acc[i][j]);
-            }
+                for (int j = 0; j < FN; j++) acc[i][j] = mma(a[i], b[j], acc[i][j]);
+        }
         __builtin_amdgcn_s_setprio(0);
         asm volatile("" : : : "memory");  // nor below the next one's wait
         st = st + 1 == S ? 0 : st + 1;
@@ -507,8 +491,8 @@ __device__ __forceinline__ void gemm_tile_x3(const bf16* __restrict__ A, long ps
     const int nk = K / BK;
 #pragma unroll
     for (int p = 0; p < 3; p++) {
-        tile_gload<bf16, BM, BK, true>(ra[p], A + p * psA, lda, m0, 0, tid);
-        tile_gload<bf16, BN, BK, true>(rb[p], B + p * psB, ldb, n0, 0, tid);
+        tile_gload<BM, BK, true>(ra[p], A + p * psA, lda, m0, 0, tid);
+        tile_gload<BN, BK, true>(rb[p], B + p * psB, ldb, n0, 0, tid);
     }
 #pragma unroll
     for (int p = 0; p < 3; p++) {
@@ -520,8 +504,8 @@ __device__ __forceinline__ void gemm_tile_x3(const bf16* __restrict__ A, long ps
         if (t + 1 < nk) {
 #pragma unroll
             for (int p = 0; p < 3; p++) {
-                tile_gload<bf16, BM, BK, true>(ra[p], A + p * psA, lda, m0, (t + 1) * BK, tid);
-                tile_gload<bf16, BN, BK, true>(rb[p], B + p * psB, ldb, n0, (t + 1) * BK, tid);
+                tile_gload<BM, BK, true>(ra[p], A + p * psA, lda, m0, (t + 1) * BK, tid);
+                tile_gload<BN, BK, true>(rb[p], B + p * psB, ldb, n0, (t + 1) * BK, tid);
             }
         }
         __builtin_amdgcn_s_setprio(1);
@@ -807,12 +791,14 @@ __global__ void __launch_bounds__(256, OCC) gemm_grouped_k(const GemmProb* __res
     }
 }
 
-// tile menu (code -> BM x BN; "deep" tiles stage twice the K slice per LDS
-// round, halving the barriers per flop at twice the LDS footprint).  The
-// 96-wide tiles exist for the split-bfloat16 product only: at two
-// workgroups per CU, 3072 x 4096 in 96 x 128 tiles (and 1024 x 3072 in
-// 128 x 96 tiles, split-K 2) fills the 256 CUs in whole rounds, where
-// 128 x 128 tiles leave the last round half empty.
+// tile menu (code -> BM x BN).  "deep" tiles: bf16 and split bf16 stage twice the
+// K slice per LDS round, halving the barriers per flop at twice the LDS footprint;
+// FP64 and FP32 keep one LDS stage more.  For every type they take K in multiples
+// of twice the plain step, the shapes for which saved tuning tables name them.
+// The 96-wide tiles exist for the split-bfloat16 product only: at two workgroups
+// per CU, 3072 x 4096 in 96 x 128 tiles (and 1024 x 3072 in 128 x 96 tiles,
+// split-K 2) fills the 256 CUs in whole rounds, where 128 x 128 tiles leave the
+// last round half empty.
 struct TileCfg { int bm, bn; bool deep; const char* name; bool x3only; };
 static const TileCfg kTiles[] = {
     {128, 128, false, "128x128", false}, {128, 64, false, "128x64", false}, {64, 128, false, "64x128", false},
@@ -829,20 +815,19 @@ const char* gemm_tile_name(int code) { return (code >= 1 && code <= kNumTiles) ?
 template <typename TO, int BK, bool AKM, bool BKM>
 static hipError_t launch_bf16(int code, const GemmParams& p, int batch, hipStream_t s)
 {
-    typedef bf16 TI;
     const TileCfg& t = kTiles[code];
     dim3 grid((p.M / t.bm) * (p.N / t.bn), batch);
     switch (code) {
-    case 0: gemm_k<TI, TO, 128, 128, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    case 1: gemm_k<TI, TO, 128, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    case 2: gemm_k<TI, TO, 64, 128, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    case 3: gemm_k<TI, TO, 64, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    case 4: gemm_k<TI, TO, 32, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    case 5: gemm_k<TI, TO, 64, 32, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    case 6: gemm_k<TI, TO, 32, 32, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    case 7: gemm_k<TI, TO, 128, 128, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    case 8: gemm_k<TI, TO, 128, 64, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
-    default: gemm_k<TI, TO, 64, 128, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 0: gemm_k<TO, 128, 128, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 1: gemm_k<TO, 128, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 2: gemm_k<TO, 64, 128, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 3: gemm_k<TO, 64, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 4: gemm_k<TO, 32, 64, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 5: gemm_k<TO, 64, 32, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 6: gemm_k<TO, 32, 32, BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 7: gemm_k<TO, 128, 128, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    case 8: gemm_k<TO, 128, 64, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
+    default: gemm_k<TO, 64, 128, 2 * BK, AKM, BKM><<<grid, 256, 0, s>>>(p); break;
     }
     return hipGetLastError();
 }
@@ -1011,6 +996,14 @@ static hipError_t gemm_x3(const GemmDesc& g, hipStream_t s)
     return hipErrorInvalidValue;
 }
 
+// K values of a step
+static int gemm_k_step(int tin, int K)
+{
+    if (tin == T_F64) return 16;
+    if (tin == T_F32) return K % 32 == 0 ? 32 : 16;
+    return K % 64 == 0 ? 64 : 32;
+}
+
 bool gemm_tile_ok(int code, int tin, int M, int N, int K)
 {
     if (code < 1 || code > kNumTiles) return false;
@@ -1024,12 +1017,6 @@ int gemm_tile_bm(int code) { return (code >= 1 && code <= kNumTiles) ? kTiles[co
 int gemm_tile_bn(int code) { return (code >= 1 && code <= kNumTiles) ? kTiles[code - 1].bn : 0; }
 static int choose_tile(int M, int N, int batch);
 int gemm_grouped_tile(int M, int N) { return choose_tile(M, N, 1) + 1; }
-int gemm_k_step(int tin, int K)
-{
-    if (tin == T_F64) return 16;
-    if (tin == T_F32) return K % 32 == 0 ? 32 : 16;
-    return K % 64 == 0 ? 64 : 32;
-}
 
 hipError_t gemm_grouped(int tin, int tout, bool akm, bool bkm, int tile, const GemmProb* probs, const int* off,
                          int nprob, int total_tiles, hipStream_t s)

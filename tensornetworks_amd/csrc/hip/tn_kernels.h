@@ -65,7 +65,6 @@ int gemm_tile_bn(int code);
 void gemm_default(int tin, int M, int N, int K, int batch, bool split, int* tile, int* ksplit);
 // built-in tile code of one problem of a grouped launch
 int gemm_grouped_tile(int M, int N);
-int gemm_k_step(int tin, int K);
 // FP64 / FP32 operands too long for the tile's 32-bit copy offsets: gemm takes its
 // 32x32 tile with 64-bit ones
 bool gemm_wide(int code, int tin, bool akm, bool bkm, long lda, long ldb);
