@@ -936,13 +936,16 @@ hipError_t lz_update(double* w, const double* V, long ldv, int k, long n, double
 // per thread) and in LDS, where every wave takes whole vectors of the basis:
 // one lane reduction per vector instead of one per vector and wave.  Bound by
 // the one CU's reads of the basis (two passes), so it pays while that is small
-// (lz_small_ok).  n = 2048: 8.8 us at k = 1, 10.5 at 8, 15.6 at 30, 19.8 at 48; the
-// four launches take 14.3 us and three launch gaps of about 1.5 us at k ~ 28.
-// n = 12288 took 23 us at k = 2, more than the four launches.
+// (lz_small_ok).  This launch and the four of the split step, launch after launch:
+// n = 1024: 9.0 and 12.3 us at k = 1, 14.1 and 13.8 at 32, 17.3 and 14.3 at 48;
+// n = 2048: 9.0 and 12.5 at 1, 12.5 and 13.7 at 16, 16.3 and 14.1 at 32;
+// n = 4096: 10.3 and 13.2 at 1, 13.3 and 13.6 at 8, 17.2 and 13.8 at 16;
+// n = 6144: 11.8 and 13.7 at 1, 13.4 and 13.9 at 4, 16.2 and 14.2 at 8 (12288: 23 at 2).
+// They cross near n k = 32768.
 #define LZ_TINY_T 1024
 #define LZ_TINY_K 64
 #define LZ_TINY_N (6 * LZ_TINY_T)
-bool lz_small_ok(long n, int k) { return n > 0 && n % 128 == 0 && n <= LZ_TINY_N && k >= 1 && k <= LZ_TINY_K && n * k <= 65536; }
+bool lz_small_ok(long n, int k) { return n > 0 && n % 128 == 0 && n <= LZ_TINY_N && k >= 1 && k <= LZ_TINY_K && n * k <= 32768; }
 
 template <int PP>
 __global__ void __launch_bounds__(LZ_TINY_T) lz_small_k(const double* __restrict__ y, double* __restrict__ V, long ldv,

@@ -33,8 +33,9 @@ def _restarted_lanczos(apply, x, steps, cycles):
 
 
 # padded lengths 2048, 8192 (last with 512-entry chunks), 9216, 131072 (last with
-# 4096-entry chunks and split vector groups), 147456 (long vectors)
-@pytest.mark.parametrize("d,D1,D2,steps", [(2, 32, 32, 9), (2, 64, 64, 8), (2, 64, 64, 33), (3, 90, 31, 17),
+# 4096-entry chunks and split vector groups), 147456 (long vectors); steps past the
+# line between one launch and four (2048 with 16 vectors, 6144 with 5)
+@pytest.mark.parametrize("d,D1,D2,steps", [(2, 32, 32, 9), (2, 32, 32, 24), (3, 64, 32, 9), (2, 64, 64, 8), (2, 64, 64, 33), (3, 90, 31, 17),
                                            (2, 256, 256, 26), (2, 288, 256, 5), (2, 288, 256, 4)])
 def test_capped_solve_matches_numpy(ctx, d, D1, D2, steps):
     rng = np.random.default_rng(100 * D1 + D2 + steps)
