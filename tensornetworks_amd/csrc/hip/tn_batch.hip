@@ -215,9 +215,11 @@ std::vector<GroupLaunch> gemm_group_stage(tn_batch* b, const std::vector<GemmDes
                    TN_ERR_ARG, "gemm_group: mixed problem types");
         int tile = gemm_choice(c, g).first;
         if (!gemm_tile_ok(tile, g.tin, g.M, g.N, g.K)) tile = gemm_grouped_tile(g.M, g.N);
-        if (gemm_wide(tile, g.tin, g.a_kmajor, g.b_kmajor, g.lda, g.ldb)) tile = 7;  // 32x32
-        TN_REQUIRE(!gemm_wide(tile, g.tin, g.a_kmajor, g.b_kmajor, g.lda, g.ldb), TN_ERR_ARG,
-                   "gemm_group: leading dimension too large");
+        if (gemm_wide(tile, g.tin, g.a_kmajor, g.b_kmajor, g.lda, g.ldb)) {
+            tile = 7;  // 32x32
+            TN_REQUIRE(!gemm_wide(tile, g.tin, g.a_kmajor, g.b_kmajor, g.lda, g.ldb), TN_ERR_ARG,
+                       "gemm_group: leading dimension too large");
+        }
         TN_REQUIRE(g.K % (128 / (int)dtype_size(g.tin)) == 0, TN_ERR_ARG, "gemm_group: K must be a multiple of 128 bytes");
         groups[tile].push_back(q);
     }

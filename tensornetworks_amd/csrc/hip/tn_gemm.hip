@@ -209,27 +209,29 @@ __device__ __forceinline__ uint32_t lds_offset(const void* p)
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
 }
 // 64 lanes copy 16 bytes each from base + off (off per lane, 32 bits unsigned) to
-// LDS address dst + 16 * lane (dst uniform).  The instruction takes dst from M0,
-// which the compiler owns (it is no register that inline assembly may declare as
-// clobbered): its value is put back.
+// LDS address dst + 16 * lane (dst uniform).  The instruction takes dst from M0.  M0
+// is reserved: the compiler writes it right before an instruction of its own that
+// reads it and keeps nothing there otherwise, so it need not be preserved (putting
+// the old value back cost 2-3 % of an apply at a left bond of 64); the clobber, of
+// which clang warns for reserved registers, keeps such a write from moving or
+// being shared across a copy.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void copy_to_lds(const void* base, uint32_t off, uint32_t dst)
 {
-    uint32_t m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
-                 "global_load_lds_dwordx4 %2, %3\n\ts_mov_b32 m0, %0"
-                 : "=&s"(m0)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
                  : "s"(dst), "v"(off), "s"(base)
-                 : "memory");
+                 : "memory", "m0");
 }
 __device__ __forceinline__ void copy_to_lds(const void* base, uint64_t off, uint32_t dst)
 {
-    uint32_t m0;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\t"
-                 "global_load_lds_dwordx4 %2, off\n\ts_mov_b32 m0, %0"
-                 : "=&s"(m0)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :
                  : "s"(dst), "v"((const char*)base + off)
-                 : "memory");
+                 : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // all but the last N copies have arrived and every LDS read has returned
 template <int N> __device__ __forceinline__ void wait_copies()
 {
@@ -253,14 +255,14 @@ template <typename TI, int ROWS, int BK, bool KM> struct Stage {
     }
     // byte offset, from the operand's first row and K index of the step, of the
     // unit that slot `slot` holds
-    static __device__ __forceinline__ uint64_t goff(int slot, long ld)
+    template <typename OFF> static __device__ __forceinline__ OFF goff(int slot, long ld)
     {
         if constexpr (KM) {
             const int row = slot / UPK, u = (slot % UPK) ^ rsw(row);
-            return (row * ld + u * E) * (long)sizeof(TI);
+            return (OFF)((row * ld + u * E) * (long)sizeof(TI));
         } else {
             const int k = slot / UPR, u = (slot % UPR) ^ ksw(k);
-            return (k * ld + u * E) * (long)sizeof(TI);
+            return (OFF)((k * ld + u * E) * (long)sizeof(TI));
         }
     }
     // values between the starts of consecutive K steps
@@ -311,12 +313,12 @@ __device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __
 
     const TI* Ab = AKM ? A + (long)m0 * lda : A + m0;
     const TI* Bb = BKM ? B + (long)n0 * ldb : B + n0;
-    typedef typename std::conditional<WIDE, uint64_t, uint32_t>::type off_t;
-    off_t off[L];
+    typedef typename std::conditional<WIDE, uint64_t, uint32_t>::type OFF;
+    OFF off[L];
 #pragma unroll
     for (int i = 0; i < L; i++) {
         const int c = wid * L + i;
-        off[i] = (off_t)(c < CA ? SA::goff(c * 64 + lane, lda) : SB::goff((c - CA) * 64 + lane, ldb));
+        off[i] = c < CA ? SA::template goff<OFF>(c * 64 + lane, lda) : SB::template goff<OFF>((c - CA) * 64 + lane, ldb);
     }
     const uint32_t base = __builtin_amdgcn_readfirstlane(lds_offset(sm));
     const long ka = SA::kstep(lda), kb = SB::kstep(ldb);
@@ -400,8 +402,11 @@ __device__ __forceinline__ void pipe_tile(const TI* __restrict__ A, const TI* __
 // column blocks of B)
 __device__ __forceinline__ void tile_of_block(int bid, int ntm, int ntn, int& tm, int& tn)
 {
+    // (two branches: with one formula the compiler read the kernel's arguments later,
+    // and the smallest products took 5 % longer)
     const int nblk = ntm * ntn, xcd = bid & 7, rest = nblk & 7;
-    bid = xcd * (nblk >> 3) + (xcd < rest ? xcd : rest) + (bid >> 3);
+    if (rest == 0) bid = xcd * (nblk >> 3) + (bid >> 3);
+    else bid = xcd * (nblk >> 3) + (xcd < rest ? xcd : rest) + (bid >> 3);
     constexpr int GM = 8;
     const int gsz = GM * ntn, g = bid / gsz, first = g * GM;
     const int rows = ntm - first < GM ? ntm - first : GM;
@@ -840,7 +845,7 @@ bool gemm_wide(int code, int tin, bool akm, bool bkm, long lda, long ldb)
 {
     if ((tin != T_F64 && tin != T_F32) || code < 1 || code > kNumTiles) return false;
     const long es = tin == T_F64 ? 8 : 4, bk = 128 / es;
-    auto far = [&](bool km, int rows, long ld) { return ld > 0 && (km ? rows : bk) * es > (1L << 32) / ld; };
+    auto far = [&](bool km, int rows, long ld) { return (km ? rows : bk) * es * ld > 1L << 32; };
     return far(akm, kTiles[code - 1].bm, lda) || far(bkm, kTiles[code - 1].bn, ldb);
 }
 
