@@ -20,10 +20,13 @@ namespace tn {
 // table in global memory) and after: transposed FP64 form, D = 8: 11.5 and
 // 4.1 us; 320 x 224, d = 2: 15.5 and 7.5 us; D = 256, d = 3: 21.7 and 6.9 us;
 // FP32 512 x 448, d = 3: 16.5 and 8.9 us; plain FP64 form, D = 256, d = 2: 6.9
-// and 6.4 us.  What comes from LDS is the same for every lane and goes back to
-// scalar registers, so that the eight addresses of an entry are one scalar sum
-// each (with the offsets left in vector registers FP32 D = 2048, d = 3 took 160 us,
-// D = 1500 78; now 114 and 63).  Sums keep the table's order.
+// and 6.4 us.  What comes from LDS is the same for every lane.  In the transposed
+// FP32 form, with eight reads per entry, it goes back to scalar registers, so that
+// the eight addresses are one scalar sum each (with the offsets left in vector
+// registers D = 2048, d = 3 took 160 us, D = 1500 78; now 114 and 63).  In FP64 the
+// memory hides the sums and small bonds lose (D = 256, d = 3: 7.0 -> 8.0 us); with one
+// read per entry it only lengthens the chain (batched form 48 -> 55 us).  Sums keep
+// the table's order.
 #define MIX_MAXO 64
 #define MIX_MAXE 512
 template <typename V> struct MixLds {
@@ -31,19 +34,20 @@ template <typename V> struct MixLds {
     long ooff[MIX_MAXO], eoff[MIX_MAXE];
     V eval[MIX_MAXE];
 };
-// STG: the table's copy in LDS (nout <= MIX_MAXO, nnz <= MIX_MAXE), else global
-template <typename V, bool STG> struct MixView {
+// STG: the table's copy in LDS (nout <= MIX_MAXO, nnz <= MIX_MAXE), else global.
+// SCALAR: what comes from LDS goes back to scalar registers
+template <typename V, bool STG, bool SCALAR> struct MixView {
     const int *optr_, *osel_, *esel_;
     const long *ooff_, *eoff_;
     const V* eval_;
     static __device__ __forceinline__ int uni(int v)
     {
-        if constexpr (STG) return __builtin_amdgcn_readfirstlane(v);
+        if constexpr (STG && SCALAR) return __builtin_amdgcn_readfirstlane(v);
         else return v;
     }
     static __device__ __forceinline__ long uni(long v)
     {
-        if constexpr (STG)
+        if constexpr (STG && SCALAR)
             return (long)(uint32_t)uni((int)v) | ((long)uni((int)(v >> 32)) << 32);
         else return v;
     }
@@ -60,11 +64,11 @@ __device__ __forceinline__ const V* mix_values(const MixTable& t)
     if constexpr (std::is_same<V, double>::value) return t.eval;
     else return t.evalf;
 }
-template <typename V, bool STG>
-__device__ __forceinline__ MixView<V, STG> mix_view(const MixTable& t, MixLds<V>* l)
+template <typename V, bool STG, bool SCALAR = false>
+__device__ __forceinline__ MixView<V, STG, SCALAR> mix_view(const MixTable& t, MixLds<V>* l)
 {
     if constexpr (!STG) {
-        return MixView<V, STG>{t.optr, t.osel, t.esel, t.ooff, t.eoff, mix_values<V>(t)};
+        return MixView<V, STG, SCALAR>{t.optr, t.osel, t.esel, t.ooff, t.eoff, mix_values<V>(t)};
     } else {
         const V* v = mix_values<V>(t);
         const bool idt = t.esel != nullptr;
@@ -79,7 +83,7 @@ __device__ __forceinline__ MixView<V, STG> mix_view(const MixTable& t, MixLds<V>
             l->esel[i] = idt ? t.esel[i] : 0;
         }
         __syncthreads();
-        return MixView<V, STG>{l->optr, l->osel, l->esel, l->ooff, l->eoff, l->eval};
+        return MixView<V, STG, SCALAR>{l->optr, l->osel, l->esel, l->ooff, l->eoff, l->eval};
     }
 }
 // grid z for nout outputs over xy workgroups
@@ -96,7 +100,7 @@ __global__ void __launch_bounds__(256) wmix_k(const TI* __restrict__ in, long is
 {
     typedef typename std::conditional<std::is_same<TI, double>::value, double, float>::type acc_t;
     __shared__ typename std::conditional<STG, MixLds<acc_t>, int>::type lds;
-    const MixView<acc_t, STG> m = mix_view<acc_t, STG>(t, (MixLds<acc_t>*)&lds);
+    const MixView<acc_t, STG, false> m = mix_view<acc_t, STG>(t, (MixLds<acc_t>*)&lds);
     const int b = blockIdx.x * 64 + (threadIdx.x & 63);
     const long x = (long)blockIdx.y * 4 + (threadIdx.x >> 6);
     if (b >= Bn || x >= X) return;
@@ -140,7 +144,8 @@ __global__ void __launch_bounds__(256) wmix_idt_k(const TI* __restrict__ in, lon
     typedef typename std::conditional<std::is_same<TI, double>::value, double, float>::type acc_t;
     __shared__ acc_t tile[64][33];
     __shared__ typename std::conditional<STG, MixLds<acc_t>, int>::type lds;
-    const MixView<acc_t, STG> m = mix_view<acc_t, STG>(t, (MixLds<acc_t>*)&lds);
+    constexpr bool SCALAR = !std::is_same<TI, double>::value;
+    const MixView<acc_t, STG, SCALAR> m = mix_view<acc_t, STG, SCALAR>(t, (MixLds<acc_t>*)&lds);
     const int tb = threadIdx.x & 63, tr = threadIdx.x >> 6;  // b within the tile, row group of 8
     const int b = blockIdx.x * 64 + tb;
     const long x0 = (long)blockIdx.y * 32 + tr * 8;
@@ -2487,19 +2492,28 @@ hipError_t bconvert(const ConvJob* jobs, int n, long nmax, hipStream_t s)
     return hipGetLastError();
 }
 
-// MPO mixing (FP32 in, TO out) for many problems: the layout of wmix_k, the
-// problem in grid z
+// MPO mixing (FP32 in, TO out) for many problems, the problem in grid z.  A
+// workgroup takes bw values of b times 256 / bw of x, bw the largest of 256, 128
+// and 64 that leaves no more threads idle than 64 does (128 chains of 32 to 256: 48
+// us with 64 throughout, 43 so).
+__host__ __device__ static inline int bwmix_width(int Bn)
+{
+    const int pad = (Bn + 63) & ~63;
+    return ((Bn + 255) & ~255) == pad ? 256 : (((Bn + 127) & ~127) == pad ? 128 : 64);
+}
 template <typename TO, bool STG>
 __global__ void __launch_bounds__(256) bwmix_k(const MixJob* __restrict__ jobs, int groups)
 {
     __shared__ typename std::conditional<STG, MixLds<float>, int>::type lds;
     const MixJob& j = jobs[blockIdx.z / groups];
-    if (blockIdx.x * 64 >= j.Bn || (long)blockIdx.y * 4 >= j.X) return;  // the whole workgroup
+    const int bw = bwmix_width(j.Bn), rows = 256 / bw, nb = (j.Bn + bw - 1) / bw;
+    const int by = blockIdx.x / nb, bx = blockIdx.x - by * nb;
+    if (by * rows >= j.X) return;  // the whole workgroup
     const MixTable t = j.t;
     const bool idt = t.esel != nullptr;
-    const MixView<float, STG> m = mix_view<float, STG>(t, (MixLds<float>*)&lds);
-    const int b = blockIdx.x * 64 + (threadIdx.x & 63);
-    const long x = (long)blockIdx.y * 4 + (threadIdx.x >> 6);
+    const MixView<float, STG, false> m = mix_view<float, STG>(t, (MixLds<float>*)&lds);
+    const int b = bx * bw + (threadIdx.x & (bw - 1));
+    const long x = by * rows + (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 64) / bw;
     if (b >= j.Bn || x >= j.X) return;
     const float* ip = (const float*)j.in + x * j.isx + b;
     TO* op = (TO*)j.out + x * j.osx + b;
@@ -2517,8 +2531,9 @@ __global__ void __launch_bounds__(256) bwmix_k(const MixJob* __restrict__ jobs, 
 hipError_t bwmix(int tout, const MixJob* jobs, int n, int Xmax, int Bnmax, int nout_max, int nnz_max, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    dim3 grid((Bnmax + 63) / 64, (Xmax + 3) / 4);
-    const int groups = mix_groups((long)grid.x * grid.y * n, nout_max);
+    // workgroups of the widest problem: no width takes more than 64 does
+    dim3 grid(((Bnmax + 63) / 64) * ((Xmax + 3) / 4));
+    const int groups = mix_groups((long)grid.x * n, nout_max);
     grid.z = n * groups;
     const bool stg = nout_max <= MIX_MAXO && nnz_max <= MIX_MAXE;
     if (tout == T_F32 && stg) bwmix_k<float, true><<<grid, 256, 0, s>>>(jobs, groups);

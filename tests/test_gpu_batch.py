@@ -52,6 +52,27 @@ def test_batch_matches_single_chain_sweeps(ctx):
     b.close()
 
 
+def test_batch_of_wide_bonds_matches_single_chain_sweeps(ctx):
+    # padded bonds of 32 to 256 in one batch: every width of the batched MPO stage
+    spec = [(18, 256, 1.0, 1.0, 0.0), (16, 100, 0.7, 1.6, 0.3), (16, 128, 1.3, 0.4, -0.2), (18, 220, 0.9, 1.1, 0.1),
+            (8, 12, 1.1, 0.8, -0.1)]
+    o = fp32_opts()
+    batch_chains = [make_chain(ctx, *s, seed=300 + k, opts=o) for k, s in enumerate(spec)]
+    b = tn.Batch(ctx, batch_chains, max_krylov=40)
+    for _ in range(3):
+        b.sweep(0, o)
+        b.sweep(1, o)
+    for k, (s, cb) in enumerate(zip(spec, batch_chains)):
+        cs = make_chain(ctx, *s, seed=300 + k, opts=o)
+        for _ in range(3):
+            cs.sweep(0, o)
+            cs.sweep(1, o)
+        eb, es = cb.expectation(), cs.expectation()
+        assert abs(eb - es) < 1e-8 * max(1.0, abs(es)), (s, eb, es)
+        assert cb.dims() == cs.dims()
+    b.close()
+
+
 def test_batch_partial_reorth_matches_single_chain_sweeps(ctx):
     # partial re-orthogonalisation in the pipelined batch (a chain whose new
     # vector needs a pass against the whole basis defers its tridiagonal
